@@ -76,8 +76,6 @@ struct dg_ctx {
   dg_walk_queue* h_queue = nullptr;  // pinned mirror
   uint32_t* d_freq = nullptr;        // cumulative visit counts
   uint64_t freq_total = 0;           // sum of d_freq
-  uint32_t* d_freq_round = nullptr;  // visits of the round being walked
-  size_t freq_round_cap = 0;
   uint32_t* d_hot_part = nullptr;    // per pack workgroup: hot-vertex counts
   size_t hot_part_cap = 0;
   uint32_t* d_tok_raw = nullptr;     // tokens in completion order
@@ -95,8 +93,7 @@ struct dg_ctx {
   uint64_t* d_scan_tmp = nullptr;    // block sums for scans
   size_t scan_tmp_cap = 0;
   double* d_term_table = nullptr;    // tabulated entropy terms for short walks
-  double* d_re_terms = nullptr;      // v_num
-  double* d_re_chunks = nullptr;
+  double* d_re_chunks = nullptr;     // relative entropy: a sum per 1024 vertices
   size_t re_cap = 0;
   dg_walk_plan* wplan = nullptr;     // the round planned for the captured step
   uint64_t cur_walks = 0;

@@ -360,12 +360,6 @@ __global__ void queue_reset_kernel(dg_walk_queue* q) {
   }
 }
 
-__global__ void add_u32_kernel(uint32_t* dst, const uint32_t* src, uint64_t n) {
-  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (uint64_t)gridDim.x * blockDim.x)
-    dst[i] += src[i];
-}
-
 __global__ void fill_u32_kernel(uint32_t* p, uint64_t n, uint32_t v) {
   for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
        i += (uint64_t)gridDim.x * blockDim.x)
@@ -555,66 +549,83 @@ __global__ __launch_bounds__(64) void hot_reduce_kernel(const uint32_t* hot_part
 }
 
 // ---- relative entropy (walk.hpp:693-725) in a fixed summation order -------
-// terms[i] = p_i (ln p_i - ln q_i); chunk sums of 1024 consecutive terms added
+// Terms p_i (ln p_i - ln q_i); chunk sums of 1024 consecutive terms added
 // left to right, then the chunk sums added left to right.
 constexpr uint32_t kReChunk = 1024;
 
-// wsum = the visits counted before this round plus the round's tokens (from
-// the queue, so the host need not know the round's token count).
-__global__ void re_terms_kernel(const uint32_t* deg, const uint32_t* freq, uint32_t v_num,
-                                uint64_t dsum, uint64_t wsum_before, double* terms,
-                                dg_walk_queue* q) {
+// One workgroup per chunk: its terms into LDS (four per thread), then the sum
+// left to right by one lane.  The order makes a chunk 1,024 dependent FP64
+// adds, so the sum is bound by their latency: reading them from LDS, several
+// ahead, one add is all that is on the chain: 16 us plus 4 us for the chunk
+// sums at 262,144 vertices, 114 us with the running sum taken through lane
+// shuffles and the terms passed through memory.  wsum = the visits counted
+// before this round plus the round's tokens (from the queue, so the host need
+// not know the round's token count).  A vertex without a term adds 0, which
+// leaves the running sum's bits as they are.
+constexpr int kReBlock = 256;
+
+// Sum of n LDS values left to right, sixteen values read ahead of the adds.
+__device__ __forceinline__ double ordered_sum(const double* v, uint32_t n, double sum) {
+  uint32_t i = 0;
+  for (; i + 16 <= n; i += 16) {
+    double t[16];
+#pragma unroll
+    for (int u = 0; u < 16; ++u) t[u] = v[i + u];
+#pragma unroll
+    for (int u = 0; u < 16; ++u) sum = sum + t[u];
+  }
+  for (; i < n; ++i) sum = sum + v[i];
+  return sum;
+}
+
+__global__ __launch_bounds__(kReBlock) void re_chunks_kernel(const uint32_t* deg, const uint32_t* freq,
+                                                             uint32_t v_num, uint64_t dsum,
+                                                             uint64_t wsum_before, double* chunks,
+                                                             dg_walk_queue* q) {
+  __shared__ __align__(16) double s_term[kReChunk];
+  __shared__ uint32_t s_zeros;
+  if (threadIdx.x == 0) s_zeros = 0;
+  __syncthreads();
   const uint64_t wsum = wsum_before + q->tokens;
-  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < v_num;
-       i += gridDim.x * blockDim.x) {
-    const uint32_t d = deg[i], f = freq[i];
+  const uint32_t lo = blockIdx.x * kReChunk;
+  const uint32_t n = v_num - lo < kReChunk ? v_num - lo : kReChunk;
+  uint32_t zeros = 0;
+#pragma unroll
+  for (uint32_t k = 0; k < kReChunk / kReBlock; ++k) {
+    const uint32_t j = k * kReBlock + threadIdx.x;
+    if (j >= n) break;
+    const uint32_t d = deg[lo + j], f = freq[lo + j];
     double t = 0.0;
     if (d == 0 || f == 0) {
-      atomicAdd(&q->zero_terms, 1u);
+      ++zeros;
     } else {
       const double pi = (double)d / (double)dsum;
       const double qi = (double)f / (double)wsum;
       t = pi * (dg_log(pi) - dg_log(qi));
     }
-    terms[i] = t;
+    s_term[j] = t;
+  }
+  if (zeros) atomicAdd(&s_zeros, zeros);
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    chunks[blockIdx.x] = ordered_sum(s_term, n, 0.0);
+    if (s_zeros) atomicAdd(&q->zero_terms, s_zeros);
   }
 }
 
-// One wavefront per chunk: the 64 lanes load 64 consecutive terms at a time
-// (coalesced) and the sum is taken in index order from the lane registers,
-// left to right as the order above requires.
-__global__ __launch_bounds__(256) void re_chunks_kernel(const double* terms, const uint32_t* deg,
-                                                        const uint32_t* freq, uint32_t v_num,
-                                                        double* chunks, uint32_t n_chunks) {
-  const uint32_t lane = threadIdx.x & 63u;
-  const uint32_t c = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-  if (c >= n_chunks) return;  // wave-uniform
-  const uint32_t lo = c * kReChunk;
-  const uint32_t hi = lo + kReChunk < v_num ? lo + kReChunk : v_num;
-  double part = 0.0;
-  for (uint32_t i0 = lo; i0 < hi; i0 += 64) {
-    const uint32_t i = i0 + lane;
-    const bool in = i < hi && deg[i] != 0 && freq[i] != 0;
-    const double t = in ? terms[i] : 0.0;
-    const uint64_t live = __ballot(in);
-    const uint32_t n = hi - i0 < 64u ? hi - i0 : 64u;
-    for (uint32_t k = 0; k < n; ++k)
-      if ((live >> k) & 1ull) part = part + __shfl(t, (int)k, 64);
-  }
-  if (lane == 0) chunks[c] = part;
-}
-
-// The chunk sums left to right, by one wavefront in the same way.
-__global__ __launch_bounds__(64) void re_final_kernel(const double* chunks, uint32_t n_chunks,
-                                                      dg_walk_queue* q) {
-  const uint32_t lane = threadIdx.x & 63u;
+// The chunk sums left to right in the same way, by one workgroup.
+__global__ __launch_bounds__(kReBlock) void re_final_kernel(const double* chunks, uint32_t n_chunks,
+                                                            dg_walk_queue* q) {
+  __shared__ __align__(16) double s_part[kReChunk];
   double total = 0.0;
-  for (uint32_t c0 = 0; c0 < n_chunks; c0 += 64) {
-    const double t = c0 + lane < n_chunks ? chunks[c0 + lane] : 0.0;
-    const uint32_t n = n_chunks - c0 < 64u ? n_chunks - c0 : 64u;
-    for (uint32_t k = 0; k < n; ++k) total = total + __shfl(t, (int)k, 64);
+  for (uint32_t c0 = 0; c0 < n_chunks; c0 += kReChunk) {
+    const uint32_t n = n_chunks - c0 < kReChunk ? n_chunks - c0 : kReChunk;
+    for (uint32_t j = threadIdx.x; j < n; j += kReBlock) s_part[j] = chunks[c0 + j];
+    __syncthreads();
+    if (threadIdx.x == 0) total = ordered_sum(s_part, n, total);
+    __syncthreads();
   }
-  if (lane == 0) q->re = total;
+  if (threadIdx.x == 0) q->re = total;
 }
 
 __global__ void offsets_shift_kernel(const uint64_t* src, uint64_t n, uint64_t add,
@@ -648,8 +659,8 @@ struct dg_walk_plan {
 void dg_walk_free(dg_ctx* ctx) {
   void* bufs[] = {ctx->d_freq,   ctx->d_tok_raw,  ctx->d_walk_off, ctx->d_walk_len,
                   ctx->d_tokens, ctx->d_offsets,  ctx->d_spill,    ctx->d_scan_tmp,
-                  ctx->d_re_terms, ctx->d_re_chunks, ctx->d_train_tokens, ctx->d_train_offsets,
-                  ctx->d_term_table, ctx->d_freq_round};
+                  ctx->d_re_chunks, ctx->d_train_tokens, ctx->d_train_offsets,
+                  ctx->d_term_table};
   for (void* p : bufs)
     if (p) hipFree(p);
   ctx->d_freq = nullptr;
@@ -660,13 +671,10 @@ void dg_walk_free(dg_ctx* ctx) {
   ctx->d_offsets = nullptr;
   ctx->d_spill = nullptr;
   ctx->d_scan_tmp = nullptr;
-  ctx->d_re_terms = nullptr;
   ctx->d_re_chunks = nullptr;
   ctx->d_train_tokens = nullptr;
   ctx->d_train_offsets = nullptr;
   ctx->d_term_table = nullptr;
-  ctx->d_freq_round = nullptr;
-  ctx->freq_round_cap = 0;
   delete ctx->wplan;
   ctx->wplan = nullptr;
   ctx->tok_raw_cap = ctx->walk_cap = ctx->walk_len_cap = ctx->tokens_cap = ctx->offsets_cap = 0;
@@ -773,9 +781,6 @@ static int plan_round(dg_ctx* ctx, const dg_walk_params* p, uint32_t round,
   const uint64_t slots_end = (uint64_t)walker_num * kPathLds;
   size_t tok_need = (size_t)slots_end + (size_t)walker_num / 8 + 4096;
   if (ctx->tok_raw_cap < tok_need) DG_CHECK(dg_reserve(ctx, &ctx->d_tok_raw, &ctx->tok_raw_cap, tok_need));
-  // this round's visits go to a separate count array, added to the cumulative
-  // counts once the round is packed
-  DG_CHECK(dg_reserve(ctx, &ctx->d_freq_round, &ctx->freq_round_cap, (size_t)ctx->v_num));
   {
     // packing: every resident workgroup slot (LDS: n_hot counters each), fewer for small rounds
     int pcu = 0;
@@ -788,8 +793,7 @@ static int plan_round(dg_ctx* ctx, const dg_walk_params* p, uint32_t round,
                         (size_t)pl->parts * (ctx->n_hot ? ctx->n_hot : 1)));
   }
   const uint32_t n_chunks = (ctx->v_num + kReChunk - 1) / kReChunk;
-  DG_CHECK(dg_reserve(ctx, &ctx->d_re_terms, &ctx->re_cap, (size_t)ctx->v_num + n_chunks));
-  ctx->d_re_chunks = nullptr;  // chunks live after the terms
+  DG_CHECK(dg_reserve(ctx, &ctx->d_re_chunks, &ctx->re_cap, (size_t)n_chunks));
   DG_CHECK(dg_reserve(ctx, &ctx->d_scan_tmp, &ctx->scan_tmp_cap,
                       (size_t)((walker_num + kScanTile - 1) / kScanTile) + 1));
 
@@ -833,42 +837,34 @@ static int enqueue_walk(dg_ctx* ctx, const dg_walk_plan& pl, bool timed) {
   return DG_OK;
 }
 
-// Everything after the walk: packing in walk-id order with the round's visit
-// counts, the cumulative counts, and the relative entropy.  Reads only device
+// Everything after the walk: packing in walk-id order with the round's visits
+// added to the cumulative counts (a round that failed packs nothing), and the
+// relative entropy.  Reads only device
 // state, so it needs no host knowledge of the round's token count.
 static int enqueue_tail(dg_ctx* ctx, const dg_walk_plan& pl, bool timed) {
   const uint32_t walker_num = pl.walker_num;
   size_t tp = 0;
   if (timed) DG_CHECK(dg_time_begin(ctx, "pack", &tp));
   DG_CHECK(dg_scan_lengths(ctx, ctx->d_walk_len, walker_num, ctx->d_offsets));
-  fill_u32_kernel<<<grid_for(ctx, ctx->v_num, 256), 256, 0, ctx->stream>>>(ctx->d_freq_round,
-                                                                           ctx->v_num, 0u);
   pack_count_kernel<<<pl.parts, kPackBlock, 0, ctx->stream>>>(
       ctx->d_tok_raw, ctx->d_walk_off, ctx->d_walk_len, ctx->d_offsets, walker_num, ctx->d_tokens,
-      ctx->d_hot_slot, ctx->n_hot, ctx->d_freq_round, ctx->d_hot_part);
+      ctx->d_hot_slot, ctx->n_hot, ctx->d_freq, ctx->d_hot_part);
   if (ctx->n_hot) {
     const dim3 grid((ctx->n_hot + 63) / 64, (pl.parts + kHotRows - 1) / kHotRows);
     hot_reduce_kernel<<<grid, 64, 0, ctx->stream>>>(ctx->d_hot_part, pl.parts, ctx->n_hot,
-                                                    ctx->d_hot_id, ctx->d_freq_round);
+                                                    ctx->d_hot_id, ctx->d_freq);
   }
   DG_HIP(ctx, hipGetLastError());
   if (timed) DG_CHECK(dg_time_end(ctx, tp));
-  add_u32_kernel<<<grid_for(ctx, ctx->v_num, 256), 256, 0, ctx->stream>>>(
-      ctx->d_freq, ctx->d_freq_round, ctx->v_num);
-  DG_HIP(ctx, hipGetLastError());
 
   // relative entropy against the cumulative visit counts
   const uint32_t n_chunks = (ctx->v_num + kReChunk - 1) / kReChunk;
-  double* chunks = ctx->d_re_terms + ctx->v_num;
   size_t tr = 0;
   if (timed) DG_CHECK(dg_time_begin(ctx, "re", &tr));
-  re_terms_kernel<<<grid_for(ctx, ctx->v_num, 256), 256, 0, ctx->stream>>>(
-      ctx->d_deg, ctx->d_freq, ctx->v_num, ctx->m, pl.freq_total_before, ctx->d_re_terms,
-      ctx->d_queue);
-  re_chunks_kernel<<<(n_chunks + 3) / 4, 256, 0, ctx->stream>>>(ctx->d_re_terms, ctx->d_deg,
-                                                                ctx->d_freq, ctx->v_num, chunks,
-                                                                n_chunks);
-  re_final_kernel<<<1, 64, 0, ctx->stream>>>(chunks, n_chunks, ctx->d_queue);
+  re_chunks_kernel<<<n_chunks, kReBlock, 0, ctx->stream>>>(ctx->d_deg, ctx->d_freq, ctx->v_num, ctx->m,
+                                                           pl.freq_total_before, ctx->d_re_chunks,
+                                                           ctx->d_queue);
+  re_final_kernel<<<1, kReBlock, 0, ctx->stream>>>(ctx->d_re_chunks, n_chunks, ctx->d_queue);
   DG_HIP(ctx, hipGetLastError());
   if (timed) DG_CHECK(dg_time_end(ctx, tr));
   return DG_OK;
