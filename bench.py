@@ -58,12 +58,12 @@ def walker_bytes(stats_list):
 
 def walker_transaction_bytes(stats_list):
     """Random 64-B transactions the kernel actually issues (a bounce-back
-    append reads nothing): one per drawn adjacency unit and one per row-offset
-    pair read (walk start and every move), plus 4 B per emitted vertex."""
+    append reads nothing): one per drawn adjacency unit (it carries the
+    neighbour's row) and one per walk start, plus 4 B per emitted vertex."""
     tokens = sum(s.tokens for s in stats_list)
     draws = sum(s.draws for s in stats_list)
-    moves = sum(s.moves for s in stats_list)
-    return 64 * (draws + moves) + 4 * tokens
+    starts = sum(s.walkers for s in stats_list)
+    return 64 * (draws + starts) + 4 * tokens
 
 
 def sgns_sent_bytes(kept, pool_rows, dim, negative):
@@ -449,7 +449,7 @@ def main():
         bf_bytes = sgns_sent_bytes(kept, pool_rows, args.dim, 5) / n_bf
         bf_gbs = bf_bytes / (bf_ms / n_bf * 1e-3) / 1e9
         # the walker's fraction of HBM: the 64-B transactions it issues (one per
-        # drawn adjacency unit, one per row-offset pair read; a bounce-back
+        # drawn adjacency unit, one per walk start; a bounce-back
         # append reads nothing) plus 4 B per emitted vertex, over its time; the
         # survey's per-step figure (two transactions for every step) is kept
         # beside it, labelled, as it overstates what the kernel reads

@@ -40,6 +40,7 @@ extern "C" int dg_open(int device, dg_ctx** out) {
     return DG_ERR_HIP;
   }
   if (hipMalloc((void**)&ctx->d_queue, sizeof(dg_walk_queue)) != hipSuccess ||
+      hipMalloc((void**)&ctx->d_shards, sizeof(dg_walk_shard) * kWalkShards) != hipSuccess ||
       hipHostMalloc((void**)&ctx->h_queue, sizeof(dg_walk_queue), hipHostMallocDefault) !=
           hipSuccess) {
     dg_close(ctx);
@@ -71,6 +72,7 @@ extern "C" void dg_close(dg_ctx* ctx) {
   for (auto e : ctx->event_pool) hipEventDestroy(e);
   if (ctx->d_stamps) hipFree(ctx->d_stamps);
   if (ctx->d_queue) hipFree(ctx->d_queue);
+  if (ctx->d_shards) hipFree(ctx->d_shards);
   if (ctx->h_queue) hipHostFree(ctx->h_queue);
   if (ctx->stream) hipStreamDestroy(ctx->stream);
   delete ctx;

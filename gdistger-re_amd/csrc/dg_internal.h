@@ -15,7 +15,6 @@
 
 // Device-side walk queue and round statistics (one per context).
 struct dg_walk_queue {
-  unsigned long long next;    // next walk index to hand out (relative to walker_begin)
   unsigned long long cursor;  // tokens of walks longer than a slot, in the overflow region
   unsigned int flags;         // DG_QFLAG_*
   unsigned int max_len;       // longest walk
@@ -23,13 +22,38 @@ struct dg_walk_queue {
   unsigned int pad;
   double re;                  // relative entropy of the round
   unsigned long long draws;   // candidate draws (adjacency units read)
-  unsigned long long moves;   // row-offset pairs read (walk starts + moves)
+  unsigned long long moves;   // rows entered (walk starts + moves)
   unsigned long long tokens;  // tokens written
 };
+
+// A shard of the walk queue, in cache lines of its own: the workgroups with
+// one id mod kWalkShards hand out their share of the round's walks and add up
+// their totals here.  One counter for the whole round served the wavefronts
+// one after another (about 50 ns each, 0.2 ms for the 4,096 resident ones at
+// the start of every round).
+struct alignas(256) dg_walk_shard {
+  unsigned long long next;    // walks handed out
+  unsigned long long draws, moves, tokens;
+  unsigned int max_len;
+};
+constexpr uint32_t kWalkShards = 64;
 
 // Hot-vertex set for visit counting: at most kHotMax vertices.
 constexpr uint32_t kHotMax = 4096;
 constexpr uint16_t kNotHot = 0xffffu;
+
+// A vertex's row in an adjacency unit: offset (40 bits), degree (23 bits,
+// kRowDegMax where it does not fit: read the row pointers), and whether the
+// vertex has degree 2 and is its own first neighbour (walk.hpp:900-902).
+constexpr uint32_t kRowDegMax = 0x7fffffu;
+
+__host__ __device__ inline uint2 dg_pack_row(uint64_t begin, uint64_t degree, bool stuck) {
+  const uint32_t d = degree < kRowDegMax ? (uint32_t)degree : kRowDegMax;
+  return make_uint2((uint32_t)begin, (uint32_t)(begin >> 32) | (d << 8) | (stuck ? 1u << 31 : 0u));
+}
+__host__ __device__ inline uint64_t dg_row_begin(uint2 r) { return (uint64_t)(r.y & 0xffu) << 32 | r.x; }
+__host__ __device__ inline uint32_t dg_row_degree(uint2 r) { return (r.y >> 8) & kRowDegMax; }
+__host__ __device__ inline bool dg_row_stuck(uint2 r) { return (r.y >> 31) != 0u; }
 
 #define DG_QFLAG_TOKEN_OVERFLOW 1u
 #define DG_QFLAG_LENGTH_LIMIT 2u
@@ -63,7 +87,7 @@ struct dg_ctx {
   uint64_t* d_row_ptr = nullptr;
   uint32_t* d_nbr = nullptr;  // neighbour ids, reference order
   uint32_t* d_cn = nullptr;   // common-neighbour counts
-  uint2* d_adj = nullptr;     // walker view {neighbour, bounce threshold}
+  uint4* d_adj = nullptr;     // walker view {neighbour, bounce threshold, neighbour's row}
   uint32_t* d_deg = nullptr;
   // the highest-degree vertices, counted per workgroup in LDS when visit
   // counts are taken (their global counters would be contended)
@@ -74,6 +98,7 @@ struct dg_ctx {
   // walker buffers
   dg_walk_queue* d_queue = nullptr;
   dg_walk_queue* h_queue = nullptr;  // pinned mirror
+  dg_walk_shard* d_shards = nullptr; // kWalkShards
   uint32_t* d_freq = nullptr;        // cumulative visit counts
   uint64_t freq_total = 0;           // sum of d_freq
   uint32_t* d_hot_part = nullptr;    // per pack workgroup: hot-vertex counts

@@ -13,9 +13,11 @@
 //   d_row_ptr : uint64[V+1]  row offsets (edge_id_t)
 //   d_nbr     : uint32[m]    neighbour ids, reference order
 //   d_cn      : uint32[m]    common-neighbour count |N(u) & N(v) \ {u,v}|
-//   d_adj     : uint2[m]     walker view {neighbour, acceptance threshold}:
-//                            8 bytes per entry like the reference
-//                            AdjUnit<real_t> (include/graph.hpp:32-37)
+//   d_adj     : uint4[m]     walker view {neighbour, acceptance threshold,
+//                            the neighbour's row offset and degree}: what a
+//                            step needs by one 16-byte read (the reference's
+//                            AdjUnit<real_t>, include/graph.hpp:32-37, holds
+//                            the first two)
 //   d_deg     : uint32[V]    degree (= row length)
 //
 // Common neighbours (src/tools/gcn.cpp:250-373, the offline tool whose
@@ -30,8 +32,8 @@
 // Acceptance threshold: the walker bounces back when tanh(pa) <= p with
 // p = u / (2^31 - 1), u the 31-bit draw (walk.hpp:928-938).  pa depends only
 // on (deg u, deg v, cn), so per entry the smallest u that satisfies the test
-// is found once by bisection (u / M is monotone in u under correctly rounded
-// division), and the walker tests `u >= threshold` - the same decision bit
+// is found once (u / M is monotone in u under correctly rounded division),
+// and the walker tests `u >= threshold` - the same decision bit
 // for bit, without tanh or the neighbour's degree in the step loop.
 #include <algorithm>
 #include <atomic>
@@ -270,7 +272,7 @@ __device__ __forceinline__ uint32_t bounce_threshold(int sd, int dd, int cnv, co
 // src: the source vertex of every entry, or null (found by binary search).
 __global__ void threshold_kernel(const uint64_t* rp, const uint32_t* src, const uint32_t* nbr, const uint32_t* cn,
                                  const float* w, const uint32_t* deg, uint32_t v_num, uint64_t m,
-                                 uint2* adj) {
+                                 uint4* adj) {
   for (uint64_t e = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; e < m;
        e += (uint64_t)gridDim.x * blockDim.x) {
     uint32_t u;
@@ -288,11 +290,14 @@ __global__ void threshold_kernel(const uint64_t* rp, const uint32_t* src, const 
       u = lo;
     }
     const uint32_t v = nbr[e];
-    adj[e] = make_uint2(v, bounce_threshold((int)deg[u], (int)deg[v], (int)cn[e], w, e));
+    const uint64_t vb = rp[v];
+    const uint32_t dv = deg[v];
+    const uint2 row = dg_pack_row(vb, dv, dv == 2 && nbr[vb] == v);
+    adj[e] = make_uint4(v, bounce_threshold((int)deg[u], (int)dv, (int)cn[e], w, e), row.x, row.y);
   }
 }
 
-__global__ void take_thresholds_kernel(const uint2* adj, uint64_t m, uint32_t* thr) {
+__global__ void take_thresholds_kernel(const uint4* adj, uint64_t m, uint32_t* thr) {
   for (uint64_t e = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; e < m;
        e += (uint64_t)gridDim.x * blockDim.x)
     thr[e] = adj[e].y;
@@ -781,7 +786,7 @@ static int alloc_graph(dg_ctx* ctx, uint32_t v_num, uint64_t m) {
   DG_HIP(ctx, hipMalloc((void**)&ctx->d_row_ptr, sizeof(uint64_t) * (v_num + 1ull)));
   DG_HIP(ctx, hipMalloc((void**)&ctx->d_nbr, sizeof(uint32_t) * n));
   DG_HIP(ctx, hipMalloc((void**)&ctx->d_cn, sizeof(uint32_t) * n));
-  DG_HIP(ctx, hipMalloc((void**)&ctx->d_adj, sizeof(uint2) * n));
+  DG_HIP(ctx, hipMalloc((void**)&ctx->d_adj, sizeof(uint4) * n));
   DG_HIP(ctx, hipMalloc((void**)&ctx->d_deg, sizeof(uint32_t) * v_num));
   DG_HIP(ctx, hipMalloc((void**)&ctx->d_hot_slot, sizeof(uint16_t) * v_num));
   DG_HIP(ctx, hipMalloc((void**)&ctx->d_hot_id, sizeof(uint32_t) * kHotMax));

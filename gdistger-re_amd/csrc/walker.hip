@@ -10,15 +10,19 @@
 //   * One lane per walk, 64 walks per wavefront, in one persistent launch.
 //     Walks have uneven lengths; a lane whose walk ends takes the next walk id
 //     from its wave's pool, and a wave refills its pool with one 64-bit atomic
-//     on the device work queue, so every lane stays busy until the queue
-//     drains and every wave then leaves the loop.
-//   * Each lane keeps its walk in LDS (kPathLds vertices, lane-major with an odd
-//     stride so lane-strided and cooperative accesses are bank-conflict free)
-//     and spills longer walks to a private global area.  The visit count f_i
-//     of walk.hpp:816 (an unordered_map per walk) is a scan of that buffer.
-//   * A finished walk is written out cooperatively by its wave into its own
-//     slot (walk index * kPathLds tokens) with one 64-lane store; only walks
-//     longer than a slot take space from a shared overflow cursor.
+//     on its shard of the device work queue, so every lane stays busy until
+//     the shard drains and every wave then leaves the loop.
+//   * Each lane keeps its walk in LDS (kPathLds vertices, in 16-byte groups of
+//     four) and spills longer walks to a private global area.  The visit count
+//     f_i of walk.hpp:816 (an unordered_map per walk) is a scan of that
+//     buffer: six 16-byte LDS reads in flight together, unused places holding
+//     an id no vertex has.
+//   * An adjacency unit carries the neighbour's row offset and degree beside
+//     its id and bounce threshold (16 bytes), so a step reads one random
+//     address, not two in a row.
+//   * A finished walk goes into its own slot (walk index * kPathLds tokens) by
+//     16-byte stores of its own lane; only walks longer than a slot take space
+//     from a shared overflow cursor.
 //   * Visit counts are not taken in the walk loop: the packing pass counts
 //     every token, the highest-degree vertices in per-workgroup LDS counters
 //     and the rest with uncontended global atomics.
@@ -34,7 +38,9 @@
 namespace {
 
 constexpr int kWalkBlock = 256;
-constexpr int kPathLds = 23;    // vertices per lane kept in LDS (odd); reference walks hold 22
+constexpr int kPathLds = 24;    // vertices per lane kept in LDS; reference walks hold 22
+constexpr int kPathVec = kPathLds / 4;
+constexpr uint32_t kNoVertex = 0xffffffffu;  // never a vertex id (ids are below a 32-bit count)
 constexpr int kTermTable = 32;  // entropy terms tabulated for walks shorter than 32
 constexpr int kTermStride = kTermTable + 1;
 constexpr uint32_t kPool = 64;
@@ -42,7 +48,7 @@ constexpr uint32_t kDefaultLengthLimit = DG_WALK_LENGTH_LIMIT_DEFAULT;
 
 struct WalkArgs {
   const uint64_t* row_ptr;
-  const uint2* adj;  // {neighbour, bounce threshold}
+  const uint4* adj;  // {neighbour, bounce threshold, neighbour's row} (dg_pack_row)
   const double* term_table;
   uint32_t v_num;
   uint32_t round;
@@ -61,14 +67,27 @@ struct WalkArgs {
   uint32_t* walk_len;
   uint32_t* spill;
   dg_walk_queue* q;
+  dg_walk_shard* shards;
 };
 
 // Running statistics of Correlation (include/walk.hpp:260-387).  Sn and N
 // both equal the number of vertices on the walk, which the kernel keeps as an
-// integer, so only the seven FP64 moments live in registers.
+// integer, and the moments of S alone (ES, ESS) depend only on it: they are
+// tabulated up to kTermTable vertices and kept in registers past that.
 struct WalkState {
-  double H, EH, ES, EHS, EHH, ESS;
+  double H, EH, EHS, EHH;
+  double ES, ESS;  // past kTermTable vertices only
 };
+
+// x / n for an integer n, given y = 1 / n correctly rounded: two corrections
+// of x * y by the exact remainder give the correctly rounded quotient
+// (Markstein 1990), in 5 operations instead of a division's dozen.  x and
+// the remainders are far from the ends of the exponent range here.
+__device__ __forceinline__ double div_by(double x, double n, double y) {
+  double q = x * y;
+  q = __builtin_fma(__builtin_fma(-n, q, x), y, q);
+  return __builtin_fma(__builtin_fma(-n, q, x), y, q);
+}
 
 // log2 term of Correlation::iterateHn with step_k = 1 (include/walk.hpp:
 // 284-304) for a walk of Sn vertices appending a vertex seen fi times before:
@@ -87,35 +106,120 @@ __device__ __forceinline__ double entropy_term(double Sn, double fi) {
 // order.  The correlation R itself is only read by the termination test
 // (walk.hpp:979-985), which runs after min_length steps, so it is formed from
 // the moments there (state_corr) instead of on every step.
-__device__ __forceinline__ void state_iterate(WalkState& w, double Sn, double t) {
-  const double one = 1.0;
-  const double H1 = (Sn * w.H - t) / (Sn + one);
-  const double S1 = Sn + one;
-  const double N1 = Sn + 1.0;
-  w.EH = w.EH + (H1 - w.EH) / N1;
-  w.ES = w.ES + (S1 - w.ES) / N1;
-  w.EHS = w.EHS + (H1 * S1 - w.EHS) / N1;
-  w.EHH = w.EHH + (H1 * H1 - w.EHH) / N1;
-  w.ESS = w.ESS + (S1 * S1 - w.ESS) / N1;
+// y = 1 / (Sn + 1), correctly rounded.
+__device__ __forceinline__ void state_iterate(WalkState& w, double Sn, double t, double y) {
+  const double S1 = Sn + 1.0;
+  const double H1 = div_by(Sn * w.H - t, S1, y);
+  w.EH = w.EH + div_by(H1 - w.EH, S1, y);
+  w.EHS = w.EHS + div_by(H1 * S1 - w.EHS, S1, y);
+  w.EHH = w.EHH + div_by(H1 * H1 - w.EHH, S1, y);
   w.H = H1;
 }
 
+// The same step of the moments of S.
+__device__ __forceinline__ void size_iterate(double& ES, double& ESS, double Sn, double y) {
+  const double S1 = Sn + 1.0;
+  ES = ES + div_by(S1 - ES, S1, y);
+  ESS = ESS + div_by(S1 * S1 - ESS, S1, y);
+}
+
 // Pearson R of the (H, S) history from the running moments (walk.hpp:342-354).
-__device__ __forceinline__ double state_corr(const WalkState& w) {
+__device__ __forceinline__ double state_corr(const WalkState& w, double ES, double ESS) {
   const double DH = w.EHH - w.EH * w.EH;
-  const double DS = w.ESS - w.ES * w.ES;
-  const double cov = w.EHS - w.EH * w.ES;
+  const double DS = ESS - ES * ES;
+  const double cov = w.EHS - w.EH * ES;
   return cov == 0.0 ? 0.0 : cov / dg_sqrt(DH * DS);
 }
 
-// term_table[S * kTermStride + f] = entropy_term(S, f) for 1 <= S < kTermTable,
-// 0 <= f <= S; computed by the same device code the walker would run inline.
+// Tables of the walk: term[S * kTermStride + f] = entropy_term(S, f) for
+// 1 <= S < kTermTable, 0 <= f <= S, computed by the same device code the
+// walker would run inline; then for n <= kTermTable vertices 1 / n, ES and ESS.
+constexpr int kTermWords = kTermTable * kTermStride;
+constexpr int kTabInv = kTermWords, kTabES = kTabInv + kTermTable + 1, kTabESS = kTabES + kTermTable + 1;
+constexpr int kTabWords = kTabESS + kTermTable + 1;
+
 __global__ void term_table_kernel(double* tbl) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= kTermTable * kTermStride) return;
-  const int S = i / kTermStride, f = i % kTermStride;
-  tbl[i] = (S >= 1 && f <= S) ? entropy_term((double)S, (double)f) : 0.0;
+  if (i < kTermWords) {
+    const int S = i / kTermStride, f = i % kTermStride;
+    tbl[i] = (S >= 1 && f <= S) ? entropy_term((double)S, (double)f) : 0.0;
+  }
+  if (i == 0) {
+    double ES = 1.0, ESS = 1.0;
+    tbl[kTabInv] = tbl[kTabES] = tbl[kTabESS] = 0.0;
+    for (int n = 1; n <= kTermTable; ++n) {
+      const double y = 1.0 / (double)n;
+      if (n > 1) size_iterate(ES, ESS, (double)(n - 1), y);
+      tbl[kTabInv + n] = y;
+      tbl[kTabES + n] = ES;
+      tbl[kTabESS + n] = ESS;
+    }
+  }
 }
+
+// A lane's draws: the words of its stream (dg_stream), two Philox blocks deep.
+// The lanes of a wavefront run out at different steps, and a block evaluated
+// for one lane costs the wavefront as much as one for all: so when any lane
+// has fewer than the two words a step takes, every lane with room evaluates
+// its next block, and the wavefront evaluates one block per two steps at
+// most (it was one or two per step).
+struct WalkDraws {
+  uint32_t k0, k1, c1, c2, block;
+  uint32_t b[4], n[4];   // words in hand (shifted down), and the next block
+  uint32_t avail;        // words in b
+  bool next;             // n holds a block
+
+  __device__ __forceinline__ void start(uint64_t seed, uint32_t walk, uint32_t round) {
+    k0 = (uint32_t)seed;
+    k1 = (uint32_t)(seed >> 32);
+    c1 = walk;
+    c2 = round;
+    block = 0;
+    avail = 0;
+    next = false;
+  }
+  __device__ __forceinline__ bool low() const { return avail < 2 && !next; }
+  __device__ __forceinline__ void refill() {
+    if (next) return;
+    const dg_u32x4 o = dg_philox4x32_10(block, c1, c2, DG_TAG_WALK, k0, k1);
+    ++block;
+    n[0] = o.x0;
+    n[1] = o.x1;
+    n[2] = o.x2;
+    n[3] = o.x3;
+    next = true;
+  }
+  // needs a word in hand or a next block
+  __device__ __forceinline__ uint32_t take() {
+    if (avail == 0) {
+      b[0] = n[0];
+      b[1] = n[1];
+      b[2] = n[2];
+      b[3] = n[3];
+      avail = 4;
+      next = false;
+    }
+    const uint32_t r = b[0];
+    b[0] = b[1];
+    b[1] = b[2];
+    b[2] = b[3];
+    --avail;
+    return r;
+  }
+  // dg_stream_uniform; leaves at least one word for dg_stream_u31
+  __device__ __forceinline__ uint32_t uniform(uint32_t range) {
+    uint64_t m = (uint64_t)take() * (uint64_t)range;
+    if ((uint32_t)m < range) {
+      const uint32_t t = (uint32_t)(0u - range) % range;
+      while ((uint32_t)m < t) {  // a rejected word: once in 2^32 / range draws
+        if (low()) refill();
+        m = (uint64_t)take() * (uint64_t)range;
+      }
+      if (low()) refill();
+    }
+    return (uint32_t)(m >> 32);
+  }
+};
 
 __device__ __forceinline__ uint32_t lanes_below(uint64_t mask) {
   return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32),
@@ -127,16 +231,34 @@ __device__ __forceinline__ uint64_t wave_sum_u64(uint64_t v) {
   return v;
 }
 
+// Bound: at small rounds (fewer walks than lanes) the latency of one walk's
+// chain, per step one random adjacency read (about 1,100 cycles), the scan of
+// the walk, the entropy arithmetic and half a Philox block (300 to 700
+// each); at large ones the instructions of four wavefronts per SIMD.
+// 10,000 vertices (50,000 walks): 104 -> 44 us; 262,144 vertices: 1.31M walks
+// 649 -> 303 us, 262,144 walks 355 -> 88 us.  Most of it is the sharded queue;
+// the one-read step, the 16-byte scan, the reciprocals and the shared Philox
+// evaluations took 12% with the queue as it was.
 __global__ __launch_bounds__(kWalkBlock) void walk_kernel(WalkArgs a) {
-  __shared__ uint32_t s_path[kWalkBlock * kPathLds];
-  __shared__ double s_term[kTermTable * kTermStride];
-  for (int i = threadIdx.x; i < kTermTable * kTermStride; i += kWalkBlock) s_term[i] = a.term_table[i];
+  __shared__ uint4 s_path[kPathVec * kWalkBlock];  // [group of four][thread]
+  __shared__ double s_tab[kTabWords];
+  for (int i = threadIdx.x; i < kTabWords; i += kWalkBlock) s_tab[i] = a.term_table[i];
   __syncthreads();
 
   const uint32_t lane = threadIdx.x & 63u;
-  uint32_t* path = s_path + threadIdx.x * kPathLds;
+  uint32_t* path = reinterpret_cast<uint32_t*>(s_path + threadIdx.x);
   const uint64_t slot = (uint64_t)blockIdx.x * kWalkBlock + threadIdx.x;
   uint32_t* spill = a.spill + slot * a.spill_per_slot;
+
+  // this workgroup's shard of the walks: the round's walks divided in
+  // proportion to the workgroups of each shard
+  const uint32_t n_sh = gridDim.x < kWalkShards ? gridDim.x : kWalkShards;
+  const uint32_t sh = blockIdx.x % n_sh, b_per = gridDim.x / n_sh, b_more = gridDim.x % n_sh;
+  const uint64_t b_before = (uint64_t)sh * b_per + (sh < b_more ? sh : b_more);
+  const uint64_t b_mine = b_per + (sh < b_more ? 1u : 0u);
+  const uint64_t id0 = a.walker_num * b_before / gridDim.x;
+  const uint64_t id1 = a.walker_num * (b_before + b_mine) / gridDim.x;
+  dg_walk_shard* const shard = a.shards + sh;
 
   bool active = false;
   bool drained = false;                   // wave-uniform
@@ -144,14 +266,14 @@ __global__ __launch_bounds__(kWalkBlock) void walk_kernel(WalkArgs a) {
 
   uint32_t wid = 0, cur = 0, cur_deg = 0, len = 0;
   uint64_t cur_rb = 0;
-  uint32_t ndraw = 0, nmove = 0;
+  bool cur_stuck = false;                 // degree 2, itself its first neighbour
   // this lane's totals over its walks, added to the queue once per wave at the end
   uint64_t tot_draw = 0, tot_move = 0, tot_tok = 0;
   uint32_t max_l = 0;
   bool pending_back = false;
   WalkState ws = {0, 0, 0, 0, 0, 0};
-  dg_stream rs;
-  dg_stream_init(&rs, a.seed, 0, 0, DG_TAG_WALK);
+  WalkDraws rs;
+  rs.start(a.seed, 0, 0);
 
   while (true) {
     // ---- hand new walk ids to idle lanes --------------------------------
@@ -167,13 +289,13 @@ __global__ __launch_bounds__(kWalkBlock) void walk_kernel(WalkArgs a) {
           pool_next += nwant;
         } else {
           unsigned long long base = 0;
-          if (lane == 0) base = atomicAdd(&a.q->next, (unsigned long long)kPool);
-          base = __shfl(base, 0, 64);
+          if (lane == 0) base = atomicAdd(&shard->next, (unsigned long long)kPool);
+          base = id0 + __shfl(base, 0, 64);
           id = rank < avail ? pool_next + rank : base + (rank - avail);
           pool_next = base + (nwant - avail);
           pool_end = base + kPool;
         }
-        if (!active && id < a.walker_num) {
+        if (!active && id < id1) {
           // walk.hpp:529-589 (start = id mod V), :661-669 (footprint, step 0),
           // :849-856 (first-visit state)
           wid = (uint32_t)id;
@@ -181,18 +303,19 @@ __global__ __launch_bounds__(kWalkBlock) void walk_kernel(WalkArgs a) {
           cur = w % a.v_num;
           cur_rb = a.row_ptr[cur];
           cur_deg = (uint32_t)(a.row_ptr[cur + 1] - cur_rb);
-          path[0] = cur;
+          cur_stuck = cur_deg == 2 && a.adj[cur_rb].x == cur;
+#pragma unroll
+          for (int j = 0; j < kPathVec; ++j)
+            s_path[j * kWalkBlock + threadIdx.x] =
+                make_uint4(j == 0 ? cur : kNoVertex, kNoVertex, kNoVertex, kNoVertex);
           len = 1;
-          ndraw = 0;
-          nmove = 1;
+          ++tot_move;
           pending_back = false;
           ws.H = 0.0;
           ws.EH = 0.0;
-          ws.ES = 1.0;
           ws.EHS = 0.0;
           ws.EHH = 0.0;
-          ws.ESS = 1.0;
-          dg_stream_init(&rs, a.seed, w, a.round, DG_TAG_WALK);
+          rs.start(a.seed, w, a.round);
           active = true;
         }
         if (__ballot(!active) != 0) drained = true;
@@ -202,6 +325,7 @@ __global__ __launch_bounds__(kWalkBlock) void walk_kernel(WalkArgs a) {
       if (drained) break;
       continue;
     }
+    if (__ballot(active && rs.low()) != 0) rs.refill();
 
     // ---- one appended vertex per active lane ------------------------------
     bool finish = false;
@@ -212,47 +336,63 @@ __global__ __launch_bounds__(kWalkBlock) void walk_kernel(WalkArgs a) {
         bool append = false;
         bool trace = false;
         uint32_t v_app = 0;
-        uint64_t next_rb = 0, next_re = 0;  // row of the vertex moved to, loaded early
+        uint2 next_row = make_uint2(0u, 0u);  // row of the vertex moved to
         if (pending_back) {
           v_app = cur;  // walk.hpp:986-1017: back to the current vertex
           append = true;
         } else if (cur_deg == 0) {
           finish = true;  // walk.hpp:887-892
         } else {
-          const uint32_t i = dg_stream_uniform(&rs, cur_deg);  // walk.hpp:899
-          const uint2 e = a.adj[cur_rb + i];
-          ++ndraw;
-          if (cur_deg == 2 && a.adj[cur_rb].x == cur) {
+          const uint32_t i = rs.uniform(cur_deg);  // walk.hpp:899
+          const uint4 e = a.adj[cur_rb + i];
+          ++tot_draw;
+          if (cur_stuck) {
             finish = true;  // walk.hpp:900-902
           } else if (!(len == 1 && e.x == cur)) {  // walk.hpp:904-906 redraw at step 0
-            const uint32_t u = dg_stream_u31(&rs);  // walk.hpp:928
-            trace = (u >= e.y);                    // walk.hpp:933-938 via the threshold
+            const uint32_t u = rs.take() >> 1;  // walk.hpp:928
+            trace = (u >= e.y);                // walk.hpp:933-938 via the threshold
             v_app = e.x;
             append = true;
-            if (!trace) {  // the walk moves to e.x unless it ends: its row, in flight during the math
-              next_rb = a.row_ptr[e.x];
-              next_re = a.row_ptr[e.x + 1];
-            }
+            next_row = make_uint2(e.z, e.w);
           }
         }
         if (append) {
           // walk.hpp:961-985: footprint, f_i = visits so far, entropy update
-          uint32_t fi = 0;
-          const uint32_t n1 = len < (uint32_t)kPathLds ? len : (uint32_t)kPathLds;
-          for (uint32_t j = 0; j < n1; ++j) fi += (path[j] == v_app);
+          uint32_t f4[4] = {0u, 0u, 0u, 0u};  // four chains of adds
+#pragma unroll
+          for (int j = 0; j < kPathVec; ++j) {
+            const uint4 p = s_path[j * kWalkBlock + threadIdx.x];
+            f4[0] += p.x == v_app;
+            f4[1] += p.y == v_app;
+            f4[2] += p.z == v_app;
+            f4[3] += p.w == v_app;
+          }
+          uint32_t fi = (f4[0] + f4[1]) + (f4[2] + f4[3]);
           for (uint32_t j = kPathLds; j < len; ++j) fi += (spill[j - kPathLds] == v_app);
-          const double t = len < (uint32_t)kTermTable ? s_term[len * kTermStride + fi]
-                                                       : entropy_term((double)len, (double)fi);
-          state_iterate(ws, (double)len, t);
+          double t, y;
+          if (len < (uint32_t)kTermTable) {
+            t = s_tab[len * kTermStride + fi];
+            y = s_tab[kTabInv + len + 1];
+          } else {
+            t = entropy_term((double)len, (double)fi);
+            y = 1.0 / ((double)len + 1.0);
+            if (len == (uint32_t)kTermTable) {
+              ws.ES = s_tab[kTabES + kTermTable];
+              ws.ESS = s_tab[kTabESS + kTermTable];
+            }
+            size_iterate(ws.ES, ws.ESS, (double)len, y);
+          }
+          state_iterate(ws, (double)len, t, y);
           if (len < (uint32_t)kPathLds)
-            path[len] = v_app;
+            path[(len >> 2) * (kWalkBlock * 4) + (len & 3u)] = v_app;
           else
             spill[len - kPathLds] = v_app;
           ++len;
           const uint32_t step = len - 1;
           bool ends = false;
           if (step > a.min_length) {
-            const double R = state_corr(ws);
+            const bool tab = len <= (uint32_t)kTermTable;
+            const double R = state_corr(ws, tab ? s_tab[kTabES + len] : ws.ES, tab ? s_tab[kTabESS + len] : ws.ESS);
             ends = R * R < a.mu || R < 0.0;
           }
           if (ends) {
@@ -268,57 +408,47 @@ __global__ __launch_bounds__(kWalkBlock) void walk_kernel(WalkArgs a) {
             pending_back = true;
           } else {
             cur = v_app;  // walk.hpp:1018-1023
-            cur_rb = next_rb;
-            cur_deg = (uint32_t)(next_re - next_rb);
-            ++nmove;
+            cur_rb = dg_row_begin(next_row);
+            cur_deg = dg_row_degree(next_row);
+            cur_stuck = dg_row_stuck(next_row);
+            if (cur_deg == kRowDegMax) {  // the packed degree is full: read the row
+              cur_deg = (uint32_t)(a.row_ptr[cur + 1] - cur_rb);
+              cur_stuck = false;
+            }
+            ++tot_move;
           }
         }
       }
     }
 
-    // ---- write finished walks out, cooperatively per wave ------------------
+    // ---- write finished walks out, each by its own lane -------------------
     // A walk of up to kPathLds vertices goes to its own slot of the raw buffer
-    // (walk index * kPathLds); longer walks take space after the slots from an
-    // overflow cursor.  No wave waits on a shared counter for a short walk.
-    const uint64_t fin = __ballot(finish);
-    if (fin != 0) {
-      uint64_t my_off = 0;
-      bool fits = true;
-      if (finish) {
-        tot_draw += ndraw;
-        tot_move += nmove;
-        tot_tok += len;
-        max_l = len > max_l ? len : max_l;
-        if (len <= (uint32_t)kPathLds) {
-          my_off = (uint64_t)wid * kPathLds;
+    // (walk index * kPathLds, whose place the packing knows); longer walks
+    // take space after the slots from an overflow cursor.  No wave waits on a
+    // shared counter for a short walk.
+    if (finish) {
+      tot_tok += len;
+      max_l = len > max_l ? len : max_l;
+      a.walk_len[wid] = len;
+      if (len <= (uint32_t)kPathLds) {
+        uint4* dst = reinterpret_cast<uint4*>(a.tokens + (uint64_t)wid * kPathLds);
+#pragma unroll
+        for (int j = 0; j < kPathVec; ++j) dst[j] = s_path[j * kWalkBlock + threadIdx.x];
+      } else {
+        const uint64_t off = a.slots_end + atomicAdd(&a.q->cursor, (unsigned long long)len);
+        a.walk_off[wid] = off;
+        if (off + len <= a.tok_cap) {
+          for (uint32_t j = 0; j < (uint32_t)kPathLds; ++j)
+            a.tokens[off + j] = path[(j >> 2) * (kWalkBlock * 4) + (j & 3u)];
+          for (uint32_t j = kPathLds; j < len; ++j) a.tokens[off + j] = spill[j - kPathLds];
         } else {
-          my_off = a.slots_end + atomicAdd(&a.q->cursor, (unsigned long long)len);
-          fits = my_off + len <= a.tok_cap;
-          if (!fits) atomicOr(&a.q->flags, DG_QFLAG_TOKEN_OVERFLOW);
+          atomicOr(&a.q->flags, DG_QFLAG_TOKEN_OVERFLOW);
         }
-        a.walk_off[wid] = my_off;
-        a.walk_len[wid] = len;
       }
-      __builtin_amdgcn_wave_barrier();
-      uint64_t mm = fin & __ballot(fits);
-      const uint32_t* wave_path = s_path + (threadIdx.x - lane) * kPathLds;
-      while (mm != 0) {
-        const int L = __builtin_ctzll(mm);
-        mm &= mm - 1;
-        const uint32_t n = __shfl(len, L, 64);
-        const unsigned long long off = __shfl((unsigned long long)my_off, L, 64);
-        const uint32_t nl = n < (uint32_t)kPathLds ? n : (uint32_t)kPathLds;
-        const uint32_t* src = wave_path + L * kPathLds;
-        // lane j < nl holds token j (nl <= kPathLds < 64)
-        const uint32_t v = (uint32_t)lane < nl ? src[lane] : 0xffffffffu;
-        if ((uint32_t)lane < nl) a.tokens[off + lane] = v;
-      }
-      if (finish && fits)  // the spilled tail, by its own lane
-        for (uint32_t j = kPathLds; j < len; ++j) a.tokens[my_off + j] = spill[j - kPathLds];
-      if (finish) active = false;
+      active = false;
     }
   }
-  // ---- the lane totals, one atomic each per wave
+  // ---- the lane totals, added to the shard once per wave
   const uint64_t wd = wave_sum_u64(tot_draw), wm = wave_sum_u64(tot_move), wt = wave_sum_u64(tot_tok);
   uint32_t wmax = max_l;
   for (int d = 32; d >= 1; d >>= 1) {
@@ -326,10 +456,28 @@ __global__ __launch_bounds__(kWalkBlock) void walk_kernel(WalkArgs a) {
     wmax = o > wmax ? o : wmax;
   }
   if (lane == 0) {
-    if (wd) atomicAdd(&a.q->draws, (unsigned long long)wd);
-    if (wm) atomicAdd(&a.q->moves, (unsigned long long)wm);
-    if (wt) atomicAdd(&a.q->tokens, (unsigned long long)wt);
-    if (wmax) atomicMax(&a.q->max_len, wmax);
+    if (wd) atomicAdd(&shard->draws, (unsigned long long)wd);
+    if (wm) atomicAdd(&shard->moves, (unsigned long long)wm);
+    if (wt) atomicAdd(&shard->tokens, (unsigned long long)wt);
+    if (wmax) atomicMax(&shard->max_len, wmax);
+  }
+}
+
+// The shards' totals into the queue; one wavefront.
+__global__ __launch_bounds__(64) void queue_sum_kernel(const dg_walk_shard* shards, dg_walk_queue* q) {
+  static_assert(kWalkShards == 64, "a lane per shard");
+  const dg_walk_shard s = shards[threadIdx.x];
+  const uint64_t draws = wave_sum_u64(s.draws), moves = wave_sum_u64(s.moves), tokens = wave_sum_u64(s.tokens);
+  uint32_t most = s.max_len;
+  for (int d = 32; d >= 1; d >>= 1) {
+    const uint32_t o = __shfl_xor(most, d, 64);
+    most = o > most ? o : most;
+  }
+  if (threadIdx.x == 0) {
+    q->draws = draws;
+    q->moves = moves;
+    q->tokens = tokens;
+    q->max_len = most;
   }
 }
 
@@ -346,18 +494,9 @@ __global__ void zero_first_kernel(uint64_t* p) {
   if (threadIdx.x == 0 && blockIdx.x == 0) p[0] = 0;
 }
 
-__global__ void queue_reset_kernel(dg_walk_queue* q) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) {
-    q->next = 0;
-    q->cursor = 0;
-    q->flags = 0;
-    q->max_len = 0;
-    q->zero_terms = 0;
-    q->re = 0.0;
-    q->draws = 0;
-    q->moves = 0;
-    q->tokens = 0;
-  }
+__global__ __launch_bounds__(64) void queue_reset_kernel(dg_walk_queue* q, dg_walk_shard* shards) {
+  shards[threadIdx.x] = dg_walk_shard{};
+  if (threadIdx.x == 0) *q = dg_walk_queue{};
 }
 
 __global__ void fill_u32_kernel(uint32_t* p, uint64_t n, uint32_t v) {
@@ -486,7 +625,7 @@ __global__ __launch_bounds__(kPackBlock) void pack_count_kernel(
       w[u] = w0 + (uint64_t)(2 * u + half);
       const bool ok = w[u] < n_walks;
       len[u] = ok ? walk_len[w[u]] : 0u;
-      src[u] = ok ? walk_off[w[u]] : 0ull;
+      src[u] = len[u] <= (uint32_t)kPathLds ? w[u] * kPathLds : walk_off[w[u]];
       dst[u] = ok ? out_off[w[u]] : 0ull;
     }
     // chunks of 32 tokens; the count is made wave-uniform so that both halves
@@ -725,8 +864,8 @@ extern "C" int dg_walk_reset(dg_ctx* ctx) {
     DG_HIP(ctx, hipMalloc((void**)&ctx->d_freq, sizeof(uint32_t) * ctx->v_num));
   }
   if (!ctx->d_term_table) {
-    DG_HIP(ctx, hipMalloc((void**)&ctx->d_term_table, sizeof(double) * kTermTable * kTermStride));
-    term_table_kernel<<<(kTermTable * kTermStride + 255) / 256, 256, 0, ctx->stream>>>(
+    DG_HIP(ctx, hipMalloc((void**)&ctx->d_term_table, sizeof(double) * kTabWords));
+    term_table_kernel<<<(kTermWords + 255) / 256, 256, 0, ctx->stream>>>(
         ctx->d_term_table);
     DG_HIP(ctx, hipGetLastError());
   }
@@ -815,6 +954,7 @@ static int plan_round(dg_ctx* ctx, const dg_walk_params* p, uint32_t round,
   a.walk_len = ctx->d_walk_len;
   a.spill = ctx->d_spill;
   a.q = ctx->d_queue;
+  a.shards = ctx->d_shards;
   a.slots_end = slots_end;
   a.tokens = ctx->d_tok_raw;
   a.tok_cap = ctx->tok_raw_cap;
@@ -828,12 +968,14 @@ static int plan_round(dg_ctx* ctx, const dg_walk_params* p, uint32_t round,
 
 // The walk itself: queue reset and the persistent launch.
 static int enqueue_walk(dg_ctx* ctx, const dg_walk_plan& pl, bool timed) {
-  queue_reset_kernel<<<1, 64, 0, ctx->stream>>>(ctx->d_queue);
+  queue_reset_kernel<<<1, 64, 0, ctx->stream>>>(ctx->d_queue, ctx->d_shards);
   size_t tk = 0;
   if (timed) DG_CHECK(dg_time_begin(ctx, "walk", &tk));
   walk_kernel<<<(unsigned)pl.blocks, kWalkBlock, 0, ctx->stream>>>(pl.a);
   DG_HIP(ctx, hipGetLastError());
   if (timed) DG_CHECK(dg_time_end(ctx, tk));
+  queue_sum_kernel<<<1, 64, 0, ctx->stream>>>(ctx->d_shards, ctx->d_queue);
+  DG_HIP(ctx, hipGetLastError());
   return DG_OK;
 }
 

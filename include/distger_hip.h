@@ -103,7 +103,7 @@ int dg_graph_get_thresholds(dg_ctx* ctx, uint32_t* thr);
 
 /* Safety limit on vertices per walk when dg_walk_params.length_limit is 0.
  * The reference has no limit (walk.hpp:979-985); a walk that reaches it ends
- * the round with DG_ERR_WALK_TOO_LONG.  The walker keeps (limit - 23)
+ * the round with DG_ERR_WALK_TOO_LONG.  The walker keeps (limit - 24)
  * vertices of spill space per resident lane. */
 #define DG_WALK_LENGTH_LIMIT_DEFAULT 1024
 
@@ -140,8 +140,8 @@ typedef struct {
   double total_ms;       /* device time of the whole round */
   uint32_t max_walk_len; /* longest walk of the round */
   uint32_t stop;         /* 1 if the round driver stops after this round */
-  uint64_t draws;        /* candidate draws (8-byte adjacency units read) */
-  uint64_t moves;        /* row-offset pairs read (walk starts + moves) */
+  uint64_t draws;        /* candidate draws (16-byte adjacency units read) */
+  uint64_t moves;        /* rows entered (walk starts + moves) */
 } dg_round_stats;
 
 /* Run one round: walks walker_begin .. walker_begin+walker_num-1 (start vertex
