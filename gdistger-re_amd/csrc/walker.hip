@@ -581,88 +581,173 @@ __global__ __launch_bounds__(kScanBlock) void scan_tile_apply(const uint32_t* le
 }
 
 // ---- corpus packing in walk-id order, and the round's visit counts ------
-// (path.hpp:91,95: context_map_freq / vertex_cn).  A half-wavefront (32
-// lanes) copies one walk at a time, two walks per pass, in chunks of 32
-// tokens.  It sorts the chunk across its lanes (bitonic network), so equal
-// vertices become runs, and counts each distinct vertex once with its
-// multiplicity (walks revisit their hub at every other step): a hot vertex
-// (hot_slot != kNotHot) in this workgroup's LDS counters, written out as one
-// partial row at the end, any other vertex with a global atomic.  The
-// partial rows are gridDim.x x n_hot.
-constexpr int kPackBlock = 256;
-constexpr int kPackWalks = 2;  // walks per half-wavefront per pass
+// (path.hpp:91,95: context_map_freq / vertex_cn).  A wavefront takes 64
+// consecutive walks, a lane each: the walk's slot is read into registers
+// (six 16-byte loads), each of its distinct vertices counted once with its
+// multiplicity (walks revisit their hub at every other step; equal pairs are
+// found by comparing registers), and the 64 walks, which are one run of the
+// packed corpus, leave through LDS as one coalesced copy.  A hot vertex
+// (hot_slot != kNotHot) is counted in this workgroup's LDS counters, written
+// out as one partial row at the end.
+//
+// The other vertices are what the counting costs: an atomic each on a random
+// counter goes at about 30 G/s however the counters are spread (0.33 of the
+// 0.45 ms of a 1.31M-walk round, the same with a counter array per XCD).  So
+// with BIN a tile of walks sorts its (vertex, multiplicity) entries
+// into kBins bins by vertex in LDS, and writes them over its own slots in the
+// raw buffer (all read by then), with the bins' offsets in bin_off; a
+// workgroup of bin_count_kernel then adds up the entries of one bin of many
+// tiles in LDS counters.  That takes graphs whose vertices fit the bins'
+// counters (kBinVertices); larger ones keep the atomics.
+// Walks longer than a slot are copied and counted by the whole wavefront.
+// The workgroup's threads are the tile's walks: 1,024 (a workgroup per CU), or
+// 256 where a round has fewer walks than that fills the CUs with.
+constexpr int kPackBig = 1024, kPackSmall = 256;
+constexpr int kBins = 128;
+constexpr uint32_t kBinCounters = 32768;  // counters of a bin: 128 KB of LDS
+constexpr uint32_t kBinVertices = kBins * kBinCounters;
 
-__device__ __forceinline__ uint32_t bitonic32(uint32_t x, uint32_t hl) {
-#pragma unroll
-  for (int k = 2; k <= 32; k <<= 1) {
-#pragma unroll
-    for (int j = k >> 1; j > 0; j >>= 1) {
-      const uint32_t y = __shfl_xor(x, j, 32);
-      const bool up = (hl & (uint32_t)k) == 0;
-      const bool lower = (hl & (uint32_t)j) == 0;
-      x = (lower == up) ? (x < y ? x : y) : (x < y ? y : x);
-    }
-  }
-  return x;
+// Bin and place in it of a vertex: runs of 16 counters (64 bytes of the
+// visit counts) go to the bins in turn, so that neighbouring ids, which often
+// have similar degrees, spread over the bins.
+__host__ __device__ __forceinline__ uint32_t bin_of(uint32_t v) { return (v >> 4) % kBins; }
+__host__ __device__ __forceinline__ uint32_t bin_place(uint32_t v) { return (v >> 4) / kBins * 16u + (v & 15u); }
+__host__ __device__ __forceinline__ uint32_t bin_vertex(uint32_t bin, uint32_t place) {
+  return ((place >> 4) * kBins + bin) * 16u + (place & 15u);
 }
 
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+template <int kPackBlock, bool BIN>
 __global__ __launch_bounds__(kPackBlock) void pack_count_kernel(
-    const uint32_t* raw, const uint64_t* walk_off, const uint32_t* walk_len, const uint64_t* out_off,
+    uint32_t* raw, const uint64_t* walk_off, const uint32_t* walk_len, const uint64_t* out_off,
     uint64_t n_walks, uint32_t* tokens, const uint16_t* hot_slot, uint32_t n_hot, uint32_t* freq,
-    uint32_t* hot_part) {
+    uint32_t* hot_part, uint32_t* bin_off) {
   __shared__ uint32_t s_hot[kHotMax];
+  __shared__ uint32_t s_out[kPackBlock * kPathLds];
+  __shared__ uint32_t s_bin[kBins], s_first[kBins + 1];
   for (uint32_t k = threadIdx.x; k < n_hot; k += kPackBlock) s_hot[k] = 0;
+  if (threadIdx.x < kBins) s_bin[threadIdx.x] = 0;
   __syncthreads();
-  const uint32_t lane = threadIdx.x & 63u, hl = lane & 31u, half = lane >> 5;
-  const uint64_t wave = ((uint64_t)blockIdx.x * kPackBlock + threadIdx.x) >> 6;
-  const uint64_t nwaves = ((uint64_t)gridDim.x * kPackBlock) >> 6;
-  const uint64_t per_pass = 2 * kPackWalks;  // walks per wavefront per pass
-  for (uint64_t w0 = wave * per_pass; w0 < n_walks; w0 += nwaves * per_pass) {
-    uint64_t w[kPackWalks], src[kPackWalks], dst[kPackWalks];
-    uint32_t len[kPackWalks];
+  const uint32_t lane = threadIdx.x & 63u, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  uint32_t* out = s_out + wv * (64 * kPathLds);
+  const uint64_t n_tiles = (n_walks + kPackBlock - 1) / kPackBlock;
+  for (uint64_t tile = blockIdx.x; tile < n_tiles; tile += gridDim.x) {
+    const uint64_t w0 = tile * kPackBlock + wv * 64;
+    const uint64_t w = w0 + lane;
+    const bool ok = w < n_walks;
+    const uint32_t len = ok ? walk_len[w] : 0u;
+    const uint64_t dst = ok ? out_off[w] : 0ull;
+    const uint64_t base = __shfl(dst, 0, 64);
+    const uint64_t too_long = __ballot(len > (uint32_t)kPathLds);
+    const bool mine = ok && len <= (uint32_t)kPathLds;
+    uint32_t t[kPathLds];
+    // entry of the vertex at place i (BIN): multiplicity, and above it its
+    // rank in the tile's bin; 0 where it is not a bin's entry
+    uint32_t n[kPathLds];
+    if (mine) {
+      const uint4* slot = reinterpret_cast<const uint4*>(raw + w * kPathLds);
 #pragma unroll
-    for (int u = 0; u < kPackWalks; ++u) {
-      w[u] = w0 + (uint64_t)(2 * u + half);
-      const bool ok = w[u] < n_walks;
-      len[u] = ok ? walk_len[w[u]] : 0u;
-      src[u] = len[u] <= (uint32_t)kPathLds ? w[u] * kPathLds : walk_off[w[u]];
-      dst[u] = ok ? out_off[w[u]] : 0ull;
+      for (int j = 0; j < kPathVec; ++j) {
+        const uint4 q = slot[j];
+        t[4 * j] = q.x;
+        t[4 * j + 1] = q.y;
+        t[4 * j + 2] = q.z;
+        t[4 * j + 3] = q.w;
+      }
+      // occurrences of the vertex at i from i on, and whether i is its first
+      uint32_t again = 0;
+#pragma unroll
+      for (int i = 0; i < kPathLds; ++i) n[i] = 1;
+#pragma unroll
+      for (int i = 0; i < kPathLds; ++i)
+#pragma unroll
+        for (int j = i + 1; j < kPathLds; ++j) {
+          const bool same = t[i] == t[j];
+          n[i] += same ? 1u : 0u;
+          again |= same ? 1u << j : 0u;
+        }
+#pragma unroll
+      for (int i = 0; i < kPathLds; ++i) {
+        if ((uint32_t)i >= len || ((again >> i) & 1u)) {
+          n[i] = 0;
+          continue;
+        }
+        const uint16_t hs = hot_slot[t[i]];
+        if (hs != kNotHot) {
+          atomicAdd(&s_hot[hs], n[i]);
+          n[i] = 0;
+        } else if constexpr (BIN) {
+          n[i] |= atomicAdd(&s_bin[bin_of(t[i])], 1u) << 8;
+        } else {
+          atomicAdd(&freq[t[i]], n[i]);
+        }
+      }
+      if (too_long == 0) {
+        const uint32_t o = (uint32_t)(dst - base);
+#pragma unroll
+        for (int i = 0; i < kPathLds; ++i)
+          if ((uint32_t)i < len) out[o + i] = t[i];
+      } else {
+#pragma unroll
+        for (int i = 0; i < kPathLds; ++i)
+          if ((uint32_t)i < len) tokens[dst + i] = t[i];
+      }
     }
-    // chunks of 32 tokens; the count is made wave-uniform so that both halves
-    // take part in every shuffle
-    uint32_t nch = 0;
+    if (too_long == 0) {
+      uint32_t total = len;
 #pragma unroll
-    for (int u = 0; u < kPackWalks; ++u) nch = max(nch, (len[u] + 31u) >> 5);
-    nch = max(nch, (uint32_t)__shfl_xor((int)nch, 32, 64));
-    for (uint32_t c = 0; c < nch; ++c) {
-      uint32_t x[kPackWalks], nvalid[kPackWalks];
-#pragma unroll
-      for (int u = 0; u < kPackWalks; ++u) {
-        const uint32_t j = c * 32u + hl;
-        nvalid[u] = len[u] > c * 32u ? min(len[u] - c * 32u, 32u) : 0u;
-        x[u] = 0xffffffffu;
-        if (j < len[u]) {
-          x[u] = raw[src[u] + j];
-          tokens[dst[u] + j] = x[u];
-        }
+      for (int d = 32; d >= 1; d >>= 1) total += __shfl_xor(total, d, 64);
+      wave_lds_sync();
+      for (uint32_t i = lane; i < total; i += 64) tokens[base + i] = out[i];
+      wave_lds_sync();
+    }
+    for (uint64_t m = too_long; m != 0; m &= m - 1) {
+      const int l = __builtin_ctzll(m);
+      const uint64_t src = walk_off[w0 + l], d = __shfl(dst, l, 64);
+      const uint32_t nl = __shfl(len, l, 64);
+      for (uint32_t i = lane; i < nl; i += 64) {
+        const uint32_t v = raw[src + i];
+        tokens[d + i] = v;
+        const uint16_t hs = hot_slot[v];
+        if (hs != kNotHot)
+          atomicAdd(&s_hot[hs], 1u);
+        else
+          atomicAdd(&freq[v], 1u);
       }
+    }
+    if constexpr (BIN) {
+      __syncthreads();  // every rank is taken, every slot of the tile read
+      if (wv == 0) {
+        static_assert(kBins == 128, "two bins per lane");
+        const uint32_t c0 = s_bin[2 * lane], c1 = s_bin[2 * lane + 1];
+        uint32_t inc = c0 + c1;
 #pragma unroll
-      for (int u = 0; u < kPackWalks; ++u) {
-        const uint32_t y = bitonic32(x[u], hl);
-        const uint32_t prev = __shfl_up(y, 1, 32);
-        const bool head = hl < nvalid[u] && (hl == 0 || prev != y);
-        const uint32_t hmask = (uint32_t)(__ballot(head) >> (32 * half));
-        if (head) {
-          const uint32_t above = hmask & ~((2u << hl) - 1u);
-          const uint32_t next = above ? (uint32_t)__builtin_ctz(above) : nvalid[u];
-          const uint32_t cnt = next - hl;
-          const uint16_t hs = hot_slot[y];
-          if (hs != kNotHot)
-            atomicAdd(&s_hot[hs], cnt);
-          else
-            atomicAdd(&freq[y], cnt);
+        for (int d = 1; d < 64; d <<= 1) {
+          const uint32_t u = __shfl_up(inc, d, 64);
+          if ((int)lane >= d) inc += u;
         }
+        s_first[2 * lane] = inc - c0 - c1;
+        s_first[2 * lane + 1] = inc - c1;
+        if (lane == 63) s_first[kBins] = inc;
+        s_bin[2 * lane] = 0;
+        s_bin[2 * lane + 1] = 0;
       }
+      __syncthreads();
+      if (mine) {
+#pragma unroll
+        for (int i = 0; i < kPathLds; ++i)
+          if (n[i]) s_out[s_first[bin_of(t[i])] + (n[i] >> 8)] = bin_place(t[i]) | (n[i] & 0xffu) << 16;
+      }
+      if (threadIdx.x <= kBins) bin_off[tile * (kBins + 1) + threadIdx.x] = s_first[threadIdx.x];
+      __syncthreads();
+      const uint32_t total = s_first[kBins];
+      for (uint32_t i = threadIdx.x; i < total; i += kPackBlock) raw[tile * (kPackBlock * kPathLds) + i] = s_out[i];
+      __syncthreads();  // s_out is the next tile's
     }
   }
   __syncthreads();
@@ -670,10 +755,39 @@ __global__ __launch_bounds__(kPackBlock) void pack_count_kernel(
     hot_part[(uint64_t)blockIdx.x * n_hot + k] = s_hot[k];
 }
 
+// Workgroup (bin, part): the bin's entries of its share of the tiles, a
+// wavefront per tile, added up in LDS and then to the visit counts.  Entries: place, and the multiplicity from bit 16.
+constexpr int kBinBlock = 1024;
+
+__global__ __launch_bounds__(kBinBlock) void bin_count_kernel(const uint32_t* raw, const uint32_t* bin_off,
+                                                              uint64_t n_tiles, uint32_t tile_words, uint32_t v_num, uint32_t places,
+                                                              uint32_t* freq) {
+  extern __shared__ uint32_t s_cnt[];
+  const uint32_t bin = blockIdx.x;
+  for (uint32_t i = threadIdx.x; i < places; i += kBinBlock) s_cnt[i] = 0;
+  __syncthreads();
+  const uint32_t lane = threadIdx.x & 63u, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  constexpr uint32_t waves = kBinBlock / 64;
+  for (uint64_t tile = (uint64_t)blockIdx.y * waves + wv; tile < n_tiles; tile += (uint64_t)gridDim.y * waves) {
+    const uint32_t lo = bin_off[tile * (kBins + 1) + bin], hi = bin_off[tile * (kBins + 1) + bin + 1];
+    const uint32_t* e = raw + tile * tile_words;
+    for (uint32_t i = lo + lane; i < hi; i += 64) {
+      const uint32_t x = e[i];
+      atomicAdd(&s_cnt[x & 0xffffu], x >> 16);
+    }
+  }
+  __syncthreads();
+  for (uint32_t i = threadIdx.x; i < places; i += kBinBlock) {
+    const uint32_t v = bin_vertex(bin, i), c = s_cnt[i];
+    if (c && v < v_num) atomicAdd(&freq[v], c);
+  }
+}
+
 // Hot-vertex counts: the partial rows summed per slot.  Grid (slots / 64,
-// rows / 64): each thread adds 64 partial rows of one slot (coalesced across
-// the slots of a wavefront) and adds that to the vertex's count.
-constexpr uint32_t kHotRows = 64;
+// rows / kHotRows): each thread adds kHotRows partial rows of one slot
+// (coalesced across the slots of a wavefront, all loads in flight) and adds
+// that to the vertex's count.
+constexpr uint32_t kHotRows = 32;
 
 __global__ __launch_bounds__(64) void hot_reduce_kernel(const uint32_t* hot_part, uint32_t n_parts,
                                                         uint32_t n_hot, const uint32_t* hot_id,
@@ -681,9 +795,12 @@ __global__ __launch_bounds__(64) void hot_reduce_kernel(const uint32_t* hot_part
   const uint32_t k = blockIdx.x * 64 + threadIdx.x;
   if (k >= n_hot) return;
   const uint32_t b0 = blockIdx.y * kHotRows;
-  const uint32_t b1 = b0 + kHotRows < n_parts ? b0 + kHotRows : n_parts;
+  uint32_t v[kHotRows];
+#pragma unroll
+  for (uint32_t r = 0; r < kHotRows; ++r) v[r] = b0 + r < n_parts ? hot_part[(uint64_t)(b0 + r) * n_hot + k] : 0u;
   uint32_t c = 0;
-  for (uint32_t b = b0; b < b1; ++b) c += hot_part[(uint64_t)b * n_hot + k];
+#pragma unroll
+  for (uint32_t r = 0; r < kHotRows; ++r) c += v[r];
   if (c) atomicAdd(&freq[hot_id[k]], c);
 }
 
@@ -733,7 +850,8 @@ __global__ __launch_bounds__(kReBlock) void re_chunks_kernel(const uint32_t* deg
   for (uint32_t k = 0; k < kReChunk / kReBlock; ++k) {
     const uint32_t j = k * kReBlock + threadIdx.x;
     if (j >= n) break;
-    const uint32_t d = deg[lo + j], f = freq[lo + j];
+    const uint32_t d = deg[lo + j];
+    const uint32_t f = freq[lo + j];
     double t = 0.0;
     if (d == 0 || f == 0) {
       ++zeros;
@@ -774,6 +892,9 @@ __global__ void offsets_shift_kernel(const uint64_t* src, uint64_t n, uint64_t a
     dst[i] = src[i] + add;
 }
 
+// Places of a bin that a vertex below v_num can have.
+uint32_t bin_places(uint32_t v_num) { return ((v_num - 1) / (16u * kBins) + 1u) * 16u; }
+
 int grid_for(dg_ctx* ctx, uint64_t n, int block) {
   uint64_t g = (n + block - 1) / block;
   uint64_t cap = (uint64_t)ctx->num_cus * 16;
@@ -788,6 +909,9 @@ struct dg_walk_plan {
   WalkArgs a;
   uint64_t blocks = 0;        // walk_kernel grid
   uint32_t parts = 0;         // pack_count_kernel grid
+  uint32_t pack_block = 0;    // and its workgroup
+  bool bins = false;          // visits counted by bins (else by atomics)
+  uint32_t bin_parts = 1;     // bin_count_kernel workgroups per bin
   uint32_t round = 0;
   uint32_t walker_num = 0;
   uint32_t length_limit = 0;
@@ -798,7 +922,7 @@ struct dg_walk_plan {
 void dg_walk_free(dg_ctx* ctx) {
   void* bufs[] = {ctx->d_freq,   ctx->d_tok_raw,  ctx->d_walk_off, ctx->d_walk_len,
                   ctx->d_tokens, ctx->d_offsets,  ctx->d_spill,    ctx->d_scan_tmp,
-                  ctx->d_re_chunks, ctx->d_train_tokens, ctx->d_train_offsets,
+                  ctx->d_re_chunks, ctx->d_bin_off, ctx->d_train_tokens, ctx->d_train_offsets,
                   ctx->d_term_table};
   for (void* p : bufs)
     if (p) hipFree(p);
@@ -811,13 +935,14 @@ void dg_walk_free(dg_ctx* ctx) {
   ctx->d_spill = nullptr;
   ctx->d_scan_tmp = nullptr;
   ctx->d_re_chunks = nullptr;
+  ctx->d_bin_off = nullptr;
   ctx->d_train_tokens = nullptr;
   ctx->d_train_offsets = nullptr;
   ctx->d_term_table = nullptr;
   delete ctx->wplan;
   ctx->wplan = nullptr;
   ctx->tok_raw_cap = ctx->walk_cap = ctx->walk_len_cap = ctx->tokens_cap = ctx->offsets_cap = 0;
-  ctx->spill_cap = ctx->scan_tmp_cap = ctx->re_cap = 0;
+  ctx->spill_cap = ctx->scan_tmp_cap = ctx->re_cap = ctx->bin_off_cap = 0;
   ctx->train_tokens_cap = ctx->train_offsets_cap = 0;
   ctx->train_walks = ctx->train_tokens = 0;
   ctx->cur_walks = ctx->cur_tokens = 0;
@@ -921,13 +1046,20 @@ static int plan_round(dg_ctx* ctx, const dg_walk_params* p, uint32_t round,
   size_t tok_need = (size_t)slots_end + (size_t)walker_num / 8 + 4096;
   if (ctx->tok_raw_cap < tok_need) DG_CHECK(dg_reserve(ctx, &ctx->d_tok_raw, &ctx->tok_raw_cap, tok_need));
   {
-    // packing: every resident workgroup slot (LDS: n_hot counters each), fewer for small rounds
-    int pcu = 0;
-    DG_HIP(ctx, hipOccupancyMaxActiveBlocksPerMultiprocessor(&pcu, pack_count_kernel, kPackBlock, 0));
-    if (pcu < 1) pcu = 1;
-    const uint64_t per_wg = (uint64_t)(kPackBlock / 64) * 2 * kPackWalks;  // walks per workgroup pass
-    const uint64_t need = ((uint64_t)walker_num + per_wg - 1) / per_wg;
-    pl->parts = (uint32_t)std::min<uint64_t>((uint64_t)ctx->num_cus * pcu, need ? need : 1);
+    // packing: a workgroup of 1,024 walks per CU (LDS: the hot counters and 96 KB of tokens)
+    pl->pack_block = walker_num < (uint64_t)ctx->num_cus * kPackBig ? kPackSmall : kPackBig;
+    const uint64_t n_tiles = std::max<uint64_t>(1, ((uint64_t)walker_num + pl->pack_block - 1) / pl->pack_block);
+    pl->parts = (uint32_t)std::min<uint64_t>((uint64_t)ctx->num_cus, n_tiles);
+    pl->bins = ctx->v_num <= kBinVertices;
+    if (pl->bins) {
+      DG_CHECK(dg_reserve(ctx, &ctx->d_bin_off, &ctx->bin_off_cap, (size_t)(n_tiles * (kBins + 1))));
+      // two workgroups of 1,024 threads per CU, fewer where their LDS does not fit
+      const size_t lds = sizeof(uint32_t) * bin_places(ctx->v_num);
+      DG_HIP(ctx, hipFuncSetAttribute((const void*)bin_count_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                      (int)lds));
+      const uint64_t fill = (uint64_t)ctx->num_cus * (lds <= 80 * 1024 ? 2 : 1) / kBins;
+      pl->bin_parts = (uint32_t)std::max<uint64_t>(1, std::min(fill, n_tiles));
+    }
     DG_CHECK(dg_reserve(ctx, &ctx->d_hot_part, &ctx->hot_part_cap,
                         (size_t)pl->parts * (ctx->n_hot ? ctx->n_hot : 1)));
   }
@@ -988,9 +1120,21 @@ static int enqueue_tail(dg_ctx* ctx, const dg_walk_plan& pl, bool timed) {
   size_t tp = 0;
   if (timed) DG_CHECK(dg_time_begin(ctx, "pack", &tp));
   DG_CHECK(dg_scan_lengths(ctx, ctx->d_walk_len, walker_num, ctx->d_offsets));
-  pack_count_kernel<<<pl.parts, kPackBlock, 0, ctx->stream>>>(
-      ctx->d_tok_raw, ctx->d_walk_off, ctx->d_walk_len, ctx->d_offsets, walker_num, ctx->d_tokens,
-      ctx->d_hot_slot, ctx->n_hot, ctx->d_freq, ctx->d_hot_part);
+  const auto pack = [&](auto kern) {
+    kern<<<pl.parts, pl.pack_block, 0, ctx->stream>>>(
+        ctx->d_tok_raw, ctx->d_walk_off, ctx->d_walk_len, ctx->d_offsets, walker_num, ctx->d_tokens,
+        ctx->d_hot_slot, ctx->n_hot, ctx->d_freq, ctx->d_hot_part, ctx->d_bin_off);
+  };
+  const bool big = pl.pack_block == (uint32_t)kPackBig;
+  if (pl.bins) {
+    big ? pack(pack_count_kernel<kPackBig, true>) : pack(pack_count_kernel<kPackSmall, true>);
+    const uint64_t n_tiles = ((uint64_t)walker_num + pl.pack_block - 1) / pl.pack_block;
+    const uint32_t places = bin_places(ctx->v_num);
+    bin_count_kernel<<<dim3(kBins, pl.bin_parts), kBinBlock, sizeof(uint32_t) * places, ctx->stream>>>(
+        ctx->d_tok_raw, ctx->d_bin_off, n_tiles, pl.pack_block * kPathLds, ctx->v_num, places, ctx->d_freq);
+  } else {
+    big ? pack(pack_count_kernel<kPackBig, false>) : pack(pack_count_kernel<kPackSmall, false>);
+  }
   if (ctx->n_hot) {
     const dim3 grid((ctx->n_hot + 63) / 64, (pl.parts + kHotRows - 1) / kHotRows);
     hot_reduce_kernel<<<grid, 64, 0, ctx->stream>>>(ctx->d_hot_part, pl.parts, ctx->n_hot,

@@ -1,5 +1,5 @@
-"""The walk kernel at the edges of its layout, against the CPU oracle: rounds
-of fewer walks than a wavefront up to more than the resident lanes (the
+"""The walk and packing kernels at the edges of their layout, against the CPU
+oracle (corpus and visit counts): rounds of fewer walks than a wavefront up to more than the resident lanes (the
 queue's shards), walks around the 24 vertices a lane holds and the 32
 tabulated lengths, rows whose degree does not fit an adjacency unit, and
 vertices a walk cannot leave."""
@@ -24,6 +24,7 @@ def _compare(ctx, p, rnd, begin, n, threads=8):
     dtok, doff = ctx.corpus()
     assert np.array_equal(doff, off)
     assert np.array_equal(dtok, tok)
+    assert np.array_equal(ctx.vertex_freq(), np.bincount(tok, minlength=g.v_num))  # after a reset
     if st is not None:
         assert st.tokens == len(tok) and st.max_walk_len == int(np.diff(off).max())
     return tok, off
@@ -66,3 +67,16 @@ def test_vertices_a_walk_cannot_leave(ctx):
     ctx.walk_reset()
     tok, off = _compare(ctx, ctx.default_walk_params(seed=9, min_length=5, max_length=50), 1, 0, 4000)
     assert len(np.unique(np.diff(off))) > 3
+
+
+@pytest.mark.parametrize("v,n", [(15, 100), (2047, 262143), (2049, 262145), (40000, 300000), (2 ** 22, 3000),
+                                 (2 ** 22 + 1, 3000)])
+def test_counts_by_bins(ctx, v, n):
+    """Bins of few and of the most counters, the first graph past them, and both tile sizes."""
+    print(f"[walk-kernel] counts of {n} walks on {v} vertices", flush=True)
+    edges = np.zeros(2 * v, ffi.EDGE_DTYPE)
+    edges["src"] = np.tile(np.arange(v), 2)
+    edges["dst"] = (edges["src"].astype(np.int64) + np.repeat([1, 5], v)) % v
+    ctx.graph_from_edges(v, edges, undirected=True, cn_mode=ffi.DG_CN_FROM_DATA)
+    ctx.walk_reset()
+    _compare(ctx, ctx.default_walk_params(seed=v, max_length=40, mu=0.99, min_length=8), 1, v // 2, n)
