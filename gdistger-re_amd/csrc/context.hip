@@ -51,6 +51,8 @@ extern "C" int dg_open(int device, dg_ctx** out) {
     dg_close(ctx);
     return DG_ERR_HIP;
   }
+  dg_hostcopy_open();
+  ctx->opened = true;
   *out = ctx;
   return DG_OK;
 }
@@ -75,6 +77,7 @@ extern "C" void dg_close(dg_ctx* ctx) {
   if (ctx->d_shards) hipFree(ctx->d_shards);
   if (ctx->h_queue) hipHostFree(ctx->h_queue);
   if (ctx->stream) hipStreamDestroy(ctx->stream);
+  if (ctx->opened) dg_hostcopy_close();
   delete ctx;
 }
 

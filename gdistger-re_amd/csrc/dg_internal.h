@@ -57,6 +57,7 @@ __host__ __device__ inline bool dg_row_stuck(uint2 r) { return (r.y >> 31) != 0u
 
 #define DG_QFLAG_TOKEN_OVERFLOW 1u
 #define DG_QFLAG_LENGTH_LIMIT 2u
+#define DG_QFLAG_NO_SPILL 4u  // a walk outgrew its LDS and no spill space was there
 
 struct dg_timing_entry {
   uint64_t launches = 0;
@@ -79,6 +80,7 @@ struct dg_ctx {
   int device = 0;
   int num_cus = 0;
   hipStream_t stream = nullptr;
+  bool opened = false;  // counted by dg_hostcopy_open
   std::string err;
 
   // graph (device-resident CSR)
@@ -116,6 +118,8 @@ struct dg_ctx {
   uint64_t* d_offsets = nullptr;     // n_walks + 1
   size_t offsets_cap = 0;
   uint32_t* d_spill = nullptr;       // per-lane overflow of the LDS path buffer
+  bool walks_spill = false;          // walks of this graph have outgrown the LDS
+  int walk_per_cu = 0;               // resident walk workgroups per CU
   size_t spill_cap = 0;
   uint64_t* d_scan_tmp = nullptr;    // block sums for scans
   size_t scan_tmp_cap = 0;
@@ -298,6 +302,12 @@ struct dg_dsgl_call {
 };
 int dg_dsgl_train(dg_ctx* ctx, const dg_dsgl_call& c, uint64_t* kept, double* ms, float* alpha_end);
 void dg_dsgl_free(dg_ctx* ctx);
+
+// Copies device memory to the caller's pageable buffer, after the context's
+// queued work, and returns when the bytes are there (hostcopy.hip).
+int dg_copy_to_host(dg_ctx* ctx, void* dst, const void* src, size_t bytes);
+void dg_hostcopy_open();   // a context opened / closed: the last one gives the
+void dg_hostcopy_close();  // staging memory and threads back
 
 // Exclusive scan of n uint32 lengths into n+1 uint64 offsets (walker.hip).
 int dg_scan_lengths(dg_ctx* ctx, const uint32_t* d_len, uint64_t n, uint64_t* d_off);

@@ -973,12 +973,9 @@ extern "C" int dg_graph_get_csr(dg_ctx* ctx, uint64_t* row_ptr, uint32_t* nbr, u
   DG_HIP(ctx, hipSetDevice(ctx->device));
   DG_HIP(ctx, hipStreamSynchronize(ctx->stream));
   if (row_ptr)
-    DG_HIP(ctx, hipMemcpy(row_ptr, ctx->d_row_ptr, sizeof(uint64_t) * (ctx->v_num + 1),
-                          hipMemcpyDeviceToHost));
-  if (nbr && ctx->m)
-    DG_HIP(ctx, hipMemcpy(nbr, ctx->d_nbr, sizeof(uint32_t) * ctx->m, hipMemcpyDeviceToHost));
-  if (cn && ctx->m)
-    DG_HIP(ctx, hipMemcpy(cn, ctx->d_cn, sizeof(uint32_t) * ctx->m, hipMemcpyDeviceToHost));
+    DG_CHECK(dg_copy_to_host(ctx, row_ptr, ctx->d_row_ptr, sizeof(uint64_t) * (ctx->v_num + 1ull)));
+  if (nbr && ctx->m) DG_CHECK(dg_copy_to_host(ctx, nbr, ctx->d_nbr, sizeof(uint32_t) * ctx->m));
+  if (cn && ctx->m) DG_CHECK(dg_copy_to_host(ctx, cn, ctx->d_cn, sizeof(uint32_t) * ctx->m));
   return DG_OK;
 }
 
@@ -993,7 +990,6 @@ extern "C" int dg_graph_get_thresholds(dg_ctx* ctx, uint32_t* thr) {
   DG_HIP(ctx, mem.get(&d_thr, ctx->m));
   take_thresholds_kernel<<<grid_for(ctx, ctx->m, 256), 256, 0, ctx->stream>>>(ctx->d_adj, ctx->m, d_thr);
   DG_HIP(ctx, hipGetLastError());
-  DG_HIP(ctx, hipStreamSynchronize(ctx->stream));
-  DG_HIP(ctx, hipMemcpy(thr, d_thr, sizeof(uint32_t) * ctx->m, hipMemcpyDeviceToHost));
+  DG_CHECK(dg_copy_to_host(ctx, thr, d_thr, sizeof(uint32_t) * ctx->m));
   return DG_OK;
 }

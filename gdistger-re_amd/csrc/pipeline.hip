@@ -12,9 +12,9 @@
 // The host does not know the round's token count while the step is captured,
 // so every buffer is sized for any outcome and each kernel reads its extent
 // from the device (offsets, queue counters).  A round that overflows the
-// walker's token buffer, or hits the length limit, is emptied on the device
-// by round_guard_kernel; the rest of the step then changes nothing, the host
-// grows the buffer and runs the step again (the walks depend only on seed,
+// walker's token buffer or lacks spill space, or hits the length limit, is
+// emptied on the device by round_guard_kernel; the rest of the step then
+// changes nothing, the host grows the buffer and runs the step again (the walks depend only on seed,
 // round and walker id, so the second run walks the same walks).
 //
 // Kernel arguments change every call (round, epoch, learning rate), so the
@@ -107,7 +107,7 @@ extern "C" int dg_pipeline_step(dg_ctx* ctx, const dg_walk_params* wp, uint32_t 
   }
   dg_pipe_state* ps = ctx->pipe;
   DG_HIP(ctx, hipStreamSynchronize(ctx->stream));
-  for (int attempt = 0; attempt < 3; ++attempt) {
+  for (int attempt = 0; attempt < 4; ++attempt) {
     uint64_t tok_bound = 0, slot_tokens = 0, overflow_tokens = 0;
     DG_CHECK(dg_walk_graph_plan(ctx, wp, round, walker_begin, walker_num, &tok_bound, &slot_tokens,
                                 &overflow_tokens));

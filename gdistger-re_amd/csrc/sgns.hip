@@ -1385,9 +1385,9 @@ extern "C" int dg_sgns_init(dg_ctx* ctx, const dg_sgns_params* p) {
   DG_HIP(ctx, hipMalloc((void**)&s->d_expt, sizeof(float) * (kExpTable + 1)));
   DG_HIP(ctx, hipMalloc((void**)&s->d_keep, sizeof(uint32_t) * vocab));
   DG_HIP(ctx, hipMemcpy(s->d_rank, rank.data(), sizeof(uint32_t) * V, hipMemcpyHostToDevice));
-  DG_HIP(ctx, hipMemcpy(s->d_syn0, syn0.data(), sizeof(float) * nrow, hipMemcpyHostToDevice));
+  DG_HIP(ctx, hipMemcpyAsync(s->d_syn0, syn0.data(), sizeof(float) * nrow, hipMemcpyHostToDevice, ctx->stream));
   DG_HIP(ctx, hipMemset(s->d_syn1, 0, sizeof(float) * nrow));
-  DG_HIP(ctx, hipMemcpy(s->d_table, table.data(), sizeof(int32_t) * p->table_size, hipMemcpyHostToDevice));
+  DG_HIP(ctx, hipMemcpyAsync(s->d_table, table.data(), sizeof(int32_t) * p->table_size, hipMemcpyHostToDevice, ctx->stream));
   DG_HIP(ctx, hipMemcpy(s->d_expt, expt.data(), sizeof(float) * (kExpTable + 1), hipMemcpyHostToDevice));
   DG_HIP(ctx, hipMemcpy(s->d_keep, keep.data(), sizeof(uint32_t) * vocab, hipMemcpyHostToDevice));
   DG_HIP(ctx, hipStreamSynchronize(ctx->stream));
@@ -1419,8 +1419,9 @@ extern "C" int dg_sgns_tables_create(dg_ctx* ctx, uint32_t rows, uint32_t dim, c
   DG_HIP(ctx, hipMalloc((void**)&s->d_syn0, sizeof(float) * nrow));
   DG_HIP(ctx, hipMalloc((void**)&s->d_syn1, sizeof(float) * nrow));
   DG_HIP(ctx, hipMemcpy(s->d_rank, s->vertex_of_rank.data(), sizeof(uint32_t) * rows, hipMemcpyHostToDevice));
-  DG_HIP(ctx, hipMemcpy(s->d_syn0, syn0, sizeof(float) * nrow, hipMemcpyHostToDevice));
-  DG_HIP(ctx, hipMemcpy(s->d_syn1, syn1, sizeof(float) * nrow, hipMemcpyHostToDevice));
+  DG_HIP(ctx, hipMemcpyAsync(s->d_syn0, syn0, sizeof(float) * nrow, hipMemcpyHostToDevice, ctx->stream));
+  DG_HIP(ctx, hipMemcpyAsync(s->d_syn1, syn1, sizeof(float) * nrow, hipMemcpyHostToDevice, ctx->stream));
+  DG_HIP(ctx, hipStreamSynchronize(ctx->stream));
   dg_sgns_written(ctx);
   return DG_OK;
 }
@@ -2041,8 +2042,8 @@ extern "C" int dg_sgns_get_tables(dg_ctx* ctx, float* syn0, float* syn1) {
   DG_HIP(ctx, hipSetDevice(ctx->device));
   DG_HIP(ctx, hipStreamSynchronize(ctx->stream));
   const size_t n = (size_t)s->vocab * s->dim;
-  if (syn0) DG_HIP(ctx, hipMemcpy(syn0, s->d_syn0, sizeof(float) * n, hipMemcpyDeviceToHost));
-  if (syn1) DG_HIP(ctx, hipMemcpy(syn1, s->d_syn1, sizeof(float) * n, hipMemcpyDeviceToHost));
+  if (syn0) DG_CHECK(dg_copy_to_host(ctx, syn0, s->d_syn0, sizeof(float) * n));
+  if (syn1) DG_CHECK(dg_copy_to_host(ctx, syn1, s->d_syn1, sizeof(float) * n));
   return DG_OK;
 }
 
@@ -2052,8 +2053,8 @@ extern "C" int dg_sgns_set_tables(dg_ctx* ctx, const float* syn0, const float* s
   if (!s) return dg_fail(ctx, DG_ERR_STATE, "dg_sgns_init has not run");
   DG_HIP(ctx, hipSetDevice(ctx->device));
   const size_t n = (size_t)s->vocab * s->dim;
-  if (syn0) DG_HIP(ctx, hipMemcpy(s->d_syn0, syn0, sizeof(float) * n, hipMemcpyHostToDevice));
-  if (syn1) DG_HIP(ctx, hipMemcpy(s->d_syn1, syn1, sizeof(float) * n, hipMemcpyHostToDevice));
+  if (syn0) DG_HIP(ctx, hipMemcpyAsync(s->d_syn0, syn0, sizeof(float) * n, hipMemcpyHostToDevice, ctx->stream));
+  if (syn1) DG_HIP(ctx, hipMemcpyAsync(s->d_syn1, syn1, sizeof(float) * n, hipMemcpyHostToDevice, ctx->stream));
   DG_HIP(ctx, hipStreamSynchronize(ctx->stream));
   dg_sgns_written(ctx);
   return DG_OK;
@@ -2075,12 +2076,12 @@ extern "C" int dg_sgns_score_pairs(dg_ctx* ctx, const uint32_t* src, const uint3
   DG_HIP(ctx, hipMalloc((void**)&ds, sizeof(uint32_t) * n));
   DG_HIP(ctx, hipMalloc((void**)&dd, sizeof(uint32_t) * n));
   DG_HIP(ctx, hipMalloc((void**)&dout, sizeof(float) * n));
-  DG_HIP(ctx, hipMemcpy(ds, src, sizeof(uint32_t) * n, hipMemcpyHostToDevice));
-  DG_HIP(ctx, hipMemcpy(dd, dst, sizeof(uint32_t) * n, hipMemcpyHostToDevice));
+  DG_HIP(ctx, hipMemcpyAsync(ds, src, sizeof(uint32_t) * n, hipMemcpyHostToDevice, ctx->stream));
+  DG_HIP(ctx, hipMemcpyAsync(dd, dst, sizeof(uint32_t) * n, hipMemcpyHostToDevice, ctx->stream));
   pair_score_kernel<<<grid_for(ctx, n * 64, 256), 256, 0, ctx->stream>>>(s->d_rank, s->d_syn0, s->dim,
                                                                           ds, dd, n, dout);
   DG_HIP(ctx, hipGetLastError());
-  DG_HIP(ctx, hipMemcpy(scores, dout, sizeof(float) * n, hipMemcpyDeviceToHost));
+  DG_CHECK(dg_copy_to_host(ctx, scores, dout, sizeof(float) * n));
   hipFree(ds);
   hipFree(dd);
   hipFree(dout);

@@ -1368,8 +1368,7 @@ int tuples_backward_run(dg_ctx* ctx, const uint32_t* tuples, uint64_t n, uint32_
   }
   if (dlogits) {
     DG_CHECK(dg_reserve(ctx, &st->d_dl, &st->dl_cap, (size_t)(n * K1)));
-    DG_HIP(ctx, hipMemcpyAsync(st->d_dl, dlogits, sizeof(float) * n * K1, hipMemcpyHostToDevice,
-                               ctx->stream));
+    DG_HIP(ctx, hipMemcpyAsync(st->d_dl, dlogits, sizeof(float) * n * K1, hipMemcpyHostToDevice, ctx->stream));
   }
   if (fused) {
     DG_CHECK(dg_reserve(ctx, &st->d_logits, &st->logits_cap, (size_t)(n * K1)));

@@ -402,6 +402,9 @@ __global__ __launch_bounds__(kWalkBlock) void walk_kernel(WalkArgs a) {
           } else if (len >= a.length_limit) {
             finish = true;
             atomicOr(&a.q->flags, DG_QFLAG_LENGTH_LIMIT);
+          } else if (len == (uint32_t)kPathLds && a.spill_per_slot == 0) {
+            finish = true;  // the round is walked again, with spill space
+            atomicOr(&a.q->flags, DG_QFLAG_NO_SPILL);
           } else if (pending_back) {
             pending_back = false;
           } else if (trace) {
@@ -463,29 +466,29 @@ __global__ __launch_bounds__(kWalkBlock) void walk_kernel(WalkArgs a) {
   }
 }
 
-// The shards' totals into the queue; one wavefront.
-__global__ __launch_bounds__(64) void queue_sum_kernel(const dg_walk_shard* shards, dg_walk_queue* q) {
+// Empties a round that overflowed the token buffer, hit the length limit or
+// lacked spill space (every walk length 0), so the kernels after it leave the
+// visit counts and the tables as they were.
+//
+// Its first wavefront also adds the shards' totals into the queue.
+__global__ void round_guard_kernel(dg_walk_queue* q, uint32_t* walk_len, uint32_t n, const dg_walk_shard* shards) {
   static_assert(kWalkShards == 64, "a lane per shard");
-  const dg_walk_shard s = shards[threadIdx.x];
-  const uint64_t draws = wave_sum_u64(s.draws), moves = wave_sum_u64(s.moves), tokens = wave_sum_u64(s.tokens);
-  uint32_t most = s.max_len;
-  for (int d = 32; d >= 1; d >>= 1) {
-    const uint32_t o = __shfl_xor(most, d, 64);
-    most = o > most ? o : most;
+  if (blockIdx.x == 0 && threadIdx.x < 64) {
+    const dg_walk_shard s = shards[threadIdx.x];
+    const uint64_t draws = wave_sum_u64(s.draws), moves = wave_sum_u64(s.moves), tokens = wave_sum_u64(s.tokens);
+    uint32_t most = s.max_len;
+    for (int d = 32; d >= 1; d >>= 1) {
+      const uint32_t o = __shfl_xor(most, d, 64);
+      most = o > most ? o : most;
+    }
+    if (threadIdx.x == 0) {
+      q->draws = draws;
+      q->moves = moves;
+      q->tokens = tokens;
+      q->max_len = most;
+    }
   }
-  if (threadIdx.x == 0) {
-    q->draws = draws;
-    q->moves = moves;
-    q->tokens = tokens;
-    q->max_len = most;
-  }
-}
-
-// Empties a round that overflowed the token buffer or hit the length limit
-// (every walk length 0), so the kernels after it leave the corpus, the visit
-// counts and the tables as they were.
-__global__ void round_guard_kernel(const dg_walk_queue* q, uint32_t* walk_len, uint32_t n) {
-  if (!(q->flags & (DG_QFLAG_TOKEN_OVERFLOW | DG_QFLAG_LENGTH_LIMIT))) return;
+  if (q->flags == 0) return;
   for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
     walk_len[i] = 0;
 }
@@ -942,6 +945,7 @@ void dg_walk_free(dg_ctx* ctx) {
   delete ctx->wplan;
   ctx->wplan = nullptr;
   ctx->tok_raw_cap = ctx->walk_cap = ctx->walk_len_cap = ctx->tokens_cap = ctx->offsets_cap = 0;
+  ctx->walks_spill = false;
   ctx->spill_cap = ctx->scan_tmp_cap = ctx->re_cap = ctx->bin_off_cap = 0;
   ctx->train_tokens_cap = ctx->train_offsets_cap = 0;
   ctx->train_walks = ctx->train_tokens = 0;
@@ -1006,9 +1010,9 @@ extern "C" int dg_walk_reset(dg_ctx* ctx) {
 // ---- one round, in three parts ---------------------------------------------
 // plan: validation, launch shapes and buffers (may allocate); enqueue: kernels
 // only, no host waits, so a stream capture can record them; collect: the
-// round's statistics once the stream has finished.  dg_walk_round runs them
-// with a host check of the token buffer between the walk and the packing;
-// the captured pipeline step (pipeline.hip) puts round_guard_kernel there.
+// round's statistics once the stream has finished.  round_guard_kernel empties
+// a round that did not complete, which is then planned and walked again
+// (dg_walk_round; the captured step does the same, pipeline.hip).
 
 static int plan_round(dg_ctx* ctx, const dg_walk_params* p, uint32_t round,
                       uint32_t walker_begin, uint32_t walker_num, dg_walk_plan* pl) {
@@ -1027,14 +1031,21 @@ static int plan_round(dg_ctx* ctx, const dg_walk_params* p, uint32_t round,
   ctx->cur_tokens = 0;
 
   // persistent grid: every resident block slot on the device, fewer for small rounds
-  int per_cu = 0;
-  DG_HIP(ctx, hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, walk_kernel, kWalkBlock, 0));
-  if (per_cu < 1) per_cu = 1;
-  uint64_t blocks = (uint64_t)ctx->num_cus * per_cu;
+  if (ctx->walk_per_cu == 0) {
+    int per_cu = 0;
+    DG_HIP(ctx, hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, walk_kernel, kWalkBlock, 0));
+    ctx->walk_per_cu = per_cu < 1 ? 1 : per_cu;
+  }
+  uint64_t blocks = (uint64_t)ctx->num_cus * ctx->walk_per_cu;
   const uint64_t need_blocks = ((uint64_t)walker_num + kWalkBlock - 1) / kWalkBlock;
   if (blocks > need_blocks) blocks = need_blocks ? need_blocks : 1;
+  // spill space for the longest walk, (limit - kPathLds) vertices per lane
+  // (1 GB for the default limit): only once a walk has needed it, or when
+  // every walk will (the reference's walks end at 22 vertices)
+  const uint32_t longest = p->max_length != 0 ? p->max_length : length_limit;
+  if (p->min_length + 1 >= (uint32_t)kPathLds) ctx->walks_spill = true;
   const uint32_t spill_per_slot =
-      length_limit > (uint32_t)kPathLds ? length_limit - (uint32_t)kPathLds : 0;
+      ctx->walks_spill && longest > (uint32_t)kPathLds ? longest - (uint32_t)kPathLds : 0;
 
   DG_CHECK(dg_reserve(ctx, &ctx->d_walk_off, &ctx->walk_cap, (size_t)walker_num));
   DG_CHECK(dg_reserve(ctx, &ctx->d_walk_len, &ctx->walk_len_cap, (size_t)walker_num + 1));
@@ -1106,7 +1117,10 @@ static int enqueue_walk(dg_ctx* ctx, const dg_walk_plan& pl, bool timed) {
   walk_kernel<<<(unsigned)pl.blocks, kWalkBlock, 0, ctx->stream>>>(pl.a);
   DG_HIP(ctx, hipGetLastError());
   if (timed) DG_CHECK(dg_time_end(ctx, tk));
-  queue_sum_kernel<<<1, 64, 0, ctx->stream>>>(ctx->d_shards, ctx->d_queue);
+  // a round that did not complete becomes empty here, so the rest of it
+  // changes nothing and it can run again
+  round_guard_kernel<<<grid_for(ctx, pl.walker_num, 256), 256, 0, ctx->stream>>>(
+      ctx->d_queue, ctx->d_walk_len, pl.walker_num, ctx->d_shards);
   DG_HIP(ctx, hipGetLastError());
   return DG_OK;
 }
@@ -1197,38 +1211,55 @@ static int read_queue(dg_ctx* ctx) {
   return DG_OK;
 }
 
+// What the flags of a round that did not complete ask for: more token space,
+// spill space, or an error.  *retry: the round is to be walked again.
+static int check_flags(dg_ctx* ctx, const dg_walk_plan& pl, bool* retry) {
+  const dg_walk_queue& q = *ctx->h_queue;
+  *retry = false;
+  if (q.flags & DG_QFLAG_LENGTH_LIMIT)
+    return dg_fail(ctx, DG_ERR_WALK_TOO_LONG,
+                   "round %u: a walk reached the length limit %u (raise length_limit)", pl.round,
+                   pl.length_limit);
+  if (q.flags & DG_QFLAG_NO_SPILL) {
+    ctx->walks_spill = true;  // the next plan reserves it
+    *retry = true;
+  }
+  if (q.flags & DG_QFLAG_TOKEN_OVERFLOW) {
+    const size_t need = (size_t)(pl.a.slots_end + q.cursor + q.cursor / 8 + 1024);
+    DG_CHECK(dg_reserve(ctx, &ctx->d_tok_raw, &ctx->tok_raw_cap, need));
+    *retry = true;
+  }
+  return DG_OK;
+}
+
 static int walk_round_impl(dg_ctx* ctx, const dg_walk_params* p, uint32_t round,
                            uint32_t walker_begin, uint32_t walker_num, dg_round_stats* out) {
   dg_walk_plan pl;
-  DG_CHECK(plan_round(ctx, p, round, walker_begin, walker_num, &pl));
-  for (int attempt = 0; attempt < 3; ++attempt) {
-    pl.a.tokens = ctx->d_tok_raw;
-    pl.a.tok_cap = ctx->tok_raw_cap;
+  // at most one repeat for spill space and two for token space
+  for (int attempt = 0; attempt < 4; ++attempt) {
+    DG_CHECK(plan_round(ctx, p, round, walker_begin, walker_num, &pl));
+    DG_CHECK(dg_reserve(ctx, &ctx->d_tokens, &ctx->tokens_cap, ctx->tok_raw_cap));
     DG_CHECK(enqueue_walk(ctx, pl, true));
+    DG_CHECK(enqueue_tail(ctx, pl, true));
     DG_CHECK(read_queue(ctx));
-    if (ctx->h_queue->flags & DG_QFLAG_LENGTH_LIMIT)
-      return dg_fail(ctx, DG_ERR_WALK_TOO_LONG,
-                     "round %u: a walk reached the length limit %u (raise length_limit)", round,
-                     pl.length_limit);
-    if (!(ctx->h_queue->flags & DG_QFLAG_TOKEN_OVERFLOW)) break;
-    const size_t need =
-        (size_t)(pl.a.slots_end + ctx->h_queue->cursor + ctx->h_queue->cursor / 8 + 1024);
-    DG_CHECK(dg_reserve(ctx, &ctx->d_tok_raw, &ctx->tok_raw_cap, need));
-    if (attempt == 2) return dg_fail(ctx, DG_ERR_STATE, "token buffer sizing did not converge");
+    bool retry = false;
+    const int rc = check_flags(ctx, pl, &retry);
+    if (rc != DG_OK || retry) {
+      DG_CHECK(dg_time_resolve(ctx));
+      if (rc != DG_OK) return rc;
+      continue;
+    }
+    double walk_ms = 0.0, total_ms = 0.0;
+    for (auto& pe : ctx->pending) {
+      float ms = 0.f;
+      DG_HIP(ctx, hipEventElapsedTime(&ms, pe.start, pe.stop));
+      if (pe.name == "walk") walk_ms = ms;
+      total_ms += ms;
+    }
+    DG_CHECK(dg_time_resolve(ctx));
+    return collect_round(ctx, pl, walk_ms, total_ms, out);
   }
-  DG_CHECK(dg_reserve(ctx, &ctx->d_tokens, &ctx->tokens_cap, (size_t)ctx->h_queue->tokens));
-  DG_CHECK(enqueue_tail(ctx, pl, true));
-  DG_CHECK(read_queue(ctx));
-
-  double walk_ms = 0.0, total_ms = 0.0;
-  for (auto& pe : ctx->pending) {
-    float ms = 0.f;
-    DG_HIP(ctx, hipEventElapsedTime(&ms, pe.start, pe.stop));
-    if (pe.name == "walk") walk_ms = ms;  // the successful (last) attempt
-    total_ms += ms;
-  }
-  DG_CHECK(dg_time_resolve(ctx));
-  return collect_round(ctx, pl, walk_ms, total_ms, out);
+  return dg_fail(ctx, DG_ERR_STATE, "token buffer sizing did not converge");
 }
 
 extern "C" int dg_walk_round(dg_ctx* ctx, const dg_walk_params* p, uint32_t round,
@@ -1260,31 +1291,15 @@ int dg_walk_graph_plan(dg_ctx* ctx, const dg_walk_params* p, uint32_t round,
 int dg_walk_graph_enqueue(dg_ctx* ctx, bool timed) {
   const dg_walk_plan& pl = *ctx->wplan;
   DG_CHECK(enqueue_walk(ctx, pl, timed));
-  // a round that overflowed the token buffer or hit the length limit becomes
-  // empty here, so the rest of the step changes nothing and can run again
-  round_guard_kernel<<<grid_for(ctx, pl.walker_num, 256), 256, 0, ctx->stream>>>(
-      ctx->d_queue, ctx->d_walk_len, pl.walker_num);
-  DG_HIP(ctx, hipGetLastError());
   return enqueue_tail(ctx, pl, timed);
 }
 
 int dg_walk_graph_collect(dg_ctx* ctx, double walk_ms, double total_ms, dg_round_stats* out,
                           bool* retry) {
-  const dg_walk_plan& pl = *ctx->wplan;
-  *retry = false;
   DG_CHECK(read_queue(ctx));
-  const dg_walk_queue& q = *ctx->h_queue;
-  if (q.flags & DG_QFLAG_LENGTH_LIMIT)
-    return dg_fail(ctx, DG_ERR_WALK_TOO_LONG,
-                   "round %u: a walk reached the length limit %u (raise length_limit)", pl.round,
-                   pl.length_limit);
-  if (q.flags & DG_QFLAG_TOKEN_OVERFLOW) {
-    const size_t need = (size_t)(pl.a.slots_end + q.cursor + q.cursor / 8 + 1024);
-    DG_CHECK(dg_reserve(ctx, &ctx->d_tok_raw, &ctx->tok_raw_cap, need));
-    *retry = true;
-    return DG_OK;
-  }
-  return collect_round(ctx, pl, walk_ms, total_ms, out);
+  DG_CHECK(check_flags(ctx, *ctx->wplan, retry));
+  if (*retry) return DG_OK;
+  return collect_round(ctx, *ctx->wplan, walk_ms, total_ms, out);
 }
 
 extern "C" int dg_corpus_append(dg_ctx* ctx) {
@@ -1368,11 +1383,9 @@ extern "C" int dg_corpus_copy(dg_ctx* ctx, uint32_t* tokens, uint64_t* offsets) 
   DG_HIP(ctx, hipSetDevice(ctx->device));
   DG_HIP(ctx, hipStreamSynchronize(ctx->stream));
   if (tokens && ctx->cur_tokens)
-    DG_HIP(ctx, hipMemcpy(tokens, ctx->d_tokens, sizeof(uint32_t) * ctx->cur_tokens,
-                          hipMemcpyDeviceToHost));
+    DG_CHECK(dg_copy_to_host(ctx, tokens, ctx->d_tokens, sizeof(uint32_t) * ctx->cur_tokens));
   if (offsets && ctx->d_offsets)
-    DG_HIP(ctx, hipMemcpy(offsets, ctx->d_offsets, sizeof(uint64_t) * (ctx->cur_walks + 1),
-                          hipMemcpyDeviceToHost));
+    DG_CHECK(dg_copy_to_host(ctx, offsets, ctx->d_offsets, sizeof(uint64_t) * (ctx->cur_walks + 1)));
   return DG_OK;
 }
 
@@ -1381,8 +1394,7 @@ extern "C" int dg_vertex_freq(dg_ctx* ctx, uint32_t* freq) {
   if (!ctx->d_freq) return dg_fail(ctx, DG_ERR_STATE, "no walk has run");
   DG_HIP(ctx, hipSetDevice(ctx->device));
   DG_HIP(ctx, hipStreamSynchronize(ctx->stream));
-  DG_HIP(ctx, hipMemcpy(freq, ctx->d_freq, sizeof(uint32_t) * ctx->v_num, hipMemcpyDeviceToHost));
-  return DG_OK;
+  return dg_copy_to_host(ctx, freq, ctx->d_freq, sizeof(uint32_t) * ctx->v_num);
 }
 
 // Walk text file of include/path.hpp:67-119.  Formatting is done into a large
