@@ -103,11 +103,7 @@ struct dg_ctx {
   dg_walk_shard* d_shards = nullptr; // kWalkShards
   uint32_t* d_freq = nullptr;        // cumulative visit counts
   uint64_t freq_total = 0;           // sum of d_freq
-  uint32_t* d_bin_off = nullptr;     // per tile of the packing: its bins' first entries
-  size_t bin_off_cap = 0;
-  uint32_t* d_hot_part = nullptr;    // per pack workgroup: hot-vertex counts
-  size_t hot_part_cap = 0;
-  uint32_t* d_tok_raw = nullptr;     // tokens in completion order
+  uint32_t* d_tok_raw = nullptr;     // walk slots, longer walks, the packing's words
   size_t tok_raw_cap = 0;
   uint64_t* d_walk_off = nullptr;    // per-walk offset into d_tok_raw
   uint32_t* d_walk_len = nullptr;

@@ -914,6 +914,8 @@ struct dg_walk_plan {
   uint32_t parts = 0;         // pack_count_kernel grid
   uint32_t pack_block = 0;    // and its workgroup
   bool bins = false;          // visits counted by bins (else by atomics)
+  uint64_t bin_words = 0, tail_words = 0;  // the packing's words at the end of the raw buffer
+  uint32_t *bin_off = nullptr, *hot_part = nullptr;
   uint32_t bin_parts = 1;     // bin_count_kernel workgroups per bin
   uint32_t round = 0;
   uint32_t walker_num = 0;
@@ -925,7 +927,7 @@ struct dg_walk_plan {
 void dg_walk_free(dg_ctx* ctx) {
   void* bufs[] = {ctx->d_freq,   ctx->d_tok_raw,  ctx->d_walk_off, ctx->d_walk_len,
                   ctx->d_tokens, ctx->d_offsets,  ctx->d_spill,    ctx->d_scan_tmp,
-                  ctx->d_re_chunks, ctx->d_bin_off, ctx->d_train_tokens, ctx->d_train_offsets,
+                  ctx->d_re_chunks, ctx->d_train_tokens, ctx->d_train_offsets,
                   ctx->d_term_table};
   for (void* p : bufs)
     if (p) hipFree(p);
@@ -938,7 +940,6 @@ void dg_walk_free(dg_ctx* ctx) {
   ctx->d_spill = nullptr;
   ctx->d_scan_tmp = nullptr;
   ctx->d_re_chunks = nullptr;
-  ctx->d_bin_off = nullptr;
   ctx->d_train_tokens = nullptr;
   ctx->d_train_offsets = nullptr;
   ctx->d_term_table = nullptr;
@@ -946,7 +947,7 @@ void dg_walk_free(dg_ctx* ctx) {
   ctx->wplan = nullptr;
   ctx->tok_raw_cap = ctx->walk_cap = ctx->walk_len_cap = ctx->tokens_cap = ctx->offsets_cap = 0;
   ctx->walks_spill = false;
-  ctx->spill_cap = ctx->scan_tmp_cap = ctx->re_cap = ctx->bin_off_cap = 0;
+  ctx->spill_cap = ctx->scan_tmp_cap = ctx->re_cap = 0;
   ctx->train_tokens_cap = ctx->train_offsets_cap = 0;
   ctx->train_walks = ctx->train_tokens = 0;
   ctx->cur_walks = ctx->cur_tokens = 0;
@@ -1052,18 +1053,19 @@ static int plan_round(dg_ctx* ctx, const dg_walk_params* p, uint32_t round,
   DG_CHECK(dg_reserve(ctx, &ctx->d_offsets, &ctx->offsets_cap, (size_t)walker_num + 1));
   DG_CHECK(dg_reserve(ctx, &ctx->d_spill, &ctx->spill_cap,
                       (size_t)blocks * kWalkBlock * spill_per_slot));
-  // raw buffer: one slot of kPathLds tokens per walk, then room for longer walks
+  // raw buffer: one slot of kPathLds tokens per walk, then room for longer
+  // walks, and at its end the packing's own words (its bins' offsets and the
+  // hot counters' rows)
   const uint64_t slots_end = (uint64_t)walker_num * kPathLds;
-  size_t tok_need = (size_t)slots_end + (size_t)walker_num / 8 + 4096;
-  if (ctx->tok_raw_cap < tok_need) DG_CHECK(dg_reserve(ctx, &ctx->d_tok_raw, &ctx->tok_raw_cap, tok_need));
   {
     // packing: a workgroup of 1,024 walks per CU (LDS: the hot counters and 96 KB of tokens)
     pl->pack_block = walker_num < (uint64_t)ctx->num_cus * kPackBig ? kPackSmall : kPackBig;
     const uint64_t n_tiles = std::max<uint64_t>(1, ((uint64_t)walker_num + pl->pack_block - 1) / pl->pack_block);
     pl->parts = (uint32_t)std::min<uint64_t>((uint64_t)ctx->num_cus, n_tiles);
     pl->bins = ctx->v_num <= kBinVertices;
+    pl->bin_words = 0;
     if (pl->bins) {
-      DG_CHECK(dg_reserve(ctx, &ctx->d_bin_off, &ctx->bin_off_cap, (size_t)(n_tiles * (kBins + 1))));
+      pl->bin_words = n_tiles * (kBins + 1);
       // two workgroups of 1,024 threads per CU, fewer where their LDS does not fit
       const size_t lds = sizeof(uint32_t) * bin_places(ctx->v_num);
       DG_HIP(ctx, hipFuncSetAttribute((const void*)bin_count_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -1071,8 +1073,11 @@ static int plan_round(dg_ctx* ctx, const dg_walk_params* p, uint32_t round,
       const uint64_t fill = (uint64_t)ctx->num_cus * (lds <= 80 * 1024 ? 2 : 1) / kBins;
       pl->bin_parts = (uint32_t)std::max<uint64_t>(1, std::min(fill, n_tiles));
     }
-    DG_CHECK(dg_reserve(ctx, &ctx->d_hot_part, &ctx->hot_part_cap,
-                        (size_t)pl->parts * (ctx->n_hot ? ctx->n_hot : 1)));
+    pl->tail_words = pl->bin_words + (uint64_t)pl->parts * ctx->n_hot;
+    const size_t need = (size_t)(slots_end + walker_num / 8 + 4096 + pl->tail_words);
+    DG_CHECK(dg_reserve(ctx, &ctx->d_tok_raw, &ctx->tok_raw_cap, need));
+    pl->bin_off = ctx->d_tok_raw + (ctx->tok_raw_cap - pl->tail_words);
+    pl->hot_part = pl->bin_off + pl->bin_words;
   }
   const uint32_t n_chunks = (ctx->v_num + kReChunk - 1) / kReChunk;
   DG_CHECK(dg_reserve(ctx, &ctx->d_re_chunks, &ctx->re_cap, (size_t)n_chunks));
@@ -1100,7 +1105,7 @@ static int plan_round(dg_ctx* ctx, const dg_walk_params* p, uint32_t round,
   a.shards = ctx->d_shards;
   a.slots_end = slots_end;
   a.tokens = ctx->d_tok_raw;
-  a.tok_cap = ctx->tok_raw_cap;
+  a.tok_cap = ctx->tok_raw_cap - pl->tail_words;
   pl->blocks = blocks;
   pl->round = round;
   pl->walker_num = walker_num;
@@ -1137,7 +1142,7 @@ static int enqueue_tail(dg_ctx* ctx, const dg_walk_plan& pl, bool timed) {
   const auto pack = [&](auto kern) {
     kern<<<pl.parts, pl.pack_block, 0, ctx->stream>>>(
         ctx->d_tok_raw, ctx->d_walk_off, ctx->d_walk_len, ctx->d_offsets, walker_num, ctx->d_tokens,
-        ctx->d_hot_slot, ctx->n_hot, ctx->d_freq, ctx->d_hot_part, ctx->d_bin_off);
+        ctx->d_hot_slot, ctx->n_hot, ctx->d_freq, pl.hot_part, pl.bin_off);
   };
   const bool big = pl.pack_block == (uint32_t)kPackBig;
   if (pl.bins) {
@@ -1145,13 +1150,13 @@ static int enqueue_tail(dg_ctx* ctx, const dg_walk_plan& pl, bool timed) {
     const uint64_t n_tiles = ((uint64_t)walker_num + pl.pack_block - 1) / pl.pack_block;
     const uint32_t places = bin_places(ctx->v_num);
     bin_count_kernel<<<dim3(kBins, pl.bin_parts), kBinBlock, sizeof(uint32_t) * places, ctx->stream>>>(
-        ctx->d_tok_raw, ctx->d_bin_off, n_tiles, pl.pack_block * kPathLds, ctx->v_num, places, ctx->d_freq);
+        ctx->d_tok_raw, pl.bin_off, n_tiles, pl.pack_block * kPathLds, ctx->v_num, places, ctx->d_freq);
   } else {
     big ? pack(pack_count_kernel<kPackBig, false>) : pack(pack_count_kernel<kPackSmall, false>);
   }
   if (ctx->n_hot) {
     const dim3 grid((ctx->n_hot + 63) / 64, (pl.parts + kHotRows - 1) / kHotRows);
-    hot_reduce_kernel<<<grid, 64, 0, ctx->stream>>>(ctx->d_hot_part, pl.parts, ctx->n_hot,
+    hot_reduce_kernel<<<grid, 64, 0, ctx->stream>>>(pl.hot_part, pl.parts, ctx->n_hot,
                                                     ctx->d_hot_id, ctx->d_freq);
   }
   DG_HIP(ctx, hipGetLastError());
@@ -1225,7 +1230,7 @@ static int check_flags(dg_ctx* ctx, const dg_walk_plan& pl, bool* retry) {
     *retry = true;
   }
   if (q.flags & DG_QFLAG_TOKEN_OVERFLOW) {
-    const size_t need = (size_t)(pl.a.slots_end + q.cursor + q.cursor / 8 + 1024);
+    const size_t need = (size_t)(pl.a.slots_end + q.cursor + q.cursor / 8 + 1024 + pl.tail_words);
     DG_CHECK(dg_reserve(ctx, &ctx->d_tok_raw, &ctx->tok_raw_cap, need));
     *retry = true;
   }
@@ -1238,7 +1243,7 @@ static int walk_round_impl(dg_ctx* ctx, const dg_walk_params* p, uint32_t round,
   // at most one repeat for spill space and two for token space
   for (int attempt = 0; attempt < 4; ++attempt) {
     DG_CHECK(plan_round(ctx, p, round, walker_begin, walker_num, &pl));
-    DG_CHECK(dg_reserve(ctx, &ctx->d_tokens, &ctx->tokens_cap, ctx->tok_raw_cap));
+    DG_CHECK(dg_reserve(ctx, &ctx->d_tokens, &ctx->tokens_cap, pl.a.tok_cap));
     DG_CHECK(enqueue_walk(ctx, pl, true));
     DG_CHECK(enqueue_tail(ctx, pl, true));
     DG_CHECK(read_queue(ctx));
@@ -1281,10 +1286,10 @@ int dg_walk_graph_plan(dg_ctx* ctx, const dg_walk_params* p, uint32_t round,
   if (!ctx->wplan) ctx->wplan = new dg_walk_plan();
   DG_CHECK(plan_round(ctx, p, round, walker_begin, walker_num, ctx->wplan));
   // the packed corpus can hold every token the raw buffer can
-  DG_CHECK(dg_reserve(ctx, &ctx->d_tokens, &ctx->tokens_cap, ctx->tok_raw_cap));
-  *tok_bound = ctx->tok_raw_cap;
+  DG_CHECK(dg_reserve(ctx, &ctx->d_tokens, &ctx->tokens_cap, ctx->wplan->a.tok_cap));
+  *tok_bound = ctx->wplan->a.tok_cap;
   *slot_tokens = kPathLds;
-  *overflow_tokens = ctx->tok_raw_cap - ctx->wplan->a.slots_end;
+  *overflow_tokens = ctx->wplan->a.tok_cap - ctx->wplan->a.slots_end;
   return DG_OK;
 }
 
