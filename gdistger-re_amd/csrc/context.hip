@@ -47,6 +47,11 @@ extern "C" int dg_open(int device, dg_ctx** out) {
     return DG_ERR_NOMEM;
   }
   memset(ctx->h_queue, 0, sizeof(dg_walk_queue));
+  if (hipHostMalloc((void**)&ctx->h_flag, 64, hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess ||
+      hipHostGetDevicePointer((void**)&ctx->d_flag, ctx->h_flag, 0) != hipSuccess) {
+    dg_close(ctx);
+    return DG_ERR_NOMEM;
+  }
   if (dg_tuples_scratch_setup(ctx) != DG_OK) {
     dg_close(ctx);
     return DG_ERR_HIP;
@@ -76,6 +81,7 @@ extern "C" void dg_close(dg_ctx* ctx) {
   if (ctx->d_queue) hipFree(ctx->d_queue);
   if (ctx->d_shards) hipFree(ctx->d_shards);
   if (ctx->h_queue) hipHostFree(ctx->h_queue);
+  if (ctx->h_flag) hipHostFree(ctx->h_flag);
   if (ctx->stream) hipStreamDestroy(ctx->stream);
   if (ctx->opened) dg_hostcopy_close();
   delete ctx;

@@ -140,6 +140,10 @@ struct dg_ctx {
   dg_tuple_state* tuples = nullptr;
   dg_pipe_state* pipe = nullptr;
   dg_dsgl_state* dsgl = nullptr;
+  // a host-visible word a kernel sets when an id it was given is out of range,
+  // and the device's address of it
+  uint32_t* h_flag = nullptr;
+  uint32_t* d_flag = nullptr;
   // this device's copy of the allocation-free entry point's scratch array
   // (its address from hipGetSymbolAddress, set when the context opens)
   float* noalloc_scratch = nullptr;

@@ -31,7 +31,7 @@ namespace {
 constexpr size_t kChunk = 1u << 20;
 constexpr size_t kChunks = 16;
 constexpr int kThreads = 8;
-constexpr size_t kMinBytes = 16u << 10;
+constexpr size_t kMinBytes = 1u << 10;
 
 // Maps the whole pages of [p, p + n) for writing in one call, where the kernel
 // can: a fresh page's fault costs about a microsecond here, one by one.

@@ -166,10 +166,26 @@ __device__ __forceinline__ float softplus_f(float a) {
   return a > 0.0f ? a + log1pf(expf(-a)) : log1pf(expf(a));
 }
 
+// A failed check of a call: the code goes to the host word (read after the
+// call) and to a device word (the update kernel then leaves the tables
+// unchanged).
+struct TupleErr {
+  uint32_t* host;
+  uint32_t* dev;
+};
+constexpr uint32_t kErrWait = 1u, kErrBound = 2u, kErrRow = 3u;
+
+__device__ __forceinline__ void tuple_fail(const TupleErr& e, uint32_t code) {
+  *e.host = code;
+  *e.dev = code;
+}
+
 struct TupleArgs {
   const uint32_t* tuples;  // n x (2 + K)
   uint64_t n;
   uint32_t K;
+  uint32_t rows;           // ids at or above it fail the call (and read row 0 until it ends)
+  TupleErr err;
   const void* xt;          // syn0 (float or BF16 shadow)
   const void* yt;          // syn1
   float* logits;           // forward (and the fused step's backward): n x (1 + K)
@@ -194,10 +210,12 @@ struct TupleArgs {
 // backward of the fused step).  BWD: dL/dz, the staged
 // context-row gradient and the sort pairs (entries [0, n) for syn0 rows,
 // [n, N) for syn1 rows, in tuple order).
+// CHK: row ids at or above a.rows fail the call (3% of the FP32 forward's time;
+// the allocation-free forward checks them in a launch of its own).
 // Register target: three wavefronts per SIMD (168 VGPRs).  The FP32 backward
 // with the forward's outputs (the fused step) otherwise takes 172 and runs
 // two, 54 us instead of 43 at 65,536 tuples.
-template <typename E, int DIM, int NV, bool BWD, int G, bool OUT>
+template <typename E, int DIM, int NV, bool BWD, int G, bool OUT, bool CHK>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void tuple_fwd_kernel(TupleArgs a) {
   constexpr int T = 64 / G;                 // tuples per wavefront
   constexpr int D = DIM / G;
@@ -220,10 +238,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void t
       a.clear[i] = 0u;
   }
   uint64_t pr = wave;
+  bool bad = false;
+  auto checked = [&](uint32_t r) {
+    if constexpr (!CHK) return r;
+    bad |= r >= a.rows;
+    return r < a.rows ? r : 0u;
+  };
   uint32_t id = 0;
   if (pr < groups) {
     const uint64_t t = (uint64_t)T * pr + grp;
-    id = (t < a.n && hl < W) ? a.tuples[t * W + hl] : 0u;
+    id = (t < a.n && hl < W) ? checked(a.tuples[t * W + hl]) : 0u;
   }
   for (; pr < groups; pr += nwaves) {
     const uint64_t t = (uint64_t)T * pr + grp;
@@ -258,7 +282,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void t
     uint32_t id_next = 0;
     if (pn < groups) {
       const uint64_t tn = (uint64_t)T * pn + grp;
-      id_next = (tn < a.n && hl < W) ? a.tuples[tn * W + hl] : 0u;
+      id_next = (tn < a.n && hl < W) ? checked(a.tuples[tn * W + hl]) : 0u;
     }
     const float z = group_multi_sum<NV, G>(p, lane);
     const bool writer = tv && (hl % kStride) == 0 && idx < K1;
@@ -318,6 +342,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void t
       }
     }
     id = id_next;
+  }
+  if constexpr (CHK) {
+    if (bad) tuple_fail(a.err, kErrRow);
   }
   if constexpr (OUT) {
     if (lane == 0) a.wloss[wave] = wsum;
@@ -393,19 +420,6 @@ __device__ __forceinline__ void lb_add(uint64_t* p, uint64_t v) {
   __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// A failed look-back wait or output bound: the code goes to the host word
-// (read after the call) and to a device word (the update kernel then leaves
-// the tables unchanged).
-struct SortErr {
-  uint32_t* host;
-  uint32_t* dev;
-};
-
-__device__ __forceinline__ void sort_fail(const SortErr& e, uint32_t code) {
-  *e.host = code;
-  *e.dev = code;
-}
-
 // Look-back words of one column (a digit): tile words tw[t * stride] and
 // group words gw[g * stride].
 struct LbColumn {
@@ -425,7 +439,7 @@ __device__ __forceinline__ void lb_publish(const LbColumn& c, uint32_t tile, uin
 // once ready (all loads of a round in flight together).
 template <int R>
 __device__ uint32_t lb_prefix_part(const LbColumn& c, uint32_t tile, uint32_t first, uint32_t step,
-                                   const SortErr& err) {
+                                   const TupleErr& err) {
   const uint32_t g = tile / kGroup, t0 = g * kGroup;
   const uint32_t m = g + (tile - t0);
   uint32_t part = 0;
@@ -444,7 +458,7 @@ __device__ uint32_t lb_prefix_part(const LbColumn& c, uint32_t tile, uint32_t fi
       uint32_t polls = 0;
       while (j < g ? (w[u] >> 32) != (uint64_t)kGroup : (w[u] & kFlagReady) == 0ull) {
         if (++polls > kSpinLimit) {
-          sort_fail(err, 1u);
+          tuple_fail(err, kErrWait);
           break;
         }
         __builtin_amdgcn_s_sleep(1);
@@ -510,7 +524,7 @@ struct SortPass {
   uint32_t* tile_words;   // this pass's [tile][digit]
   uint64_t* group_words;  // this pass's [group][digit]
   uint32_t* ticket;       // null: tile = workgroup id (every tile is resident at once)
-  SortErr err;
+  TupleErr err;
   uint32_t* okeys;
   uint32_t* ovals;
 };
@@ -617,12 +631,13 @@ __global__ __launch_bounds__(kSortThreads) void radix_pass_kernel(SortPass a) {
       a.okeys[dst] = key;
       a.ovals[dst] = sval[j];
     } else {
-      sort_fail(a.err, 2u);
+      tuple_fail(a.err, kErrBound);
     }
   }
 }
 
 struct SegArgs {
+  uint32_t rows;
   const uint32_t* keys;   // sorted, N
   const uint32_t* vals;   // entry ids in sorted order
   uint64_t N;
@@ -637,7 +652,7 @@ struct SegArgs {
   float* carry;           // per block: sum of its last run when that run continues
   float* headp;           // per block: sum of its first run when that run started earlier
   uint32_t* fin;          // per block: 1 if headp finishes a row
-  const uint32_t* sort_err;  // non-zero: the sort failed, the tables are left unchanged
+  const uint32_t* err;    // non-zero: a check failed, the tables are left unchanged
   // apply (W -= lr * grad), or syn0 == null for gradients only
   float lr;
   float* syn0;
@@ -810,6 +825,7 @@ __global__ __launch_bounds__(256) void tuple_seg_kernel(SegArgs a) {
       } else {
         const uint32_t t = val / K1;
         src = a.tuples[(uint64_t)t * W + 1];
+        if (src >= a.rows) src = 0;  // a failed call's
         scale = a.dz[val];
       }
     }
@@ -900,7 +916,7 @@ __global__ __launch_bounds__(64 * kFixWaves) void tuple_fix_kernel(SegArgs a) {
   constexpr uint32_t kHalf = kFixWaves / 2;
   const uint64_t b = (uint64_t)blockIdx.x * kHalf + (wv % kHalf);
   const bool completes = wv < kHalf;
-  const bool upd = a.syn0 != nullptr && *a.sort_err == 0u;  // the update, unless the sort failed
+  const bool upd = a.syn0 != nullptr && *a.err == 0u;  // the update, unless a check failed
   if (completes && b < n_blocks && a.fin[b]) {
     const uint32_t k = a.keys[b * kSegBlock];
     uint64_t first, b0;
@@ -1026,6 +1042,10 @@ __global__ void to_bf16_kernel(const float* src, uint64_t n, uint16_t* dst) {
     dst[i] = to_bf16(src[i]);
 }
 
+__global__ void clear_word_kernel(uint32_t* flag) {
+  if (threadIdx.x == 0 && blockIdx.x == 0) *flag = 0u;
+}
+
 int waves_grid(dg_ctx* ctx, uint64_t waves) {
   uint64_t g = (waves + 3) / 4;  // 4 wavefronts per 256-thread block
   const uint64_t cap = (uint64_t)ctx->num_cus * 32;
@@ -1048,7 +1068,6 @@ struct dg_tuple_state {
   size_t logits_cap = 0;
   double* d_wloss = nullptr;  // loss partial per forward wavefront
   size_t wloss_cap = 0;
-  double* d_loss = nullptr;
   float* d_dl = nullptr;  // upstream dL/dz
   size_t dl_cap = 0;
   float* d_dz = nullptr;
@@ -1061,8 +1080,11 @@ struct dg_tuple_state {
   size_t v_cap[2] = {0, 0};
   uint32_t* d_lb = nullptr;     // tickets, then the look-back words of the sort and segment launches
   size_t lb_cap = 0;
-  uint32_t* h_err = nullptr;    // host-visible: set by a kernel whose look-back wait or store bound failed
+  // host-visible words: [0] set by a kernel whose check failed (a row id, a
+  // look-back wait, a store bound), [2..3] the loss (a double)
+  uint32_t* h_err = nullptr;
   uint32_t* d_err = nullptr;    // the device's address of h_err
+  uint32_t* d_fail = nullptr;   // the failed check's code on the device; zero between calls
   float* d_grad = nullptr;
   size_t grad_cap = 0;
   float* d_carry = nullptr;
@@ -1071,6 +1093,10 @@ struct dg_tuple_state {
   size_t headp_cap = 0;
   uint32_t* d_fin = nullptr;
   size_t fin_cap = 0;
+  uint32_t* d_rows = nullptr;   // dg_sgns_grad_rows: the rows asked for, and their gradients
+  size_t rows_cap = 0;
+  float* d_rows_out = nullptr;
+  size_t rows_out_cap = 0;
   // BF16 copies of the tables and the table version they were made from
   uint16_t* d_bf0 = nullptr;
   uint16_t* d_bf1 = nullptr;
@@ -1088,10 +1114,11 @@ struct dg_tuple_state {
 void dg_tuples_free(dg_ctx* ctx) {
   dg_tuple_state* t = ctx->tuples;
   if (!t) return;
-  void* bufs[] = {t->d_tuples, t->d_logits, t->d_wloss,    t->d_loss,       t->d_dl,    t->d_dz,
+  void* bufs[] = {t->d_tuples, t->d_logits, t->d_wloss,    t->d_fail,       t->d_dl,    t->d_dz,
                   t->d_stage,  t->d_k[0],   t->d_k[1],     t->d_v[0],       t->d_v[1],
                   t->d_lb,
-                  t->d_grad,   t->d_carry,  t->d_headp,    t->d_fin,        t->d_bf0,   t->d_bf1};
+                  t->d_grad,   t->d_carry,  t->d_headp,    t->d_fin,        t->d_bf0,   t->d_bf1,
+                  t->d_rows,   t->d_rows_out};
   for (void* b : bufs)
     if (b) hipFree(b);
   if (t->h_err) hipHostFree(t->h_err);
@@ -1110,8 +1137,10 @@ dg_tuple_state* tuple_state(dg_ctx* ctx) {
   return ctx->tuples;
 }
 
-// Validate a tuple batch on the host (every id is dereferenced on the device)
-// and copy it to the device.
+// Check a tuple batch's shape and copy it to the device, where the gathering
+// kernel checks every row id as it reads it (check_rows after the call): a
+// host pass over 65,536 tuples of 7 ids took longer than the whole step's
+// kernels.  Makes the words those checks report to.
 int upload_tuples(dg_ctx* ctx, dg_tuple_state* st, const dg_table_view& tv, const uint32_t* tuples,
                   uint64_t n, uint32_t K) {
   if (K > (uint32_t)kMaxTupleNeg)
@@ -1122,14 +1151,36 @@ int upload_tuples(dg_ctx* ctx, dg_tuple_state* st, const dg_table_view& tv, cons
   if (n == 0 || n * W >= (1ull << 31))
     return dg_fail(ctx, DG_ERR_ARG, "tuple count %llu: must be in [1, 2^31 / (K + 2))",
                    (unsigned long long)n);
-  for (uint64_t i = 0; i < n * W; ++i)
-    if (tuples[i] >= tv.rows)
-      return dg_fail(ctx, DG_ERR_ARG, "tuple %llu: row %u out of range (%u rows)",
-                     (unsigned long long)(i / W), tuples[i], tv.rows);
+  if (!st->h_err) {
+    DG_HIP(ctx, hipHostMalloc((void**)&st->h_err, 4 * sizeof(uint32_t), hipHostMallocMapped | hipHostMallocCoherent));
+    DG_HIP(ctx, hipHostGetDevicePointer((void**)&st->d_err, st->h_err, 0));
+  }
+  if (!st->d_fail) {
+    DG_HIP(ctx, hipMalloc((void**)&st->d_fail, sizeof(uint32_t)));
+    clear_word_kernel<<<1, 64, 0, ctx->stream>>>(st->d_fail);
+    DG_HIP(ctx, hipGetLastError());
+  }
+  *st->h_err = 0u;  // the previous call's kernels have finished
   DG_CHECK(dg_reserve(ctx, &st->d_tuples, &st->tuples_cap, (size_t)(n * W)));
   DG_HIP(ctx, hipMemcpyAsync(st->d_tuples, tuples, sizeof(uint32_t) * n * W, hipMemcpyHostToDevice,
                              ctx->stream));
   return DG_OK;
+}
+
+// The checks of a call whose kernels have finished.
+int check_call(dg_ctx* ctx, dg_tuple_state* st, const dg_table_view& tv, const uint32_t* tuples, uint64_t n,
+               uint32_t K) {
+  const uint32_t code = *st->h_err;
+  if (code == 0u) return DG_OK;
+  clear_word_kernel<<<1, 64, 0, ctx->stream>>>(st->d_fail);
+  DG_HIP(ctx, hipGetLastError());
+  const uint64_t W = K + 2;
+  for (uint64_t i = 0; i < n * W; ++i)
+    if (tuples[i] >= tv.rows)
+      return dg_fail(ctx, DG_ERR_ARG, "tuple %llu: row %u out of range (%u rows)",
+                     (unsigned long long)(i / W), tuples[i], tv.rows);
+  return dg_fail(ctx, DG_ERR_HIP,
+                 "tuple sort: a look-back wait or an output bound failed (%u); tables left unchanged", code);
 }
 
 // BF16 copies of both tables, remade when the FP32 tables changed.
@@ -1157,39 +1208,39 @@ int ensure_bf16(dg_ctx* ctx, dg_tuple_state* st, const dg_table_view& tv) {
 // row is half an FP32 row, so twice the tuples fit the same registers), 16
 // for K + 2 <= 16, otherwise 32.  Returns the wavefronts launched (at most
 // 128 per CU: the forward writes one loss partial per wavefront).
-template <typename E, int DIM, bool BWD, bool OUT>
+template <typename E, int DIM, bool BWD, bool OUT, bool CHK>
 uint32_t launch_fwd(dg_ctx* ctx, const TupleArgs& a) {
   if (sizeof(E) == 2 && DIM >= 128 && a.K + 2 <= 8) {
     const int g = waves_grid(ctx, (a.n + 7) / 8);  // a tuple per 8 lanes
-    tuple_fwd_kernel<E, DIM, 8, BWD, 8, OUT><<<g, 256, 0, ctx->stream>>>(a);
+    tuple_fwd_kernel<E, DIM, 8, BWD, 8, OUT, CHK><<<g, 256, 0, ctx->stream>>>(a);
     return 4u * (uint32_t)g;
   }
   if (a.K + 2 <= 16) {
     const int g = waves_grid(ctx, (a.n + 3) / 4);  // a tuple per 16 lanes
     if (a.K + 1 <= 8)
-      tuple_fwd_kernel<E, DIM, 8, BWD, 16, OUT><<<g, 256, 0, ctx->stream>>>(a);
+      tuple_fwd_kernel<E, DIM, 8, BWD, 16, OUT, CHK><<<g, 256, 0, ctx->stream>>>(a);
     else
-      tuple_fwd_kernel<E, DIM, 16, BWD, 16, OUT><<<g, 256, 0, ctx->stream>>>(a);
+      tuple_fwd_kernel<E, DIM, 16, BWD, 16, OUT, CHK><<<g, 256, 0, ctx->stream>>>(a);
     return 4u * (uint32_t)g;
   }
   const int g = waves_grid(ctx, (a.n + 1) / 2);  // a tuple per half-wavefront
   if (a.K + 1 <= 8)
-    tuple_fwd_kernel<E, DIM, 8, BWD, 32, OUT><<<g, 256, 0, ctx->stream>>>(a);
+    tuple_fwd_kernel<E, DIM, 8, BWD, 32, OUT, CHK><<<g, 256, 0, ctx->stream>>>(a);
   else
-    tuple_fwd_kernel<E, DIM, 16, BWD, 32, OUT><<<g, 256, 0, ctx->stream>>>(a);
+    tuple_fwd_kernel<E, DIM, 16, BWD, 32, OUT, CHK><<<g, 256, 0, ctx->stream>>>(a);
   return 4u * (uint32_t)g;
 }
 
-template <bool BWD, bool OUT = !BWD>
+template <bool BWD, bool OUT = !BWD, bool CHK = true>
 uint32_t launch_fwd_form(dg_ctx* ctx, const TupleArgs& a, int bf16, uint32_t dim) {
   if (bf16) {
-    if (dim == 64) return launch_fwd<uint16_t, 64, BWD, OUT>(ctx, a);
-    if (dim == 128) return launch_fwd<uint16_t, 128, BWD, OUT>(ctx, a);
-    return launch_fwd<uint16_t, 256, BWD, OUT>(ctx, a);
+    if (dim == 64) return launch_fwd<uint16_t, 64, BWD, OUT, true>(ctx, a);
+    if (dim == 128) return launch_fwd<uint16_t, 128, BWD, OUT, true>(ctx, a);
+    return launch_fwd<uint16_t, 256, BWD, OUT, true>(ctx, a);
   }
-  if (dim == 64) return launch_fwd<float, 64, BWD, OUT>(ctx, a);
-  if (dim == 128) return launch_fwd<float, 128, BWD, OUT>(ctx, a);
-  return launch_fwd<float, 256, BWD, OUT>(ctx, a);
+  if (dim == 64) return launch_fwd<float, 64, BWD, OUT, CHK>(ctx, a);
+  if (dim == 128) return launch_fwd<float, 128, BWD, OUT, CHK>(ctx, a);
+  return launch_fwd<float, 256, BWD, OUT, CHK>(ctx, a);
 }
 
 template <typename E>
@@ -1220,11 +1271,12 @@ extern "C" int dg_sgns_tuples_forward(dg_ctx* ctx, const uint32_t* tuples, uint6
   const uint32_t K1 = K + 1;
   DG_CHECK(dg_reserve(ctx, &st->d_logits, &st->logits_cap, (size_t)(n * K1)));
   DG_CHECK(dg_reserve(ctx, &st->d_wloss, &st->wloss_cap, (size_t)ctx->num_cus * 128));
-  if (!st->d_loss) DG_HIP(ctx, hipMalloc((void**)&st->d_loss, sizeof(double)));
   TupleArgs a{};
   a.tuples = st->d_tuples;
   a.n = n;
   a.K = K;
+  a.rows = tv.rows;
+  a.err = TupleErr{st->d_err, st->d_fail};
   a.xt = bf16 ? (const void*)st->d_bf0 : (const void*)tv.syn0;
   a.yt = bf16 ? (const void*)st->d_bf1 : (const void*)tv.syn1;
   a.logits = st->d_logits;
@@ -1232,17 +1284,17 @@ extern "C" int dg_sgns_tuples_forward(dg_ctx* ctx, const uint32_t* tuples, uint6
   size_t tk;
   DG_CHECK(dg_time_begin(ctx, "tuple_fwd", &tk));
   const uint32_t waves = launch_fwd_form<false>(ctx, a, bf16, tv.dim);
-  loss_sum_kernel<<<1, kLossThreads, 0, ctx->stream>>>(st->d_wloss, waves, st->d_loss);
+  loss_sum_kernel<<<1, kLossThreads, 0, ctx->stream>>>(st->d_wloss, waves,
+                                                       reinterpret_cast<double*>(st->d_err + 2));
   DG_HIP(ctx, hipGetLastError());
   DG_CHECK(dg_time_end(ctx, tk));
   if (logits)
-    DG_HIP(ctx, hipMemcpyAsync(logits, st->d_logits, sizeof(float) * n * K1, hipMemcpyDeviceToHost,
-                               ctx->stream));
-  double h_loss = 0.0;
-  DG_HIP(ctx, hipMemcpyAsync(&h_loss, st->d_loss, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-  DG_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    DG_CHECK(dg_copy_to_host(ctx, logits, st->d_logits, sizeof(float) * n * K1));
+  else
+    DG_HIP(ctx, hipStreamSynchronize(ctx->stream));
   DG_CHECK(dg_time_resolve(ctx));
-  if (loss) *loss = h_loss;
+  DG_CHECK(check_call(ctx, st, tv, tuples, n, K));
+  if (loss) memcpy(loss, st->h_err + 2, sizeof(double));
   return DG_OK;
 }
 
@@ -1250,29 +1302,23 @@ namespace {
 
 // ---- the allocation-free forward ---------------------------------------------
 // Scratch of dg_sgns_tuples_forward_noalloc: the loss partial of each
-// forward wavefront (at most kNoAllocMaxWaves doubles), then a range-check
-// flag.  Each device holds its own copy; host code reaches it only through
-// the address hipGetSymbolAddress gives on that device
-// (dg_tuples_scratch_setup).
+// forward wavefront (at most kNoAllocMaxWaves doubles).  Each device holds its
+// own copy; host code reaches it only through the address hipGetSymbolAddress
+// gives on that device (dg_tuples_scratch_setup).
 constexpr uint64_t kNoAllocMaxTuples = 1ull << 20;
 constexpr uint32_t kNoAllocMaxWaves = 65536;              // 128 per CU on up to 512 CUs
-constexpr int kNoAllocFlag = 2 * kNoAllocMaxWaves;        // float index of the flag
-static __device__ __align__(256) float scratch[kNoAllocFlag + 64];
+static __device__ __align__(256) float scratch[2 * kNoAllocMaxWaves];
 
 constexpr int kMaxScratchDevices = 64;
 std::mutex g_scratch_mu;
 float* g_scratch_dev[kMaxScratchDevices] = {};
-
-__global__ void noalloc_clear_kernel(uint32_t* flag) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) *flag = 0u;
-}
 
 __global__ void tuple_check_kernel(const uint32_t* tuples, uint64_t count, uint32_t rows, uint32_t* flag) {
   bool bad = false;
   for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < count;
        i += (uint64_t)gridDim.x * blockDim.x)
     bad |= tuples[i] >= rows;
-  if (__ballot(bad) != 0 && (threadIdx.x & 63) == 0) atomicOr(flag, 1u);
+  if (__ballot(bad) != 0 && (threadIdx.x & 63) == 0) *flag = 1u;
 }
 
 }  // namespace
@@ -1312,26 +1358,27 @@ extern "C" int dg_sgns_tuples_forward_noalloc(dg_ctx* ctx, const uint32_t* d_tup
   DG_HIP(ctx, hipSetDevice(ctx->device));
   float* base = ctx->noalloc_scratch;
   double* wloss = reinterpret_cast<double*>(base);
-  uint32_t* flag = reinterpret_cast<uint32_t*>(base + kNoAllocFlag);
-  // every row id is dereferenced by the forward: check them on the device
+  // every row id is dereferenced by the forward: check them on the device,
+  // into a host-visible word
   const uint64_t count = n * (K + 2);
-  noalloc_clear_kernel<<<1, 64, 0, ctx->stream>>>(flag);
+  *ctx->h_flag = 0u;  // the kernels that can set it have finished (each call that uses it waits)
   tuple_check_kernel<<<waves_grid(ctx, count / 64 + 1), 256, 0, ctx->stream>>>(d_tuples, count, tv.rows,
-                                                                               flag);
+                                                                               ctx->d_flag);
   DG_HIP(ctx, hipGetLastError());
-  uint32_t bad = 0;
-  DG_HIP(ctx, hipMemcpyAsync(&bad, flag, sizeof(bad), hipMemcpyDeviceToHost, ctx->stream));
   DG_HIP(ctx, hipStreamSynchronize(ctx->stream));
+  const uint32_t bad = *ctx->h_flag;
   if (bad) return dg_fail(ctx, DG_ERR_ARG, "a tuple row is out of range (%u rows)", tv.rows);
   TupleArgs a{};
   a.tuples = d_tuples;
   a.n = n;
   a.K = K;
+  a.rows = tv.rows;  // checked above
+  a.err = TupleErr{ctx->d_flag, ctx->d_flag};
   a.xt = tv.syn0;
   a.yt = tv.syn1;
   a.logits = d_logits;
   a.wloss = wloss;
-  const uint32_t waves = launch_fwd_form<false>(ctx, a, 0, tv.dim);
+  const uint32_t waves = launch_fwd_form<false, true, false>(ctx, a, 0, tv.dim);
   loss_sum_kernel<<<1, kLossThreads, 0, ctx->stream>>>(wloss, waves, d_loss);
   DG_HIP(ctx, hipGetLastError());
   return DG_OK;
@@ -1373,14 +1420,8 @@ int tuples_backward_run(dg_ctx* ctx, const uint32_t* tuples, uint64_t n, uint32_
   if (fused) {
     DG_CHECK(dg_reserve(ctx, &st->d_logits, &st->logits_cap, (size_t)(n * K1)));
     DG_CHECK(dg_reserve(ctx, &st->d_wloss, &st->wloss_cap, (size_t)ctx->num_cus * 128));
-    if (!st->d_loss) DG_HIP(ctx, hipMalloc((void**)&st->d_loss, sizeof(double)));
   }
   // the sort's sizes and the words it expects zero (cleared by the backward kernel)
-  if (!st->h_err) {
-    DG_HIP(ctx, hipHostMalloc((void**)&st->h_err, sizeof(uint32_t), hipHostMallocMapped | hipHostMallocCoherent));
-    DG_HIP(ctx, hipHostGetDevicePointer((void**)&st->d_err, st->h_err, 0));
-  }
-  *st->h_err = 0u;  // the previous call's kernels have finished
   const int passes = (rb + 1 + 7) / 8;
   const uint64_t n_tiles = (N + kSortTile - 1) / kSortTile;
   const uint64_t n_groups = (n_tiles + kGroup - 1) / kGroup;
@@ -1388,13 +1429,11 @@ int tuples_backward_run(dg_ctx* ctx, const uint32_t* tuples, uint64_t n, uint32_
   const uint64_t n_blocks = (N + kSegBlock - 1) / kSegBlock;
   // words cleared by the backward kernel, in 32-bit units (64-bit group
   // words at even offsets): the digit counts [copy][pass][digit], kMaxPasses
-  // tickets, the device error word, then per pass the [tile][digit] and
-  // [group][digit] look-back words.  Tiles are numbered by workgroup id when every tile is resident
+  // tickets, then per pass the [tile][digit] and [group][digit] look-back words.  Tiles are numbered by workgroup id when every tile is resident
   // at once (one 1,024-thread workgroup per CU), by ticket otherwise.
   auto even = [](uint64_t x) { return (x + 1) & ~1ull; };
   const uint64_t o_tick = (uint64_t)kHistCopies * kMaxPasses * 256;
-  const uint64_t o_err = o_tick + kMaxPasses;  // the device error word
-  const uint64_t o_sort = even(o_err + 1);
+  const uint64_t o_sort = even(o_tick + kMaxPasses);
   const uint64_t pass_words = even(n_tiles * 256) + 2 * n_groups * 256;
   const uint64_t n_lb = o_sort + (uint64_t)passes * pass_words;
   const bool tickets = n_tiles > (uint64_t)ctx->num_cus;
@@ -1403,6 +1442,8 @@ int tuples_backward_run(dg_ctx* ctx, const uint32_t* tuples, uint64_t n, uint32_
   a.tuples = st->d_tuples;
   a.n = n;
   a.K = K;
+  a.rows = tv.rows;
+  a.err = TupleErr{st->d_err, st->d_fail};
   a.xt = bf16 ? (const void*)st->d_bf0 : (const void*)tv.syn0;
   a.yt = bf16 ? (const void*)st->d_bf1 : (const void*)tv.syn1;
   a.dlogits = dlogits ? st->d_dl : nullptr;
@@ -1421,7 +1462,9 @@ int tuples_backward_run(dg_ctx* ctx, const uint32_t* tuples, uint64_t n, uint32_
   DG_CHECK(dg_time_begin(ctx, "tuple_prep", &tk));
   const uint32_t waves = fused ? launch_fwd_form<true, true>(ctx, a, bf16, dim)
                                : launch_fwd_form<true, false>(ctx, a, bf16, dim);
-  if (fused) loss_sum_kernel<<<1, kLossThreads, 0, ctx->stream>>>(st->d_wloss, waves, st->d_loss);
+  if (fused)
+    loss_sum_kernel<<<1, kLossThreads, 0, ctx->stream>>>(st->d_wloss, waves,
+                                                         reinterpret_cast<double*>(st->d_err + 2));
   DG_HIP(ctx, hipGetLastError());
   DG_CHECK(dg_time_end(ctx, tk));
   // sort (key, entry) pairs on rb + 1 key bits
@@ -1439,7 +1482,7 @@ int tuples_backward_run(dg_ctx* ctx, const uint32_t* tuples, uint64_t n, uint32_
     sp.tile_words = pw;
     sp.group_words = reinterpret_cast<uint64_t*>(pw + even(n_tiles * 256));
     sp.ticket = tickets ? st->d_lb + o_tick + p : nullptr;
-    sp.err = SortErr{st->d_err, st->d_lb + o_err};
+    sp.err = a.err;
     sp.okeys = st->d_k[1 - cur];
     sp.ovals = st->d_v[1 - cur];
     radix_pass_kernel<<<(unsigned)n_tiles, kSortThreads, 0, ctx->stream>>>(sp);
@@ -1453,6 +1496,7 @@ int tuples_backward_run(dg_ctx* ctx, const uint32_t* tuples, uint64_t n, uint32_
   DG_CHECK(dg_reserve(ctx, &st->d_headp, &st->headp_cap, (size_t)(n_blocks * dim)));
   DG_CHECK(dg_reserve(ctx, &st->d_fin, &st->fin_cap, (size_t)n_blocks));
   SegArgs sa{};
+  sa.rows = tv.rows;
   sa.keys = st->d_k[cur];
   sa.vals = st->d_v[cur];
   sa.N = N;
@@ -1467,7 +1511,7 @@ int tuples_backward_run(dg_ctx* ctx, const uint32_t* tuples, uint64_t n, uint32_
   sa.carry = st->d_carry;
   sa.headp = st->d_headp;
   sa.fin = st->d_fin;
-  sa.sort_err = st->d_lb + o_err;
+  sa.err = st->d_fail;
   const bool shadow = st->d_bf0 && st->bf_version == tv.version;
   if (apply) {
     sa.lr = lr;
@@ -1494,21 +1538,14 @@ int tuples_backward_run(dg_ctx* ctx, const uint32_t* tuples, uint64_t n, uint32_
     const uint64_t v = dg_sgns_written(ctx);
     if (shadow) st->bf_version = v;  // the shadow rows were updated with the FP32 rows
   }
-  double h_loss = 0.0;
-  if (fused) {
-    if (logits)
-      DG_HIP(ctx, hipMemcpyAsync(logits, st->d_logits, sizeof(float) * n * K1, hipMemcpyDeviceToHost,
-                                 ctx->stream));
-    DG_HIP(ctx, hipMemcpyAsync(&h_loss, st->d_loss, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-  }
-  DG_HIP(ctx, hipStreamSynchronize(ctx->stream));
+  if (fused && logits)
+    DG_CHECK(dg_copy_to_host(ctx, logits, st->d_logits, sizeof(float) * n * K1));
+  else
+    DG_HIP(ctx, hipStreamSynchronize(ctx->stream));
   DG_CHECK(dg_time_resolve(ctx));
-  if (*st->h_err)
-    return dg_fail(ctx, DG_ERR_HIP,
-                   "tuple sort: a look-back wait or an output bound failed (%u); tables left unchanged",
-                   *st->h_err);
+  DG_CHECK(check_call(ctx, st, tv, tuples, n, K));
   st->have_grads = true;
-  if (fused && loss) *loss = h_loss;
+  if (fused && loss) memcpy(loss, st->h_err + 2, sizeof(double));
   return DG_OK;
 }
 
@@ -1534,23 +1571,12 @@ extern "C" int dg_sgns_grad_rows(dg_ctx* ctx, int table, const uint32_t* rows, u
     if (rows[i] >= st->grad_rows)
       return dg_fail(ctx, DG_ERR_ARG, "row %u out of range (%u rows)", rows[i], st->grad_rows);
   DG_HIP(ctx, hipSetDevice(ctx->device));
-  uint32_t* d_rows = nullptr;
-  float* d_out = nullptr;
-  DG_HIP(ctx, hipMalloc((void**)&d_rows, sizeof(uint32_t) * n_rows));
-  DG_HIP(ctx, hipMalloc((void**)&d_out, sizeof(float) * n_rows * st->grad_dim));
-  int rc = DG_OK;
-  hipError_t e = hipMemcpy(d_rows, rows, sizeof(uint32_t) * n_rows, hipMemcpyHostToDevice);
-  if (e == hipSuccess) {
-    grad_rows_kernel<<<waves_grid(ctx, n_rows), 256, 0, ctx->stream>>>(
-        st->d_k[st->sorted], st->d_grad, st->grad_N, st->grad_rb, (uint32_t)table, d_rows, n_rows,
-        st->grad_dim, d_out);
-    e = hipGetLastError();
-  }
-  if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
-  if (e == hipSuccess)
-    e = hipMemcpy(out, d_out, sizeof(float) * n_rows * st->grad_dim, hipMemcpyDeviceToHost);
-  if (e != hipSuccess) rc = dg_fail(ctx, DG_ERR_HIP, "grad_rows: %s", hipGetErrorString(e));
-  hipFree(d_rows);
-  hipFree(d_out);
-  return rc;
+  DG_CHECK(dg_reserve(ctx, &st->d_rows, &st->rows_cap, (size_t)n_rows));
+  DG_CHECK(dg_reserve(ctx, &st->d_rows_out, &st->rows_out_cap, (size_t)(n_rows * st->grad_dim)));
+  DG_HIP(ctx, hipMemcpyAsync(st->d_rows, rows, sizeof(uint32_t) * n_rows, hipMemcpyHostToDevice, ctx->stream));
+  grad_rows_kernel<<<waves_grid(ctx, n_rows), 256, 0, ctx->stream>>>(
+      st->d_k[st->sorted], st->d_grad, st->grad_N, st->grad_rb, (uint32_t)table, st->d_rows, n_rows, st->grad_dim,
+      st->d_rows_out);
+  DG_HIP(ctx, hipGetLastError());
+  return dg_copy_to_host(ctx, out, st->d_rows_out, sizeof(float) * n_rows * st->grad_dim);
 }
