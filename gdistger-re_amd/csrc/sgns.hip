@@ -372,6 +372,45 @@ struct Chunk<uint16_t> {
   }
 };
 
+// Operands whose k index is an output column, and their product.  Sixteen
+// columns fill a chunk.  With eight, the BF16 step takes zeros past them; the
+// FP32 steps take k = 2 (l/16) + e, e = 0..1, two steps instead of four.
+template <typename E, int KC>
+struct OutputCols {
+  typedef Chunk<E> C;
+  typedef typename C::v_t v_t;
+  __device__ static v_t zero() { return C::from(0.f, 0.f, 0.f, 0.f); }
+  // from a row of KC values
+  __device__ static v_t row(const float* src, int g4) {
+    if (4 * g4 >= KC) return zero();
+    const float4 q = *reinterpret_cast<const float4*>(src + 4 * g4);
+    return C::from(q.x, q.y, q.z, q.w);
+  }
+  // column l16 of the KC rows from blk: groups past them read rows 0..3 and take zeros
+  template <int LDN>
+  __device__ static v_t col(const E* blk, int g4, int l16) {
+    const bool ok = 4 * g4 < KC;
+    const v_t v = C::template col4<LDN>(blk + (ok ? 4 * g4 : 0) * LDN, l16);
+    return ok ? v : zero();
+  }
+  __device__ static f32x4_t mma(v_t a, v_t b, f32x4_t c) { return C::mma(a, b, c); }
+};
+
+template <>
+struct OutputCols<float, 8> {
+  typedef float2 v_t;
+  __device__ static v_t zero() { return make_float2(0.f, 0.f); }
+  __device__ static v_t row(const float* src, int g4) { return *reinterpret_cast<const float2*>(src + 2 * g4); }
+  template <int LDN>
+  __device__ static v_t col(const float* blk, int g4, int l16) {
+    return make_float2(blk[2 * g4 * LDN + l16], blk[(2 * g4 + 1) * LDN + l16]);
+  }
+  __device__ static f32x4_t mma(v_t a, v_t b, f32x4_t c) {
+    c = __builtin_amdgcn_mfma_f32_16x16x4f32(a.x, b.x, c, 0, 0, 0);
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a.y, b.y, c, 0, 0, 0);
+  }
+};
+
 // word j of a Philox stream (block j/4, word j%4)
 __device__ __forceinline__ uint32_t stream_word(uint64_t seed, uint32_t c1, uint32_t c2,
                                                 uint32_t tag, uint32_t j) {
@@ -966,32 +1005,9 @@ void sg_sent_kernel(SentArgs t) {
         }
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        // ---- dX = Gp Y + H X into the deltas (dX^T[d][u] layout)
-#pragma unroll
-        for (int p = 0; p < NPT; ++p) {
-          V bgp = vzero;
-          if (kchk) {
-            const float4 gq = *reinterpret_cast<const float4*>(L.Gp + (p * 16 + l16) * GPL + 4 * g4);
-            bgp = C::from(gq.x, gq.y, gq.z, gq.w);
-          }
-#pragma unroll
-          for (int tt = 0; tt < NT; ++tt) {
-            // groups past the KC output rows read rows 0..3 and take zeros
-            const V yk = C::template col4<LD>(L.yb + (kchk ? 4 * g4 : 0) * LD + 16 * tt, l16);
-            dx[p][tt] = C::mma(kchk ? yk : vzero, bgp, dx[p][tt]);
-          }
-#pragma unroll
-          for (int p2 = 0; p2 < NPT; ++p2) {
-            const float4 hq = *reinterpret_cast<const float4*>(L.H + (p * 16 + l16) * GXL + p2 * 16 + 4 * g4);
-            const V bh = C::from(hq.x, hq.y, hq.z, hq.w);
-#pragma unroll
-            for (int tt = 0; tt < NT; ++tt) {
-              const V ax = C::template col4<LD>(L.xc + (p2 * 16 + 4 * g4) * LD + 16 * tt, l16);
-              dx[p][tt] = C::mma(ax, bh, dx[p][tt]);
-            }
-          }
-        }
-        // ---- dY = Gp^T X + M Y -> output rows
+        // ---- dX = Gp Y + H X into the deltas (dX^T[d][u] layout), and
+        // dY = Gp^T X + M Y -> output rows: tile by tile, so that X and Y are
+        // read down their rows once for both
         int drow[4];
         bool dok[4];
 #pragma unroll
@@ -1000,32 +1016,39 @@ void sg_sent_kernel(SentArgs t) {
           drow[e] = __shfl(orow, n, 64);
           dok[e] = n <= K && (n == 0 || drow[e] != row0);
         }
-        V am = vzero;
-        if (krow && kchk) {
-          const float4 mq = *reinterpret_cast<const float4*>(L.Mm + l16 * GPL + 4 * g4);
-          am = C::from(mq.x, mq.y, mq.z, mq.w);
-        }
-        // Gp^T operands, the same for every dim tile
-        V agp[NPT];
+        typedef OutputCols<E, KC> O;
+        typename O::v_t bgp[NPT], am = O::zero();
+        V bh[NPT][NPT], agp[NPT];
+        if (krow) am = O::row(L.Mm + l16 * GPL, g4);
 #pragma unroll
         for (int p = 0; p < NPT; ++p) {
+          bgp[p] = O::row(L.Gp + (p * 16 + l16) * GPL, g4);
           agp[p] = vzero;
           if (krow) {
             const float* gc = L.Gp + (p * 16 + 4 * g4) * GPL + l16;
             agp[p] = C::from(gc[0], gc[GPL], gc[2 * GPL], gc[3 * GPL]);
           }
+#pragma unroll
+          for (int p2 = 0; p2 < NPT; ++p2) {
+            const float4 hq = *reinterpret_cast<const float4*>(L.H + (p * 16 + l16) * GXL + p2 * 16 + 4 * g4);
+            bh[p][p2] = C::from(hq.x, hq.y, hq.z, hq.w);
+          }
         }
 #pragma unroll
         for (int tt = 0; tt < NT; ++tt) {
+          const typename O::v_t yk = O::template col<LD>(L.yb + 16 * tt, g4, l16);
+          V ax[NPT];
+#pragma unroll
+          for (int p = 0; p < NPT; ++p) ax[p] = C::template col4<LD>(L.xc + (p * 16 + 4 * g4) * LD + 16 * tt, l16);
           f32x4_t dy = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
+          for (int p = 0; p < NPT; ++p) dy = C::mma(agp[p], ax[p], dy);
+          dy = O::mma(am, yk, dy);
+#pragma unroll
           for (int p = 0; p < NPT; ++p) {
-            const V bx = C::template col4<LD>(L.xc + (p * 16 + 4 * g4) * LD + 16 * tt, l16);
-            dy = C::mma(agp[p], bx, dy);
-          }
-          {
-            const V yk = C::template col4<LD>(L.yb + (kchk ? 4 * g4 : 0) * LD + 16 * tt, l16);
-            dy = C::mma(am, kchk ? yk : vzero, dy);
+            dx[p][tt] = O::mma(yk, bgp[p], dx[p][tt]);
+#pragma unroll
+            for (int p2 = 0; p2 < NPT; ++p2) dx[p][tt] = C::mma(ax[p2], bh[p][p2], dx[p][tt]);
           }
 #pragma unroll
           for (int e = 0; e < 4; ++e)
