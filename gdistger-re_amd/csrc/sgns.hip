@@ -331,6 +331,7 @@ struct Chunk<float> {
   __device__ static void put4(float* dst, float a, float b, float c, float d) {
     *reinterpret_cast<float4*>(dst) = make_float4(a, b, c, d);
   }
+  __device__ static void put(float* dst, v_t v) { *reinterpret_cast<float4*>(dst) = v; }
   // four consecutive stored elements
   __device__ static v_t load4(const float* src) { return *reinterpret_cast<const float4*>(src); }
 };
@@ -364,6 +365,11 @@ struct Chunk<uint16_t> {
   }
   __device__ static void put4(uint16_t* dst, float a, float b, float c, float d) {
     *reinterpret_cast<uint2*>(dst) = make_uint2(f2bf2(a, b), f2bf2(c, d));
+  }
+  __device__ static void put(uint16_t* dst, v_t v) {
+    U u;
+    u.v = v;
+    *reinterpret_cast<uint2*>(dst) = u.q;
   }
   __device__ static v_t load4(const uint16_t* src) {
     U u;
@@ -810,6 +816,13 @@ void sg_sent_kernel(SentArgs t) {
           yv[r] = make_float4(0.f, 0.f, 0.f, 0.f);
           if (n <= K) yv[r] = *reinterpret_cast<const float4*>(t.syn1 + (uint64_t)row * DIM + 4 * c4);
         }
+        // A lane's part of its pool row is also its operand of the products
+        // over the dims; LDS holds the rows for the reads down the columns.
+        // Up to dim 128 the operands stay in registers for both Gram products
+        // (FP32, dim 128: 13.6 -> 13.3 ms a launch of 131,072 sentences); at
+        // 256 that spills, and they are read back.
+        constexpr bool kKeep = DIM <= 128;
+        V xr[NPT][NT];
 #pragma unroll
         for (int p = 0; p < NPT; ++p)
 #pragma unroll
@@ -822,11 +835,13 @@ void sg_sent_kernel(SentArgs t) {
               u.v = ox[p][tt];
               o[0] = bf2f(u.h[0]); o[1] = bf2f(u.h[1]); o[2] = bf2f(u.h[2]); o[3] = bf2f(u.h[3]);
             }
-            C::put4(L.xc + (p * 16 + l16) * LD + 16 * tt + 4 * g4, o[0] + dx[p][tt][0],
-                    o[1] + dx[p][tt][1], o[2] + dx[p][tt][2], o[3] + dx[p][tt][3]);
+            xr[p][tt] = C::from(o[0] + dx[p][tt][0], o[1] + dx[p][tt][1], o[2] + dx[p][tt][2], o[3] + dx[p][tt][3]);
+            C::put(L.xc + (p * 16 + l16) * LD + 16 * tt + 4 * g4, xr[p][tt]);
           }
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        if constexpr (!kKeep) {
+          __builtin_amdgcn_wave_barrier();
+          __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        }
 #pragma unroll
         for (int p = 0; p < NPT; ++p)
 #pragma unroll
@@ -834,8 +849,9 @@ void sg_sent_kernel(SentArgs t) {
             f32x4_t gx = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int tt = 0; tt < NT; ++tt)
-              gx = C::mma(C::load4(L.xc + (p * 16 + l16) * LD + 16 * tt + 4 * g4),
-                          C::load4(L.xc + (p2 * 16 + l16) * LD + 16 * tt + 4 * g4), gx);
+              gx = kKeep ? C::mma(xr[p][tt], xr[p2][tt], gx)
+                         : C::mma(C::load4(L.xc + (p * 16 + l16) * LD + 16 * tt + 4 * g4),
+                                  C::load4(L.xc + (p2 * 16 + l16) * LD + 16 * tt + 4 * g4), gx);
 #pragma unroll
             for (int e = 0; e < 4; ++e) L.Gx[(p * 16 + 4 * g4 + e) * GXL + p2 * 16 + l16] = gx[e];
           }
@@ -866,7 +882,7 @@ void sg_sent_kernel(SentArgs t) {
 #pragma unroll
           for (int tt = 0; tt < NT; ++tt)
             st = C::mma(krow ? C::load4(L.yb + l16 * LD + 16 * tt + 4 * g4) : vzero,
-                        C::load4(L.xc + (p * 16 + l16) * LD + 16 * tt + 4 * g4), st);
+                        kKeep ? xr[p][tt] : C::load4(L.xc + (p * 16 + l16) * LD + 16 * tt + 4 * g4), st);
           // st[e] = S^T[n = 4 g4 + e][u = p*16 + l16]
           if (kchk) {
 #pragma unroll
