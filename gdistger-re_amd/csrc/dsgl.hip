@@ -39,6 +39,7 @@
 // the M dimension (target, at most 14 distinct negatives, target2), the distinct contexts are the N (or
 // K) dimension in tiles of 16, the embedding dims the K (or N) dimension.
 #include <algorithm>
+#include <type_traits>
 #include <cstring>
 #include <vector>
 
@@ -95,6 +96,19 @@ __device__ __forceinline__ float load_l2(const float* p) {
 // row at a time would expose one memory round trip per row.
 template <int DIM>
 constexpr int row_batch() { return DIM <= 128 ? 16 : 8; }
+
+// A value that is waited for here.
+__device__ __forceinline__ void settle(float& v) { asm volatile("" : "+v"(v)); }
+__device__ __forceinline__ void settle(float2& v) {
+  settle(v.x);
+  settle(v.y);
+}
+__device__ __forceinline__ void settle(float4& v) {
+  settle(v.x);
+  settle(v.y);
+  settle(v.z);
+  settle(v.w);
+}
 
 // A lane's PER consecutive dims of a row, in one access.
 template <int PER>
@@ -281,7 +295,11 @@ __device__ __forceinline__ int first_earlier(const int* v, int n, int i0, int i)
 // SIG: the sigmoid table is copied behind the wavefront's LDS.  Loads return
 // in order, so a table read from memory waits for the atomics and stores of
 // the step before.
-template <int DIM, bool SIG>
+// NX: output rows of a group of 16 lanes, output NX g + x in register x of
+// group g.  Up to eight rows (six negatives) take two: every lane holds
+// outputs, so an epilogue or a store takes half the instructions of four and
+// the product over the outputs two MFMA steps instead of four.
+template <int DIM, int NX, bool SIG>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(DIM <= 128 ? 2 : 1)))
 void dsgl_kernel(DsglArgs a) {
   extern __shared__ __attribute__((aligned(16))) char dsgl_smem[];
@@ -619,7 +637,7 @@ void dsgl_kernel(DsglArgs a) {
         L.ent_cnt[e] = (uint8_t)cnt;
       }
       stage_rows(out_key, 0, yv);
-      if (yr > 8) {
+      if constexpr (NX == 4) {
         // more than six negatives: rows 8 .. 15
         Part yw[8];
         load_rows(out_key, 8, yw);
@@ -645,62 +663,18 @@ void dsgl_kernel(DsglArgs a) {
           xo[et][x] = e4 < E ? L.ent_row[e4] * LDV : zoff;
         }
       }
-      // this lane's output rows 4 g4 .. 4 g4 + 3
-      int ky[4];
-      float om[4];
+      // this lane's outputs
+      int ky[NX];
+      float om[NX];
 #pragma unroll
-      for (int x = 0; x < 4; ++x) {
-        ky[x] = __shfl(out_key, 4 * g4 + x, 64);
-        om[x] = (float)__shfl(out_meta, 4 * g4 + x, 64);
-      }
-      // G = Y X^T and g (dsgl.hpp:1241-1273)
-      {
-        f32x4_t acc[kET];
-#pragma unroll
-        for (int et = 0; et < kET; ++et) acc[et] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-        const float* yrow = l16 < yr ? L.Y + l16 * LDV : L.Z;
-#pragma unroll
-        for (int kc = 0; kc < NT; ++kc) {
-          const float4 ya = *reinterpret_cast<const float4*>(yrow + 16 * kc + 4 * g4);
-#pragma unroll
-          for (int et = 0; et < kET; ++et) {
-            if (et >= ET) break;
-            const float4 xb = *reinterpret_cast<const float4*>(L.V + xg[et] + 16 * kc + 4 * g4);
-            acc[et] = mma4(ya, xb, acc[et]);
-          }
-        }
-#pragma unroll
-        for (int et = 0; et < kET; ++et) {
-          if (et >= ET) break;
-          const int e = 16 * et + l16;
-          const float ec = (float)L.ent_cnt[e];
-          const bool s1 = e < E1;
-#pragma unroll
-          for (int x = 0; x < 4; ++x) {
-            const int i = 4 * g4 + x;
-            const float label = ((i == 0 && s1) || (i == K + 1 && !s1)) ? 1.0f : 0.0f;
-            const float g = (label - dsgl_sig(acc[et][x], sig, a.exact)) * alpha * om[x] * ec;
-            if (i < yr) L.G[i * gl + e] = e < E && !dead(ky[x]) ? g : 0.0f;
-          }
-        }
-      }
-      wave_sync();
-      // this lane's rows 4 g4 .. 4 g4 + 3 of G and Y, rows past yr read from
-      // the zero row
-      const float* yk[4];
-      const float* gk[4];
-      float* dst[4];
-#pragma unroll
-      for (int x = 0; x < 4; ++x) {
-        const int i = 4 * g4 + x;
-        yk[x] = i < yr ? L.Y + i * LDV : L.Z;
-        gk[x] = i < yr ? L.G + i * gl : L.Z;
-        dst[x] = row_of(ky[x]) + l16;
+      for (int x = 0; x < NX; ++x) {
+        ky[x] = __shfl(out_key, NX * g4 + x, 64);
+        om[x] = (float)__shfl(out_meta, NX * g4 + x, 64);
       }
       // ---- the next step's output rows, where neither sentence ends (so the
       // batch stays) and none of them is moved by this step: their loads are
       // in flight during this step's products
-      if (yr <= 8 && pos[0] + 1 < len[0] && pos[1] + 1 < len[1]) {
+      if (NX == 2 && pos[0] + 1 < len[0] && pos[1] + 1 < len[1]) {
         const int key_now = out_key, nst_now = nst;
         outputs(pos[0] + 1, pos[1] + 1, out_key, out_meta);
         bool moved = false;
@@ -715,23 +689,76 @@ void dsgl_kernel(DsglArgs a) {
           nst = nst_now;
         }
       }
-      float4 yb[NT];
+      // the row of the outputs that lane l16 supplies to a product
+      const int arow = NX == 4 ? l16 : (l16 & 3) < 2 ? 2 * (l16 >> 2) + (l16 & 3) : yr;
+      // The two products over the contexts, for a number of their tiles that
+      // is known when they are compiled: reads in flight and no branch in
+      // between.
+      auto over_tiles = [&](auto&& body) {
+        if (ET == 1) body(std::integral_constant<int, 1>{});
+        else if (ET == 2) body(std::integral_constant<int, 2>{});
+        else body(std::integral_constant<int, kET>{});
+      };
+      // G = Y X^T and g (dsgl.hpp:1241-1273)
+      over_tiles([&](auto tiles) {
+        constexpr int T = decltype(tiles)::value;
+        f32x4_t acc[T];
+#pragma unroll
+        for (int et = 0; et < T; ++et) acc[et] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        const float* yrow = arow < yr ? L.Y + arow * LDV : L.Z;
+#pragma unroll
+        for (int kc = 0; kc < NT; ++kc) {
+          const float4 ya = *reinterpret_cast<const float4*>(yrow + 16 * kc + 4 * g4);
+#pragma unroll
+          for (int et = 0; et < T; ++et) {
+            const float4 xb = *reinterpret_cast<const float4*>(L.V + xg[et] + 16 * kc + 4 * g4);
+            acc[et] = mma4(ya, xb, acc[et]);
+          }
+        }
+#pragma unroll
+        for (int et = 0; et < T; ++et) {
+          const int e = 16 * et + l16;
+          const float ec = (float)L.ent_cnt[e];
+          const bool s1 = e < E1;
+#pragma unroll
+          for (int x = 0; x < NX; ++x) {
+            const int i = NX * g4 + x;
+            const float label = ((i == 0 && s1) || (i == K + 1 && !s1)) ? 1.0f : 0.0f;
+            const float g = (label - dsgl_sig(acc[et][x], sig, a.exact)) * alpha * om[x] * ec;
+            if (i < yr) L.G[i * gl + e] = e < E && !dead(ky[x]) ? g : 0.0f;
+          }
+        }
+      });
+      wave_sync();
+      // this lane's rows of G and Y, rows past yr read from the zero row
+      const float* yk[NX];
+      const float* gk[NX];
+      float* dst[NX];
+#pragma unroll
+      for (int x = 0; x < NX; ++x) {
+        const int i = NX * g4 + x;
+        yk[x] = i < yr ? L.Y + i * LDV : L.Z;
+        gk[x] = i < yr ? L.G + i * gl : L.Z;
+        dst[x] = row_of(ky[x]) + l16;
+      }
+      float yb[NT][NX];
 #pragma unroll
       for (int tt = 0; tt < NT; ++tt)
-        yb[tt] = make_float4(yk[0][16 * tt + l16], yk[1][16 * tt + l16], yk[2][16 * tt + l16], yk[3][16 * tt + l16]);
-      // dY = G X: lane holds dY[4 g4 + x][16 tt + l16], added to the row of
-      // output 4 g4 + x: the targets' rows in syn1 by atomics, the negatives'
+#pragma unroll
+        for (int x = 0; x < NX; ++x) yb[tt][x] = yk[x][16 * tt + l16];
+      // dY = G X: lane holds dY[NX g4 + x][16 tt + l16], added to the row of
+      // output NX g4 + x: the targets' rows in syn1 by atomics, the negatives'
       // in the batch buffer, which is this wavefront's own, by a store of the
       // staged row and its update (the memory adds some 20 G requests of 64
       // bytes per second, and these were 5 of a step's 7 rows)
-      {
+      over_tiles([&](auto tiles) {
+        constexpr int T = decltype(tiles)::value;
         f32x4_t acc[NT];
 #pragma unroll
         for (int tt = 0; tt < NT; ++tt) acc[tt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-        const float* grow = l16 < yr ? L.G + l16 * gl : L.Z;
+        const float* grow = arow < yr ? L.G + arow * gl : L.Z;
 #pragma unroll
-        for (int ec = 0; ec < kET; ++ec) {
-          if (ec >= ET) break;
+        for (int ec = 0; ec < T; ++ec) {
           const float4 ga = *reinterpret_cast<const float4*>(grow + 16 * ec + 4 * g4);
 #pragma unroll
           for (int tt = 0; tt < NT; ++tt) {
@@ -741,31 +768,40 @@ void dsgl_kernel(DsglArgs a) {
             acc[tt] = mma4(ga, make_float4(xv[0], xv[1], xv[2], xv[3]), acc[tt]);
           }
         }
+        // The next step's rows have to be here before the stores and atomics
+        // go out: a wait for them afterwards is a wait for those as well.
+        if constexpr (NX == 2) {
 #pragma unroll
-        for (int x = 0; x < 4; ++x) {
-          const int i = 4 * g4 + x;
+          for (int r = 0; r < 8; ++r) settle(yv[r]);
+        }
+#pragma unroll
+        for (int x = 0; x < NX; ++x) {
+          const int i = NX * g4 + x;
           if (i > 0 && i <= K && !dead(ky[x])) {
 #pragma unroll
-            for (int tt = 0; tt < NT; ++tt) {
-              const float y = x == 0 ? yb[tt].x : (x == 1 ? yb[tt].y : (x == 2 ? yb[tt].z : yb[tt].w));
-              dst[x][16 * tt] = y + acc[tt][x];
-            }
+            for (int tt = 0; tt < NT; ++tt) dst[x][16 * tt] = yb[tt][x] + acc[tt][x];
           } else if (i == 0 || i == K + 1) {
 #pragma unroll
             for (int tt = 0; tt < NT; ++tt) atomicAdd(dst[x] + 16 * tt, acc[tt][x]);
           }
         }
-      }
+      });
       // dX = G^T Y into the sentence buffers: lane holds dX[16 et + 4 g4 + x][16 tt + l16]
       {
 #pragma unroll
         for (int et = 0; et < kET; ++et) {
           if (et >= ET) break;
-          const float4 a4 = make_float4(gk[0][16 * et + l16], gk[1][16 * et + l16], gk[2][16 * et + l16],
-                                        gk[3][16 * et + l16]);
           f32x4_t acc[NT], xv[NT];
+          float ga[NX];
 #pragma unroll
-          for (int tt = 0; tt < NT; ++tt) acc[tt] = mma4(a4, yb[tt], f32x4_t{0.f, 0.f, 0.f, 0.f});
+          for (int x = 0; x < NX; ++x) ga[x] = gk[x][16 * et + l16];
+#pragma unroll
+          for (int tt = 0; tt < NT; ++tt) {
+            acc[tt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int x = 0; x < NX; ++x)
+              acc[tt] = __builtin_amdgcn_mfma_f32_16x16x4f32(ga[x], yb[tt][x], acc[tt], 0, 0, 0);
+          }
           // all reads, then all writes: a branch around each row's would make
           // every one of them a round trip.  Rows past E are the zero row,
           // which gets zeros.
@@ -900,9 +936,9 @@ __global__ void dsgl_state_init_kernel(unsigned long long* actual, float* alpha,
   if (blockIdx.x == 0 && threadIdx.x == 0) *kept = 0ull;
 }
 
-template <int DIM, bool SIG>
-int launch_dims(dg_ctx* ctx, const DsglArgs& a, size_t lds, unsigned grid) {
-  auto k = dsgl_kernel<DIM, SIG>;
+template <int DIM, int NX, bool SIG>
+int launch_unit(dg_ctx* ctx, const DsglArgs& a, size_t lds, unsigned grid) {
+  auto k = dsgl_kernel<DIM, NX, SIG>;
   hipError_t e = hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   if (e != hipSuccess) return dg_fail(ctx, DG_ERR_HIP, "DSGL kernel LDS attribute: %s", hipGetErrorString(e));
   k<<<grid, 64, lds, ctx->stream>>>(a);
@@ -911,15 +947,22 @@ int launch_dims(dg_ctx* ctx, const DsglArgs& a, size_t lds, unsigned grid) {
   return DG_OK;
 }
 
+template <int DIM>
+int launch_dims(dg_ctx* ctx, const DsglArgs& a, bool sig, size_t lds, unsigned grid) {
+  if (a.yrows <= 8)
+    return sig ? launch_unit<DIM, 2, true>(ctx, a, lds, grid) : launch_unit<DIM, 2, false>(ctx, a, lds, grid);
+  return sig ? launch_unit<DIM, 4, true>(ctx, a, lds, grid) : launch_unit<DIM, 4, false>(ctx, a, lds, grid);
+}
+
 constexpr size_t kSigBytes = ((kDsglExpTable + 1) * sizeof(float) + 15) & ~(size_t)15;
 
 // Workgroups (wavefronts) of a kernel that fit a CU.
-template <int DIM, bool SIG>
-int resident_dims(dg_ctx* ctx, size_t lds, unsigned* per_cu) {
+template <int DIM, int NX, bool SIG>
+int resident_unit(dg_ctx* ctx, size_t lds, unsigned* per_cu) {
   int n = 0;
-  hipError_t e = hipFuncSetAttribute((const void*)dsgl_kernel<DIM, SIG>,
+  hipError_t e = hipFuncSetAttribute((const void*)dsgl_kernel<DIM, NX, SIG>,
                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-  if (e == hipSuccess) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, dsgl_kernel<DIM, SIG>, 64, lds);
+  if (e == hipSuccess) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, dsgl_kernel<DIM, NX, SIG>, 64, lds);
   if (e != hipSuccess) return dg_fail(ctx, DG_ERR_HIP, "DSGL occupancy: %s", hipGetErrorString(e));
   *per_cu = n < 1 ? 1u : (unsigned)n;
   return DG_OK;
@@ -933,9 +976,12 @@ int plan_dims(dg_ctx* ctx, uint32_t lcap, uint32_t vcap, uint32_t ncap, uint32_t
     return dg_fail(ctx, DG_ERR_UNSUPPORTED,
                    "DSGL form: sentences of %u tokens at dim %d need %zu bytes of LDS per wavefront "
                    "(160 KB available)", lcap, DIM, *lds);
-  DG_CHECK((resident_dims<DIM, false>(ctx, *lds, per_cu)));
+  const bool few = yrows <= 8;
+  DG_CHECK((few ? resident_unit<DIM, 2, false>(ctx, *lds, per_cu) : resident_unit<DIM, 4, false>(ctx, *lds, per_cu)));
   *per_cu_sig = 0;
-  if (*lds + kSigBytes <= 160 * 1024) DG_CHECK((resident_dims<DIM, true>(ctx, *lds + kSigBytes, per_cu_sig)));
+  const size_t more = *lds + kSigBytes;
+  if (more <= 160 * 1024)
+    DG_CHECK((few ? resident_unit<DIM, 2, true>(ctx, more, per_cu_sig) : resident_unit<DIM, 4, true>(ctx, more, per_cu_sig)));
   return DG_OK;
 }
 
@@ -1056,9 +1102,9 @@ int dg_dsgl_train(dg_ctx* ctx, const dg_dsgl_call& c, uint64_t* kept, double* ms
     a.key = dg_epoch_key(c.seed, c.epoch0 + ep);
     DG_CHECK(dg_time_begin(ctx, "sgns_dsgl", &tk));
     switch (c.dim) {
-      case 64: DG_CHECK((sig ? launch_dims<64, true>(ctx, a, lds, grid) : launch_dims<64, false>(ctx, a, lds, grid))); break;
-      case 128: DG_CHECK((sig ? launch_dims<128, true>(ctx, a, lds, grid) : launch_dims<128, false>(ctx, a, lds, grid))); break;
-      default: DG_CHECK((sig ? launch_dims<256, true>(ctx, a, lds, grid) : launch_dims<256, false>(ctx, a, lds, grid))); break;
+      case 64: DG_CHECK(launch_dims<64>(ctx, a, sig, lds, grid)); break;
+      case 128: DG_CHECK(launch_dims<128>(ctx, a, sig, lds, grid)); break;
+      default: DG_CHECK(launch_dims<256>(ctx, a, sig, lds, grid)); break;
     }
     DG_CHECK(dg_time_end(ctx, tk));
   }
