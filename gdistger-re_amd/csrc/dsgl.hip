@@ -613,15 +613,20 @@ void dsgl_kernel(DsglArgs a) {
       {
         const int i = b + li + (b + li >= W ? 1 : 0);
         const int c = pos[hs] - W + i;
-        if (li < span && c >= 0 && c < len[hs]) my = L.slot[hs * lcap + c];
+        const int len_h = hs ? len[1] : len[0];
+        const bool in = li < span && c >= 0 && c < len_h;
+        const int at = L.slot[hs * lcap + (in ? c : 0)];
+        if (in) my = at;
       }
       L.tmp[lane] = my;
       wave_sync();
       bool first = my >= 0;
       int cnt = 0;
+      int4 o4 = *reinterpret_cast<const int4*>(L.tmp + hs * 32);
       for (int j0 = 0; j0 < span; j0 += 4) {  // entries past the window are -1
-        const int4 o4 = *reinterpret_cast<const int4*>(L.tmp + hs * 32 + j0);
-        const int o[4] = {o4.x, o4.y, o4.z, o4.w};
+        const int4 now = o4;
+        o4 = *reinterpret_cast<const int4*>(L.tmp + hs * 32 + ((j0 + 4) & 31));
+        const int o[4] = {now.x, now.y, now.z, now.w};
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
           cnt += o[j] == my ? 1 : 0;
@@ -656,11 +661,13 @@ void dsgl_kernel(DsglArgs a) {
 #pragma unroll
       for (int et = 0; et < kET; ++et) {
         const int e = 16 * et + l16;
-        xg[et] = e < E ? L.ent_row[e] * LDV : zoff;
+        const int at = L.ent_row[e] * LDV;  // read past E too: no branch around a read
+        xg[et] = e < E ? at : zoff;
 #pragma unroll
         for (int x = 0; x < 4; ++x) {
           const int e4 = 16 * et + 4 * g4 + x;
-          xo[et][x] = e4 < E ? L.ent_row[e4] * LDV : zoff;
+          const int at4 = L.ent_row[e4] * LDV;
+          xo[et][x] = e4 < E ? at4 : zoff;
         }
       }
       // this lane's outputs
