@@ -273,18 +273,27 @@ __device__ __forceinline__ float dsgl_sig(float f, const float* expt, int exact)
 }
 
 // For lane i = i0 + lane of a list v[0, n): the first j < i with v[j] ==
-// v[i], or -1.  Earlier entries are compared 64 at a time from a register
-// (v_readlane), not by a loop of dependent LDS reads per lane.
+// v[i], or -1.  Earlier entries are compared from a register (v_readlane), 64
+// at a time and the last first, so that the first match stays without a test
+// whether there is one: four instructions an entry, eight entries unrolled.
 __device__ __forceinline__ int first_earlier(const int* v, int n, int i0, int i) {
   const int lane = (int)(threadIdx.x & 63u);
-  const int w = i < n ? v[i] : 0;
+  const int w = v[i < n ? i : n - 1];
   int first_of = -1;
-  for (int c0 = 0; c0 <= i0; c0 += 64) {
-    const int cj = c0 + lane < n ? v[c0 + lane] : 0;
-    const int kn = n - c0 < 64 ? n - c0 : 64;
-    for (int k = 0; k < kn; ++k) {
-      const int vk = __builtin_amdgcn_readlane(cj, k);
-      if (first_of < 0 && c0 + k < i && vk == w) first_of = c0 + k;
+  // of the entries beside lane i's own, those of the lanes before it
+  for (int k0 = n - i0 < 64 ? ((n - i0 - 1) & ~7) : 56; k0 >= 0; k0 -= 8) {
+#pragma unroll
+    for (int k = 7; k >= 0; --k) {
+      const bool hit = __builtin_amdgcn_readlane(w, k0 + k) == w && k0 + k < lane;
+      first_of = hit ? i0 + k0 + k : first_of;
+    }
+  }
+  for (int c0 = i0 - 64; c0 >= 0; c0 -= 64) {
+    const int cj = v[c0 + lane];
+    for (int k0 = 56; k0 >= 0; k0 -= 8) {
+#pragma unroll
+      for (int k = 7; k >= 0; --k)
+        first_of = __builtin_amdgcn_readlane(cj, k0 + k) == w ? c0 + k0 + k : first_of;
     }
   }
   return i < n ? first_of : -1;
@@ -727,11 +736,19 @@ void dsgl_kernel(DsglArgs a) {
           const int e = 16 * et + l16;
           const float ec = (float)L.ent_cnt[e];
           const bool s1 = e < E1;
+          float sg[NX];
+          if (a.exact) {
+#pragma unroll
+            for (int x = 0; x < NX; ++x) sg[x] = dsgl_sig(acc[et][x], sig, 1);
+          } else {
+#pragma unroll
+            for (int x = 0; x < NX; ++x) sg[x] = dsgl_sig(acc[et][x], sig, 0);
+          }
 #pragma unroll
           for (int x = 0; x < NX; ++x) {
             const int i = NX * g4 + x;
             const float label = ((i == 0 && s1) || (i == K + 1 && !s1)) ? 1.0f : 0.0f;
-            const float g = (label - dsgl_sig(acc[et][x], sig, a.exact)) * alpha * om[x] * ec;
+            const float g = (label - sg[x]) * alpha * om[x] * ec;
             if (i < yr) L.G[i * gl + e] = e < E && !dead(ky[x]) ? g : 0.0f;
           }
         }
