@@ -97,20 +97,10 @@ __device__ __forceinline__ float load_l2(const float* p) {
 template <int DIM>
 constexpr int row_batch() { return DIM <= 128 ? 16 : 8; }
 
-// A value that is waited for here.
-__device__ __forceinline__ void settle(float& v) { asm volatile("" : "+v"(v)); }
-__device__ __forceinline__ void settle(float2& v) {
-  settle(v.x);
-  settle(v.y);
-}
-__device__ __forceinline__ void settle(float4& v) {
-  settle(v.x);
-  settle(v.y);
-  settle(v.z);
-  settle(v.w);
-}
-
-// A lane's PER consecutive dims of a row, in one access.
+// A lane's PER consecutive dims of a row, in one access.  (Compiler vectors:
+// an array of float4 structures stays in scratch memory.)
+typedef float f2_t __attribute__((ext_vector_type(2)));
+typedef float f4_t __attribute__((ext_vector_type(4)));
 template <int PER>
 struct RowPart;
 template <>
@@ -119,20 +109,25 @@ struct RowPart<1> {
 };
 template <>
 struct RowPart<2> {
-  typedef float2 t;
+  typedef f2_t t;
 };
 template <>
 struct RowPart<4> {
-  typedef float4 t;
+  typedef f4_t t;
 };
+
+// A value that is waited for here.
+template <typename T>
+__device__ __forceinline__ void settle(T& v) { asm volatile("" : "+v"(v)); }
+
 __device__ __forceinline__ float row_load_l2(const float* p, float) { return load_l2(p); }
-__device__ __forceinline__ float2 row_load_l2(const float* p, float2) {
+__device__ __forceinline__ f2_t row_load_l2(const float* p, f2_t) {
   const uint64_t v = __hip_atomic_load(reinterpret_cast<const uint64_t*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  return make_float2(__uint_as_float((uint32_t)v), __uint_as_float((uint32_t)(v >> 32)));
+  return f2_t{__uint_as_float((uint32_t)v), __uint_as_float((uint32_t)(v >> 32))};
 }
-__device__ __forceinline__ float4 row_load_l2(const float* p, float4) {
-  const float2 a = row_load_l2(p, float2()), b = row_load_l2(p + 2, float2());
-  return make_float4(a.x, a.y, b.x, b.y);
+__device__ __forceinline__ f4_t row_load_l2(const float* p, f4_t) {
+  const f2_t a = row_load_l2(p, f2_t{0.f, 0.f}), b = row_load_l2(p + 2, f2_t{0.f, 0.f});
+  return f4_t{a.x, a.y, b.x, b.y};
 }
 
 __device__ __forceinline__ uint64_t uni64(uint64_t v) {
@@ -590,7 +585,7 @@ void dsgl_kernel(DsglArgs a) {
 #pragma unroll
         for (int r = 0; r < 8; ++r) {
           const int i = r0 + r <= K + 1 ? r0 + r : K + 1;
-          y[r] = row_load_l2(row_of(__builtin_amdgcn_readlane(key, i)) + PER * lane, Part());
+          y[r] = row_load_l2(row_of(__builtin_amdgcn_readlane(key, i)) + PER * lane, Part(0.0f));
         }
       };
       auto stage_rows = [&](int key, int r0, const Part (&y)[8]) {
@@ -598,7 +593,7 @@ void dsgl_kernel(DsglArgs a) {
         for (int r = 0; r < 8; ++r)
           if (r0 + r < yr)
             *reinterpret_cast<Part*>(L.Y + (r0 + r) * LDV + PER * lane) =
-                dead(__builtin_amdgcn_readlane(key, r0 + r)) ? Part() : y[r];
+                dead(__builtin_amdgcn_readlane(key, r0 + r)) ? Part(0.0f) : y[r];
       };
       if (!have) {
         outputs(pos[0], pos[1], out_key, out_meta);
