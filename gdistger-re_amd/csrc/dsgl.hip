@@ -116,10 +116,6 @@ struct RowPart<4> {
   typedef f4_t t;
 };
 
-// A value that is waited for here.
-template <typename T>
-__device__ __forceinline__ void settle(T& v) { asm volatile("" : "+v"(v)); }
-
 __device__ __forceinline__ float row_load_l2(const float* p, float) { return load_l2(p); }
 __device__ __forceinline__ f2_t row_load_l2(const float* p, f2_t) {
   const uint64_t v = __hip_atomic_load(reinterpret_cast<const uint64_t*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -200,9 +196,6 @@ struct DsglLds {
   int* nslot;     // [ncap] batch-buffer index of each draw
   int* nid;       // [ncap] distinct negatives
   int* ent_row;   // [kEntCap] row of each distinct context (s * vcap + word index)
-  int* out_id;    // [16]
-  int* out_meta;  // [16]
-  int* out_slot;  // [16]
   uint8_t* ent_cnt;  // [kEntCap] occurrences of each distinct context (<= 32)
   int* tmp;       // [64], in G's storage
 };
@@ -215,9 +208,14 @@ __host__ __device__ inline size_t dsgl_lds_bytes(uint32_t lcap, uint32_t vcap, u
                                                  uint32_t yrows, uint32_t gl) {
   constexpr int LDV = dsgl_ldv<DIM>();
   size_t f = (size_t)2 * vcap * LDV + (size_t)yrows * LDV + dsgl_g_floats(yrows, gl) + LDV;
-  size_t i = (size_t)2 * 2 * lcap + 2 * (size_t)vcap + 3 * (size_t)ncap + kEntCap + 3 * 16;
+  size_t i = (size_t)2 * 2 * lcap + 2 * (size_t)vcap + 3 * (size_t)ncap + kEntCap;
   return ((f * 4 + i * 4 + kEntCap) + 15) & ~(size_t)15;
 }
+
+// Bytes more that the default number of workers is planned with: it is part
+// of the results (a worker is a share of the corpus), so it does not follow
+// what the layout has come to take.
+constexpr size_t kPlanBytes = 192;
 
 template <int DIM>
 __device__ DsglLds dsgl_carve(char* base, uint32_t lcap, uint32_t vcap, uint32_t ncap, uint32_t yrows,
@@ -249,12 +247,6 @@ __device__ DsglLds dsgl_carve(char* base, uint32_t lcap, uint32_t vcap, uint32_t
   p += ncap;
   L.ent_row = p;
   p += kEntCap;
-  L.out_id = p;
-  p += 16;
-  L.out_meta = p;
-  p += 16;
-  L.out_slot = p;
-  p += 16;
   L.ent_cnt = reinterpret_cast<uint8_t*>(p);
   return L;
 }
@@ -684,8 +676,10 @@ void dsgl_kernel(DsglArgs a) {
       }
       // ---- the next step's output rows, where neither sentence ends (so the
       // batch stays) and none of them is moved by this step: their loads are
-      // in flight during this step's products
-      if (NX == 2 && pos[0] + 1 < len[0] && pos[1] + 1 < len[1]) {
+      // in flight during this step's products.  A sigmoid table in memory
+      // would wait for them, so they go out behind its reads then.
+      auto ahead = [&]() {
+        if (pos[0] + 1 >= len[0] || pos[1] + 1 >= len[1]) return;
         const int key_now = out_key, nst_now = nst;
         outputs(pos[0] + 1, pos[1] + 1, out_key, out_meta);
         bool moved = false;
@@ -699,7 +693,8 @@ void dsgl_kernel(DsglArgs a) {
           --neg_count;  // drawn again by that step
           nst = nst_now;
         }
-      }
+      };
+      if constexpr (NX == 2 && SIG) ahead();
       // the row of the outputs that lane l16 supplies to a product
       const int arow = NX == 4 ? l16 : (l16 & 3) < 2 ? 2 * (l16 >> 2) + (l16 & 3) : yr;
       // The two products over the contexts, for a number of their tiles that
@@ -749,6 +744,7 @@ void dsgl_kernel(DsglArgs a) {
         }
       });
       wave_sync();
+      if constexpr (NX == 2 && !SIG) ahead();
       // this lane's rows of G and Y, rows past yr read from the zero row
       const float* yk[NX];
       const float* gk[NX];
@@ -786,12 +782,6 @@ void dsgl_kernel(DsglArgs a) {
             for (int x = 0; x < 4; ++x) xv[x] = L.V[xo[ec][x] + 16 * tt + l16];
             acc[tt] = mma4(ga, make_float4(xv[0], xv[1], xv[2], xv[3]), acc[tt]);
           }
-        }
-        // The next step's rows have to be here before the stores and atomics
-        // go out: a wait for them afterwards is a wait for those as well.
-        if constexpr (NX == 2) {
-#pragma unroll
-          for (int r = 0; r < 8; ++r) settle(yv[r]);
         }
 #pragma unroll
         for (int x = 0; x < NX; ++x) {
@@ -990,7 +980,8 @@ int resident_unit(dg_ctx* ctx, size_t lds, unsigned* per_cu) {
 template <int DIM>
 int plan_dims(dg_ctx* ctx, uint32_t lcap, uint32_t vcap, uint32_t ncap, uint32_t yrows, uint32_t gl,
               size_t* lds, unsigned* per_cu, unsigned* per_cu_sig) {
-  *lds = dsgl_lds_bytes<DIM>(lcap, vcap, ncap, yrows, gl);
+  const size_t used = dsgl_lds_bytes<DIM>(lcap, vcap, ncap, yrows, gl);
+  *lds = used + kPlanBytes;
   if (*lds > 160 * 1024)
     return dg_fail(ctx, DG_ERR_UNSUPPORTED,
                    "DSGL form: sentences of %u tokens at dim %d need %zu bytes of LDS per wavefront "
@@ -998,7 +989,7 @@ int plan_dims(dg_ctx* ctx, uint32_t lcap, uint32_t vcap, uint32_t ncap, uint32_t
   const bool few = yrows <= 8;
   DG_CHECK((few ? resident_unit<DIM, 2, false>(ctx, *lds, per_cu) : resident_unit<DIM, 4, false>(ctx, *lds, per_cu)));
   *per_cu_sig = 0;
-  const size_t more = *lds + kSigBytes;
+  const size_t more = used + kSigBytes;
   if (more <= 160 * 1024)
     DG_CHECK((few ? resident_unit<DIM, 2, true>(ctx, more, per_cu_sig) : resident_unit<DIM, 4, true>(ctx, more, per_cu_sig)));
   return DG_OK;
@@ -1075,7 +1066,7 @@ int dg_dsgl_train(dg_ctx* ctx, const dg_dsgl_call& c, uint64_t* kept, double* ms
   const unsigned grid = c.deterministic ? 1u : (unsigned)std::min<uint64_t>(workers, resident);
   // the sigmoid table goes to LDS where that leaves as many wavefronts resident
   const bool sig = (uint64_t)per_cu_sig * (uint64_t)ctx->num_cus >= grid;
-  if (sig) lds += kSigBytes;
+  lds += sig ? kSigBytes - kPlanBytes : 0;
   const uint64_t stride = ((uint64_t)2 * lcap + 2 * (uint64_t)ncap) * c.dim;
   DG_CHECK(dg_reserve(ctx, &st->scratch, &st->scratch_cap, (size_t)(grid * stride)));
   DG_CHECK(dg_reserve(ctx, &st->actual, &st->actual_cap, (size_t)workers));
