@@ -288,13 +288,20 @@ __device__ __forceinline__ int first_earlier(const int* v, int n, int i0, int i)
 
 // Two wavefronts per SIMD up to dim 128 (at most 256 registers): the LDS of
 // a wavefront (27 KB at dim 128 on 22-token walks) fits six per CU.
+// Bound by its chain of steps, 18 thousand cycles each at dim 128: about a
+// quarter at sentence and batch ends, half in the three products and their
+// LDS reads, the rest in the choice of outputs and contexts.  One epoch over
+// 65,536 vertices (14.4M words, dim 128): 51.8 ms, 85.3 when each row, branch
+// and atomic was waited for; a round of 2.24M walks over 2.2M vertices 183 ms
+// (301).
 // SIG: the sigmoid table is copied behind the wavefront's LDS.  Loads return
 // in order, so a table read from memory waits for the atomics and stores of
-// the step before.
+// the step before (53.3 and 191 ms).
 // NX: output rows of a group of 16 lanes, output NX g + x in register x of
 // group g.  Up to eight rows (six negatives) take two: every lane holds
 // outputs, so an epilogue or a store takes half the instructions of four and
-// the product over the outputs two MFMA steps instead of four.
+// the product over the outputs two MFMA steps instead of four (the epoch
+// above 56.3 ms with two, 65.6 with four).
 template <int DIM, int NX, bool SIG>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(DIM <= 128 ? 2 : 1)))
 void dsgl_kernel(DsglArgs a) {
@@ -1064,7 +1071,8 @@ int dg_dsgl_train(dg_ctx* ctx, const dg_dsgl_call& c, uint64_t* kept, double* ms
   uint32_t workers = c.workers ? c.workers : (uint32_t)dflt;
   if ((uint64_t)workers > c.n_walks + c.n_tok) workers = (uint32_t)std::max<uint64_t>(1, (c.n_walks + c.n_tok) / 64);
   const unsigned grid = c.deterministic ? 1u : (unsigned)std::min<uint64_t>(workers, resident);
-  // the sigmoid table goes to LDS where that leaves as many wavefronts resident
+  // the sigmoid table goes to LDS where that leaves as many wavefronts resident:
+  // it saves 3 to 4% of a launch, a wavefront less per CU costs a fifth
   const bool sig = (uint64_t)per_cu_sig * (uint64_t)ctx->num_cus >= grid;
   lds += sig ? kSigBytes - kPlanBytes : 0;
   const uint64_t stride = ((uint64_t)2 * lcap + 2 * (uint64_t)ncap) * c.dim;
