@@ -39,7 +39,6 @@
 // the M dimension (target, at most 14 distinct negatives, target2), the distinct contexts are the N (or
 // K) dimension in tiles of 16, the embedding dims the K (or N) dimension.
 #include <algorithm>
-#include <type_traits>
 #include <cstring>
 #include <vector>
 
@@ -86,45 +85,18 @@ __device__ __forceinline__ float load_l2(const float* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// The rows a wavefront reads back are its own scratch rows (and, in the
-// deterministic order, every row).  A wavefront's operations on one address
-// are performed in their order, so neither a wait for its stores and atomics
-// nor a release stands between them and the loads above.
+// Waits until every memory operation this wavefront has issued is complete:
+// its stores and atomics have reached the level-2 cache of its XCD, where
+// the level-2 loads above read them.  The rows a wavefront reads back this
+// way are its own scratch rows (and, in the deterministic order, every row),
+// so an agent-scope release, which also writes the XCD's level-2 cache back
+// to memory, is not needed; it made each step 38% slower.
+__device__ __forceinline__ void drain() { __builtin_amdgcn_s_waitcnt(0); }
 
 // Rows whose loads are issued together before any of them is used: the
 // kernel runs at one or two wavefronts per SIMD (its LDS sets that), so a
 // row at a time would expose one memory round trip per row.
-template <int DIM>
-constexpr int row_batch() { return DIM <= 128 ? 16 : 8; }
-
-// A lane's PER consecutive dims of a row, in one access.  (Compiler vectors:
-// an array of float4 structures stays in scratch memory.)
-typedef float f2_t __attribute__((ext_vector_type(2)));
-typedef float f4_t __attribute__((ext_vector_type(4)));
-template <int PER>
-struct RowPart;
-template <>
-struct RowPart<1> {
-  typedef float t;
-};
-template <>
-struct RowPart<2> {
-  typedef f2_t t;
-};
-template <>
-struct RowPart<4> {
-  typedef f4_t t;
-};
-
-__device__ __forceinline__ float row_load_l2(const float* p, float) { return load_l2(p); }
-__device__ __forceinline__ f2_t row_load_l2(const float* p, f2_t) {
-  const uint64_t v = __hip_atomic_load(reinterpret_cast<const uint64_t*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  return f2_t{__uint_as_float((uint32_t)v), __uint_as_float((uint32_t)(v >> 32))};
-}
-__device__ __forceinline__ f4_t row_load_l2(const float* p, f4_t) {
-  const f2_t a = row_load_l2(p, f2_t{0.f, 0.f}), b = row_load_l2(p + 2, f2_t{0.f, 0.f});
-  return f4_t{a.x, a.y, b.x, b.y};
-}
+constexpr int kRowBatch = 8;
 
 __device__ __forceinline__ uint64_t uni64(uint64_t v) {
   const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v);
@@ -196,6 +168,9 @@ struct DsglLds {
   int* nslot;     // [ncap] batch-buffer index of each draw
   int* nid;       // [ncap] distinct negatives
   int* ent_row;   // [kEntCap] row of each distinct context (s * vcap + word index)
+  int* out_id;    // [16]
+  int* out_meta;  // [16]
+  int* out_slot;  // [16]
   uint8_t* ent_cnt;  // [kEntCap] occurrences of each distinct context (<= 32)
   int* tmp;       // [64], in G's storage
 };
@@ -208,14 +183,9 @@ __host__ __device__ inline size_t dsgl_lds_bytes(uint32_t lcap, uint32_t vcap, u
                                                  uint32_t yrows, uint32_t gl) {
   constexpr int LDV = dsgl_ldv<DIM>();
   size_t f = (size_t)2 * vcap * LDV + (size_t)yrows * LDV + dsgl_g_floats(yrows, gl) + LDV;
-  size_t i = (size_t)2 * 2 * lcap + 2 * (size_t)vcap + 3 * (size_t)ncap + kEntCap;
+  size_t i = (size_t)2 * 2 * lcap + 2 * (size_t)vcap + 3 * (size_t)ncap + kEntCap + 3 * 16;
   return ((f * 4 + i * 4 + kEntCap) + 15) & ~(size_t)15;
 }
-
-// Bytes more that the default number of workers is planned with: it is part
-// of the results (a worker is a share of the corpus), so it does not follow
-// what the layout has come to take.
-constexpr size_t kPlanBytes = 192;
 
 template <int DIM>
 __device__ DsglLds dsgl_carve(char* base, uint32_t lcap, uint32_t vcap, uint32_t ncap, uint32_t yrows,
@@ -247,40 +217,36 @@ __device__ DsglLds dsgl_carve(char* base, uint32_t lcap, uint32_t vcap, uint32_t
   p += ncap;
   L.ent_row = p;
   p += kEntCap;
+  L.out_id = p;
+  p += 16;
+  L.out_meta = p;
+  p += 16;
+  L.out_slot = p;
+  p += 16;
   L.ent_cnt = reinterpret_cast<uint8_t*>(p);
   return L;
 }
 
 __device__ __forceinline__ float dsgl_sig(float f, const float* expt, int exact) {
   if (exact) return (float)(1.0 / (1.0 + exp(-(double)f)));
-  // read at a clamped index and selected afterwards: no branch per value
-  const float fc = fminf(fmaxf(f, -(float)kDsglMaxExp), (float)kDsglMaxExp);
-  const float v = expt[(int)((fc + (float)kDsglMaxExp) * (float)(kDsglExpTable / kDsglMaxExp / 2))];
-  return f > (float)kDsglMaxExp ? 1.0f : (f < -(float)kDsglMaxExp ? 0.0f : v);
+  if (f > (float)kDsglMaxExp) return 1.0f;
+  if (f < -(float)kDsglMaxExp) return 0.0f;
+  return expt[(int)((f + (float)kDsglMaxExp) * (float)(kDsglExpTable / kDsglMaxExp / 2))];
 }
 
 // For lane i = i0 + lane of a list v[0, n): the first j < i with v[j] ==
-// v[i], or -1.  Earlier entries are compared from a register (v_readlane), 64
-// at a time and the last first, so that the first match stays without a test
-// whether there is one: four instructions an entry, eight entries unrolled.
+// v[i], or -1.  Earlier entries are compared 64 at a time from a register
+// (v_readlane), not by a loop of dependent LDS reads per lane.
 __device__ __forceinline__ int first_earlier(const int* v, int n, int i0, int i) {
   const int lane = (int)(threadIdx.x & 63u);
-  const int w = v[i < n ? i : n - 1];
+  const int w = i < n ? v[i] : 0;
   int first_of = -1;
-  // of the entries beside lane i's own, those of the lanes before it
-  for (int k0 = n - i0 < 64 ? ((n - i0 - 1) & ~7) : 56; k0 >= 0; k0 -= 8) {
-#pragma unroll
-    for (int k = 7; k >= 0; --k) {
-      const bool hit = __builtin_amdgcn_readlane(w, k0 + k) == w && k0 + k < lane;
-      first_of = hit ? i0 + k0 + k : first_of;
-    }
-  }
-  for (int c0 = i0 - 64; c0 >= 0; c0 -= 64) {
-    const int cj = v[c0 + lane];
-    for (int k0 = 56; k0 >= 0; k0 -= 8) {
-#pragma unroll
-      for (int k = 7; k >= 0; --k)
-        first_of = __builtin_amdgcn_readlane(cj, k0 + k) == w ? c0 + k0 + k : first_of;
+  for (int c0 = 0; c0 <= i0; c0 += 64) {
+    const int cj = c0 + lane < n ? v[c0 + lane] : 0;
+    const int kn = n - c0 < 64 ? n - c0 : 64;
+    for (int k = 0; k < kn; ++k) {
+      const int vk = __builtin_amdgcn_readlane(cj, k);
+      if (first_of < 0 && c0 + k < i && vk == w) first_of = c0 + k;
     }
   }
   return i < n ? first_of : -1;
@@ -288,38 +254,25 @@ __device__ __forceinline__ int first_earlier(const int* v, int n, int i0, int i)
 
 // Two wavefronts per SIMD up to dim 128 (at most 256 registers): the LDS of
 // a wavefront (27 KB at dim 128 on 22-token walks) fits six per CU.
-// Bound by its chain of steps, 18 thousand cycles each at dim 128: about a
-// quarter at sentence and batch ends, half in the three products and their
-// LDS reads, the rest in the choice of outputs and contexts.  One epoch over
-// 65,536 vertices (14.4M words, dim 128): 51.8 ms, 85.3 when each row, branch
-// and atomic was waited for; a round of 2.24M walks over 2.2M vertices 183 ms
-// (301).
-// SIG: the sigmoid table is copied behind the wavefront's LDS.  Loads return
-// in order, so a table read from memory waits for the atomics and stores of
-// the step before (53.3 and 191 ms).
-// NX: output rows of a group of 16 lanes, output NX g + x in register x of
-// group g.  Up to eight rows (six negatives) take two: every lane holds
-// outputs, so an epilogue or a store takes half the instructions of four and
-// the product over the outputs two MFMA steps instead of four (the epoch
-// above 56.3 ms with two, 65.6 with four).
-template <int DIM, int NX, bool SIG>
+// Bound by its chain of steps, some 15 us each at dim 128: one epoch over
+// 65,536 vertices (14.4M words) takes 85.3 ms.  What a concurrent launch
+// leaves in the tables follows the pace of the workers against each other: a
+// constant wait added to every step, nothing else changed, moves them 2.5 to
+// 7 times as far as two runs lie apart.  Rewrites of the step that took 51.8
+// ms (rows loaded ahead, no wait after the stores and atomics, the products
+// and their LDS reads unrolled) moved them 2 to 3.6 times as far, each of
+// them its part, the loads ahead none: so the steps are as they were.
+template <int DIM>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(DIM <= 128 ? 2 : 1)))
 void dsgl_kernel(DsglArgs a) {
   extern __shared__ __attribute__((aligned(16))) char dsgl_smem[];
   constexpr int LDV = dsgl_ldv<DIM>();
   constexpr int NT = DIM / 16;  // dim tiles / k chunks
   constexpr int PER = DIM / 64; // dims per lane in row copies
-  constexpr int kRowBatch = row_batch<DIM>();
-  typedef typename RowPart<PER>::t Part;
   const int lane = threadIdx.x & 63;
+  const int l16 = lane & 15, g4 = lane >> 4;
   DsglLds L = dsgl_carve<DIM>(dsgl_smem, a.lcap, a.vcap, a.ncap, a.yrows, a.gl);
   for (int i = lane; i < LDV; i += 64) L.Z[i] = 0.0f;
-  const float* sig = a.expt;
-  if constexpr (SIG) {
-    float* copy = reinterpret_cast<float*>(dsgl_smem + dsgl_lds_bytes<DIM>(a.lcap, a.vcap, a.ncap, a.yrows, a.gl));
-    for (int i = lane; i <= kDsglExpTable; i += 64) copy[i] = a.expt[i];
-    sig = copy;
-  }
   const uint64_t gw = blockIdx.x;
   uint64_t nw = gridDim.x;
   if (a.deterministic) {
@@ -355,11 +308,6 @@ void dsgl_kernel(DsglArgs a) {
     int len[2] = {0, 0}, pos[2] = {0, 0}, nwords[2] = {0, 0};
     int tsn = 0, change_neg = 1, nbn = 0, nneg = 0;
     uint32_t neg_count = 0, step = 0, batch = 0;
-    int shrinks = 0;  // the window shrinks of 64 steps, one per lane
-    // the step's output rows, loaded a step ahead where that can be done
-    bool have = false;
-    int out_key = 0, out_meta = 0, nst = 0;
-    Part yv[8];
 
     while (true) {
       if (a.deterministic) __threadfence();
@@ -371,9 +319,6 @@ void dsgl_kernel(DsglArgs a) {
         if (al < a.alpha0 * 0.0001f) al = a.alpha0 * 0.0001f;
         alpha = al;
       }
-      // The step's output rows are already on their way (`have`) only where no
-      // sentence ended, so there is nothing to refill.
-      if (!have) {
       // ---- sentences (dsgl.hpp:899-1030)
       for (int s = 0; s < 2; ++s) {
         while (len[s] == 0) {
@@ -463,19 +408,23 @@ void dsgl_kernel(DsglArgs a) {
           nwords[s] = nwd;
           // live rows in LDS, snapshots in scratch (dsgl.hpp:942-945)
           for (int u0 = 0; u0 < nwd; u0 += kRowBatch) {
-            Part v[kRowBatch];
-            // past the last row the last one again: no branch per row
-            const int ids = L.word[s * vcap + (u0 + lane < nwd ? u0 + lane : nwd - 1)];
+            float v[kRowBatch][PER];
 #pragma unroll
             for (int i = 0; i < kRowBatch; ++i) {
-              const float* src = a.syn0 + (uint64_t)(uint32_t)__builtin_amdgcn_readlane(ids, i) * DIM;
-              v[i] = *reinterpret_cast<const Part*>(src + PER * lane);
+              if (u0 + i >= nwd) continue;
+              const float* src = a.syn0 + (uint64_t)L.word[s * vcap + u0 + i] * DIM;
+#pragma unroll
+              for (int j = 0; j < PER; ++j) v[i][j] = src[lane + 64 * j];
             }
 #pragma unroll
             for (int i = 0; i < kRowBatch; ++i) {
-              const int u = u0 + i < nwd ? u0 + i : nwd - 1;
-              *reinterpret_cast<Part*>(L.V + (s * vcap + u) * LDV + PER * lane) = v[i];
-              *reinterpret_cast<Part*>(snap + ((size_t)s * lcap + u) * DIM + PER * lane) = v[i];
+              const int u = u0 + i;
+              if (u >= nwd) continue;
+#pragma unroll
+              for (int j = 0; j < PER; ++j) {
+                L.V[(s * vcap + u) * LDV + lane + 64 * j] = v[i][j];
+                snap[((size_t)s * lcap + u) * DIM + lane + 64 * j] = v[i][j];
+              }
             }
           }
           wave_sync();
@@ -519,96 +468,84 @@ void dsgl_kernel(DsglArgs a) {
           wave_sync();
         }
         nneg = nd_first;
-        // beside its row, each draw's multiplicity among its step's draws, and
-        // whether it is the first of them
-        for (int i0 = 0; i0 < nd; i0 += 64) {
-          const int i = i0 + lane;
-          if (i < nd) {
-            const int at = i - i % K, w = L.nword[i];
-            int mt = 0;
-            bool first = true;
-            for (int j = 0; j < K; ++j) {
-              const bool same = L.nword[at + j] == w;
-              mt += same ? 1 : 0;
-              if (same && at + j < i) first = false;
-            }
-            L.nslot[i] |= mt << 16 | (first ? 1 << 24 : 0);
-          }
-        }
-        nst = (int)(neg_count % (uint32_t)nbn);
-        wave_sync();
         for (int k0 = 0; k0 < nneg; k0 += kRowBatch) {
-          Part v[kRowBatch];
-          const int ids = L.nid[k0 + lane < nneg ? k0 + lane : nneg - 1];
+          float v[kRowBatch][PER];
 #pragma unroll
           for (int i = 0; i < kRowBatch; ++i) {
-            const float* src = a.syn1 + (uint64_t)(uint32_t)__builtin_amdgcn_readlane(ids, i) * DIM;
-            v[i] = *reinterpret_cast<const Part*>(src + PER * lane);
+            if (k0 + i >= nneg) continue;
+            const float* src = a.syn1 + (uint64_t)L.nid[k0 + i] * DIM;
+#pragma unroll
+            for (int j = 0; j < PER; ++j) v[i][j] = src[lane + 64 * j];
           }
 #pragma unroll
           for (int i = 0; i < kRowBatch; ++i) {
-            const size_t k = (size_t)(k0 + i < nneg ? k0 + i : nneg - 1);
-            *reinterpret_cast<Part*>(nsnap + k * DIM + PER * lane) = v[i];
-            *reinterpret_cast<Part*>(nlive + k * DIM + PER * lane) = v[i];
+            const size_t k = (size_t)(k0 + i);
+            if (k0 + i >= nneg) continue;
+#pragma unroll
+            for (int j = 0; j < PER; ++j) {
+              nsnap[k * DIM + lane + 64 * j] = v[i][j];
+              nlive[k * DIM + lane + 64 * j] = v[i][j];
+            }
           }
         }
+        drain();
         ++batch;
         change_neg = 0;
       }
-      }
       // ---- one step: both positions (dsgl.hpp:1085-1356)
-      // outputs: [target, the K negatives with multiplicity, target2].  Lane i
-      // of `key` holds output i: a target's vocabulary index, or a negative's
-      // row in the batch buffer with the top bit set, and the next one too if
-      // it takes no part (a repeat of another draw, or the target): its row
-      // of Y is zero then.
-      auto outputs = [&](int p0, int p1, int& key, int& meta) {
-        ++neg_count;
-        nst = nst + 1 == nbn ? 0 : nst + 1;
-        const bool neg = lane > 0 && lane <= K;
-        const int at = neg ? nst * K + lane - 1 : 0;
-        const int word = L.nword[at], info = L.nslot[at];
-        const int tg = uni(L.sen[p0]), tg2 = uni(L.sen[lcap + p1]);
-        const bool live = neg && (info >> 24) != 0 && word != tg;
-        key = lane == 0 ? tg : (lane == K + 1 ? tg2 : (int)((live ? 0x80000000u : 0xC0000000u) | (uint32_t)(info & 0xffff)));
-        meta = neg ? (info >> 16) & 0xff : 1;
-      };
-      auto dead = [](int key) { return ((uint32_t)key & 0xC0000000u) == 0xC0000000u; };
-      // an output's row: the targets' in syn1, the negatives' in the batch buffer
-      auto row_of = [&](int key) -> float* {
-        return key < 0 ? nlive + (size_t)(uint32_t)(key & 0x3fffffff) * DIM : a.syn1 + (uint64_t)(uint32_t)key * DIM;
-      };
-      // eight rows, from the level-2 cache (the rows this wavefront's stores
-      // and atomics moved); past the last the last one again, not used
-      auto load_rows = [&](int key, int r0, Part (&y)[8]) {
-#pragma unroll
-        for (int r = 0; r < 8; ++r) {
-          const int i = r0 + r <= K + 1 ? r0 + r : K + 1;
-          y[r] = row_load_l2(row_of(__builtin_amdgcn_readlane(key, i)) + PER * lane, Part(0.0f));
+      const int target = uni(L.sen[pos[0]]);
+      const int target2 = uni(L.sen[lcap + pos[1]]);
+      // outputs: [target, distinct negatives with multiplicity, target2]
+      ++neg_count;
+      const int nst = (int)(neg_count % (uint32_t)nbn);
+      int smp = -1, meta = 0, sl = 0;
+      bool nfirst = false;
+      if (lane < K) {
+        smp = L.nword[nst * K + lane];
+        sl = L.nslot[nst * K + lane];
+        nfirst = smp != target;
+        for (int k = 0; k < K; ++k) {
+          const int o = L.nword[nst * K + k];
+          if (o == smp) {
+            ++meta;
+            if (k < lane) nfirst = false;
+          }
         }
-      };
-      auto stage_rows = [&](int key, int r0, const Part (&y)[8]) {
-#pragma unroll
-        for (int r = 0; r < 8; ++r)
-          if (r0 + r < yr)
-            *reinterpret_cast<Part*>(L.Y + (r0 + r) * LDV + PER * lane) =
-                dead(__builtin_amdgcn_readlane(key, r0 + r)) ? Part(0.0f) : y[r];
-      };
-      if (!have) {
-        outputs(pos[0], pos[1], out_key, out_meta);
-        load_rows(out_key, 0, yv);  // in flight while the contexts are found
       }
-      have = false;
-      if ((step & 63u) == 0)
-        shrinks = (int)(draw_word(a.key, (uint32_t)t, step + (uint32_t)lane, DG_TAG_DSGL_WIN, 0) % (uint32_t)W);
-      const int b = __builtin_amdgcn_readlane(shrinks, step & 63u);
+      const uint64_t om = __ballot(nfirst);
+      const int O = 2 + __popcll(om);
+      if (nfirst) {
+        const int o = 1 + (int)lanes_below(om);
+        L.out_id[o] = smp;
+        L.out_meta[o] = meta;
+        L.out_slot[o] = sl;
+      }
+      if (lane == 0) {
+        L.out_id[0] = target;
+        L.out_meta[0] = 1;
+        L.out_id[O - 1] = target2;
+        L.out_meta[O - 1] = 1;
+      }
+      wave_sync();
+      // output rows: the targets from syn1, the negatives from the batch
+      // buffer, from the level-2 cache (the rows this wavefront's atomics
+      // moved); the first eight rows' loads are in flight while the contexts
+      // are found
+      float yv[8][PER];
+#pragma unroll
+      for (int r = 0; r < 8; ++r) {
+#pragma unroll
+        for (int j = 0; j < PER; ++j) yv[r][j] = 0.0f;
+        if (r < O) {
+          const bool tab = (r == 0 || r == O - 1);
+          const float* src = tab ? a.syn1 + (uint64_t)L.out_id[r] * DIM
+                                 : nlive + (size_t)L.out_slot[r] * DIM;
+#pragma unroll
+          for (int j = 0; j < PER; ++j) yv[r][j] = load_l2(src + lane + 64 * j);
+        }
+      }
+      const int b = (int)(draw_word(a.key, (uint32_t)t, step, DG_TAG_DSGL_WIN, 0) % (uint32_t)W);
       ++step;
-      // The step's LDS addresses are formed from a lane index that the compiler
-      // cannot hoist: held for the whole launch they left no registers for
-      // the rows in flight at a sentence's or a batch's ends.
-      int lane_now = lane;
-      asm volatile("" : "+v"(lane_now));
-      const int l16 = lane_now & 15, g4 = lane_now >> 4;
       // contexts: lanes 0..31 the first window, 32..63 the second
       const int hs = lane >> 5, li = lane & 31;
       const int span = 2 * (W - b);
@@ -616,25 +553,16 @@ void dsgl_kernel(DsglArgs a) {
       {
         const int i = b + li + (b + li >= W ? 1 : 0);
         const int c = pos[hs] - W + i;
-        const int len_h = hs ? len[1] : len[0];
-        const bool in = li < span && c >= 0 && c < len_h;
-        const int at = L.slot[hs * lcap + (in ? c : 0)];
-        if (in) my = at;
+        if (li < span && c >= 0 && c < len[hs]) my = L.slot[hs * lcap + c];
       }
       L.tmp[lane] = my;
       wave_sync();
       bool first = my >= 0;
       int cnt = 0;
-      int4 o4 = *reinterpret_cast<const int4*>(L.tmp + hs * 32);
-      for (int j0 = 0; j0 < span; j0 += 4) {  // entries past the window are -1
-        const int4 now = o4;
-        o4 = *reinterpret_cast<const int4*>(L.tmp + hs * 32 + ((j0 + 4) & 31));
-        const int o[4] = {now.x, now.y, now.z, now.w};
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          cnt += o[j] == my ? 1 : 0;
-          if (j0 + j < li && o[j] == my) first = false;
-        }
+      for (int j = 0; j < 32; ++j) {
+        const int o = L.tmp[hs * 32 + j];
+        cnt += (my >= 0 && o == my) ? 1 : 0;
+        if (j < li && o == my) first = false;
       }
       const uint64_t em = __ballot(first);
       const int E = __popcll(em);
@@ -644,12 +572,31 @@ void dsgl_kernel(DsglArgs a) {
         L.ent_row[e] = hs * (int)vcap + my;
         L.ent_cnt[e] = (uint8_t)cnt;
       }
-      stage_rows(out_key, 0, yv);
-      if constexpr (NX == 4) {
+#pragma unroll
+      for (int r = 0; r < 8; ++r)
+        if (r < yr)  // rows O .. yr - 1 zero
+#pragma unroll
+          for (int j = 0; j < PER; ++j) L.Y[r * LDV + lane + 64 * j] = yv[r][j];
+      if (yr > 8) {
         // more than six negatives: rows 8 .. 15
-        Part yw[8];
-        load_rows(out_key, 8, yw);
-        stage_rows(out_key, 8, yw);
+        float yw[8][PER];
+#pragma unroll
+        for (int r = 0; r < 8; ++r) {
+#pragma unroll
+          for (int j = 0; j < PER; ++j) yw[r][j] = 0.0f;
+          if (8 + r < O) {
+            const bool tab = 8 + r == O - 1;
+            const float* src = tab ? a.syn1 + (uint64_t)L.out_id[8 + r] * DIM
+                                   : nlive + (size_t)L.out_slot[8 + r] * DIM;
+#pragma unroll
+            for (int j = 0; j < PER; ++j) yw[r][j] = load_l2(src + lane + 64 * j);
+          }
+        }
+#pragma unroll
+        for (int r = 0; r < 8; ++r)
+          if (8 + r < yr)
+#pragma unroll
+            for (int j = 0; j < PER; ++j) L.Y[(8 + r) * LDV + lane + 64 * j] = yw[r][j];
       }
       wave_sync();
       // LDS offsets (from V) of the context rows: xg[et] the row lane l16
@@ -664,123 +611,67 @@ void dsgl_kernel(DsglArgs a) {
 #pragma unroll
       for (int et = 0; et < kET; ++et) {
         const int e = 16 * et + l16;
-        const int at = L.ent_row[e] * LDV;  // read past E too: no branch around a read
-        xg[et] = e < E ? at : zoff;
+        xg[et] = e < E ? L.ent_row[e] * LDV : zoff;
 #pragma unroll
         for (int x = 0; x < 4; ++x) {
           const int e4 = 16 * et + 4 * g4 + x;
-          const int at4 = L.ent_row[e4] * LDV;
-          xo[et][x] = e4 < E ? at4 : zoff;
+          xo[et][x] = e4 < E ? L.ent_row[e4] * LDV : zoff;
         }
       }
-      // this lane's outputs
-      int ky[NX];
-      float om[NX];
-#pragma unroll
-      for (int x = 0; x < NX; ++x) {
-        ky[x] = __shfl(out_key, NX * g4 + x, 64);
-        om[x] = (float)__shfl(out_meta, NX * g4 + x, 64);
-      }
-      // ---- the next step's output rows, where neither sentence ends (so the
-      // batch stays) and none of them is moved by this step: their loads are
-      // in flight during this step's products.  A sigmoid table in memory
-      // would wait for them, so they go out behind its reads then.
-      auto ahead = [&]() {
-        if (pos[0] + 1 >= len[0] || pos[1] + 1 >= len[1]) return;
-        const int key_now = out_key, nst_now = nst;
-        outputs(pos[0] + 1, pos[1] + 1, out_key, out_meta);
-        bool moved = false;
-#pragma unroll
-        for (int r = 0; r < 8; ++r)
-          moved |= out_key == __builtin_amdgcn_readlane(key_now, r < K + 1 ? r : K + 1);
-        if (__ballot(moved && lane <= K + 1 && !dead(out_key)) == 0) {
-          load_rows(out_key, 0, yv);
-          have = true;
-        } else {
-          --neg_count;  // drawn again by that step
-          nst = nst_now;
-        }
-      };
-      if constexpr (NX == 2 && SIG) ahead();
-      // the row of the outputs that lane l16 supplies to a product
-      const int arow = NX == 4 ? l16 : (l16 & 3) < 2 ? 2 * (l16 >> 2) + (l16 & 3) : yr;
-      // The two products over the contexts, for a number of their tiles that
-      // is known when they are compiled: reads in flight and no branch in
-      // between.
-      auto over_tiles = [&](auto&& body) {
-        if (ET == 1) body(std::integral_constant<int, 1>{});
-        else if (ET == 2) body(std::integral_constant<int, 2>{});
-        else body(std::integral_constant<int, kET>{});
-      };
       // G = Y X^T and g (dsgl.hpp:1241-1273)
-      over_tiles([&](auto tiles) {
-        constexpr int T = decltype(tiles)::value;
-        f32x4_t acc[T];
+      {
+        f32x4_t acc[kET];
 #pragma unroll
-        for (int et = 0; et < T; ++et) acc[et] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-        const float* yrow = arow < yr ? L.Y + arow * LDV : L.Z;
+        for (int et = 0; et < kET; ++et) acc[et] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        const float* yrow = l16 < yr ? L.Y + l16 * LDV : L.Z;
 #pragma unroll
         for (int kc = 0; kc < NT; ++kc) {
           const float4 ya = *reinterpret_cast<const float4*>(yrow + 16 * kc + 4 * g4);
 #pragma unroll
-          for (int et = 0; et < T; ++et) {
+          for (int et = 0; et < kET; ++et) {
+            if (et >= ET) break;
             const float4 xb = *reinterpret_cast<const float4*>(L.V + xg[et] + 16 * kc + 4 * g4);
             acc[et] = mma4(ya, xb, acc[et]);
           }
         }
 #pragma unroll
-        for (int et = 0; et < T; ++et) {
+        for (int et = 0; et < kET; ++et) {
+          if (et >= ET) break;
           const int e = 16 * et + l16;
-          const float ec = (float)L.ent_cnt[e];
-          const bool s1 = e < E1;
-          float sg[NX];
-          if (a.exact) {
 #pragma unroll
-            for (int x = 0; x < NX; ++x) sg[x] = dsgl_sig(acc[et][x], sig, 1);
-          } else {
-#pragma unroll
-            for (int x = 0; x < NX; ++x) sg[x] = dsgl_sig(acc[et][x], sig, 0);
-          }
-#pragma unroll
-          for (int x = 0; x < NX; ++x) {
-            const int i = NX * g4 + x;
-            const float label = ((i == 0 && s1) || (i == K + 1 && !s1)) ? 1.0f : 0.0f;
-            const float g = (label - sg[x]) * alpha * om[x] * ec;
-            if (i < yr) L.G[i * gl + e] = e < E && !dead(ky[x]) ? g : 0.0f;
+          for (int x = 0; x < 4; ++x) {
+            const int i = 4 * g4 + x;
+            float g = 0.0f;
+            if (i < O && e < E) {
+              const bool s1 = e < E1;
+              const float label = ((i == 0 && s1) || (i == O - 1 && !s1)) ? 1.0f : 0.0f;
+              g = (label - dsgl_sig(acc[et][x], a.expt, a.exact)) * alpha * (float)L.out_meta[i] *
+                  (float)L.ent_cnt[e];
+            }
+            if (i < yr) L.G[i * gl + e] = g;
           }
         }
-      });
-      wave_sync();
-      if constexpr (NX == 2 && !SIG) ahead();
-      // this lane's rows of G and Y, rows past yr read from the zero row
-      const float* yk[NX];
-      const float* gk[NX];
-      float* dst[NX];
-#pragma unroll
-      for (int x = 0; x < NX; ++x) {
-        const int i = NX * g4 + x;
-        yk[x] = i < yr ? L.Y + i * LDV : L.Z;
-        gk[x] = i < yr ? L.G + i * gl : L.Z;
-        dst[x] = row_of(ky[x]) + l16;
       }
-      float yb[NT][NX];
+      wave_sync();
+      // dY = G X: lane holds dY[4 g4 + x][16 tt + l16], added to the row of
+      // output 4 g4 + x (the targets in syn1, the negatives in the batch buffer)
+      {
+        float* dst[4];
 #pragma unroll
-      for (int tt = 0; tt < NT; ++tt)
-#pragma unroll
-        for (int x = 0; x < NX; ++x) yb[tt][x] = yk[x][16 * tt + l16];
-      // dY = G X: lane holds dY[NX g4 + x][16 tt + l16], added to the row of
-      // output NX g4 + x: the targets' rows in syn1 by atomics, the negatives'
-      // in the batch buffer, which is this wavefront's own, by a store of the
-      // staged row and its update (the memory adds some 20 G requests of 64
-      // bytes per second, and these were 5 of a step's 7 rows)
-      over_tiles([&](auto tiles) {
-        constexpr int T = decltype(tiles)::value;
+        for (int x = 0; x < 4; ++x) {
+          const int i = 4 * g4 + x;
+          dst[x] = i >= O ? nullptr
+                          : (i == 0 ? a.syn1 + (uint64_t)target * DIM
+                                    : (i == O - 1 ? a.syn1 + (uint64_t)target2 * DIM
+                                                  : nlive + (size_t)L.out_slot[i] * DIM));
+        }
         f32x4_t acc[NT];
 #pragma unroll
         for (int tt = 0; tt < NT; ++tt) acc[tt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-        const float* grow = arow < yr ? L.G + arow * gl : L.Z;
+        const float* grow = l16 < yr ? L.G + l16 * gl : L.Z;
 #pragma unroll
-        for (int ec = 0; ec < T; ++ec) {
+        for (int ec = 0; ec < kET; ++ec) {
+          if (ec >= ET) break;
           const float4 ga = *reinterpret_cast<const float4*>(grow + 16 * ec + 4 * g4);
 #pragma unroll
           for (int tt = 0; tt < NT; ++tt) {
@@ -791,77 +682,61 @@ void dsgl_kernel(DsglArgs a) {
           }
         }
 #pragma unroll
-        for (int x = 0; x < NX; ++x) {
-          const int i = NX * g4 + x;
-          if (i > 0 && i <= K && !dead(ky[x])) {
+        for (int tt = 0; tt < NT; ++tt)
 #pragma unroll
-            for (int tt = 0; tt < NT; ++tt) dst[x][16 * tt] = yb[tt][x] + acc[tt][x];
-          } else if (i == 0 || i == K + 1) {
-#pragma unroll
-            for (int tt = 0; tt < NT; ++tt) atomicAdd(dst[x] + 16 * tt, acc[tt][x]);
-          }
-        }
-      });
+          for (int x = 0; x < 4; ++x)
+            if (dst[x]) atomicAdd(dst[x] + 16 * tt + l16, acc[tt][x]);
+      }
       // dX = G^T Y into the sentence buffers: lane holds dX[16 et + 4 g4 + x][16 tt + l16]
       {
+        // this lane's k rows 4 g4 .. 4 g4 + 3, rows past yr read from the zero row
+        const float* yk[4];
+        const float* gk[4];
+#pragma unroll
+        for (int x = 0; x < 4; ++x) {
+          const int i = 4 * g4 + x;
+          yk[x] = i < yr ? L.Y + i * LDV : L.Z;
+          gk[x] = i < yr ? L.G + i * gl : L.Z;
+        }
+        float4 yb[NT];
+#pragma unroll
+        for (int tt = 0; tt < NT; ++tt)
+          yb[tt] = make_float4(yk[0][16 * tt + l16], yk[1][16 * tt + l16], yk[2][16 * tt + l16], yk[3][16 * tt + l16]);
 #pragma unroll
         for (int et = 0; et < kET; ++et) {
           if (et >= ET) break;
-          f32x4_t acc[NT], xv[NT];
-          float ga[NX];
+          const float4 a4 = make_float4(gk[0][16 * et + l16], gk[1][16 * et + l16], gk[2][16 * et + l16],
+                                        gk[3][16 * et + l16]);
+          f32x4_t acc[NT];
 #pragma unroll
-          for (int x = 0; x < NX; ++x) ga[x] = gk[x][16 * et + l16];
-#pragma unroll
-          for (int tt = 0; tt < NT; ++tt) {
-            acc[tt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int x = 0; x < NX; ++x)
-              acc[tt] = __builtin_amdgcn_mfma_f32_16x16x4f32(ga[x], yb[tt][x], acc[tt], 0, 0, 0);
-          }
-          // all reads, then all writes: a branch around each row's would make
-          // every one of them a round trip.  Rows past E are the zero row,
-          // which gets zeros.
-#pragma unroll
-          for (int x = 0; x < 4; ++x) {
-            const bool in = 16 * et + 4 * g4 + x < E;
-#pragma unroll
-            for (int tt = 0; tt < NT; ++tt) {
-              xv[tt][x] = L.V[xo[et][x] + 16 * tt + l16];
-              acc[tt][x] = in ? acc[tt][x] : 0.0f;
-            }
-          }
+          for (int tt = 0; tt < NT; ++tt) acc[tt] = mma4(a4, yb[tt], f32x4_t{0.f, 0.f, 0.f, 0.f});
           wave_sync();
 #pragma unroll
-          for (int x = 0; x < 4; ++x)
+          for (int tt = 0; tt < NT; ++tt)
 #pragma unroll
-            for (int tt = 0; tt < NT; ++tt) L.V[xo[et][x] + 16 * tt + l16] = xv[tt][x] + acc[tt][x];
+            for (int x = 0; x < 4; ++x)
+              if (16 * et + 4 * g4 + x < E) L.V[xo[et][x] + 16 * tt + l16] += acc[tt][x];
         }
       }
+      drain();
       wave_sync();
       // ---- finished sentences and batch back to the tables (dsgl.hpp:1358-1404)
-      if (have) {
-        ++pos[0];
-        ++pos[1];
-        wave_sync();
-        continue;
-      }
       for (int s = 0; s < 2; ++s) {
         if (++pos[s] < len[s]) continue;
         for (int u0 = 0; u0 < nwords[s]; u0 += kRowBatch) {
           float sv[kRowBatch][PER];
-          const int ids = L.word[s * vcap + (u0 + lane < nwords[s] ? u0 + lane : nwords[s] - 1)];
 #pragma unroll
           for (int i = 0; i < kRowBatch; ++i) {
-            const int u = u0 + i < nwords[s] ? u0 + i : nwords[s] - 1;
+            if (u0 + i >= nwords[s]) continue;
 #pragma unroll
             for (int j = 0; j < PER; ++j)
-              sv[i][j] = load_l2(snap + ((size_t)s * lcap + u) * DIM + lane + 64 * j);
+              sv[i][j] = load_l2(snap + ((size_t)s * lcap + u0 + i) * DIM + lane + 64 * j);
           }
 #pragma unroll
           for (int i = 0; i < kRowBatch; ++i) {
             const int u = u0 + i;
             if (u >= nwords[s]) continue;
-            float* dst = a.syn0 + (uint64_t)(uint32_t)__builtin_amdgcn_readlane(ids, i) * DIM;
+            float* dst = a.syn0 + (uint64_t)L.word[s * vcap + u] * DIM;
 #pragma unroll
             for (int j = 0; j < PER; ++j) {
               const int d = lane + 64 * j;
@@ -875,10 +750,10 @@ void dsgl_kernel(DsglArgs a) {
       if (tsn >= 2) {
         for (int k0 = 0; k0 < nneg; k0 += kRowBatch) {
           float lv[kRowBatch][PER], sv[kRowBatch][PER];
-          const int ids = L.nid[k0 + lane < nneg ? k0 + lane : nneg - 1];
 #pragma unroll
           for (int i = 0; i < kRowBatch; ++i) {
-            const size_t k = (size_t)(k0 + i < nneg ? k0 + i : nneg - 1);
+            if (k0 + i >= nneg) continue;
+            const size_t k = (size_t)(k0 + i);
 #pragma unroll
             for (int j = 0; j < PER; ++j) {
               lv[i][j] = load_l2(nlive + k * DIM + lane + 64 * j);
@@ -888,7 +763,7 @@ void dsgl_kernel(DsglArgs a) {
 #pragma unroll
           for (int i = 0; i < kRowBatch; ++i) {
             if (k0 + i >= nneg) continue;
-            float* dst = a.syn1 + (uint64_t)(uint32_t)__builtin_amdgcn_readlane(ids, i) * DIM;
+            float* dst = a.syn1 + (uint64_t)L.nid[k0 + i] * DIM;
 #pragma unroll
             for (int j = 0; j < PER; ++j) atomicAdd(dst + lane + 64 * j, lv[i][j] - sv[i][j]);
           }
@@ -952,9 +827,9 @@ __global__ void dsgl_state_init_kernel(unsigned long long* actual, float* alpha,
   if (blockIdx.x == 0 && threadIdx.x == 0) *kept = 0ull;
 }
 
-template <int DIM, int NX, bool SIG>
-int launch_unit(dg_ctx* ctx, const DsglArgs& a, size_t lds, unsigned grid) {
-  auto k = dsgl_kernel<DIM, NX, SIG>;
+template <int DIM>
+int launch_dims(dg_ctx* ctx, const DsglArgs& a, size_t lds, unsigned grid) {
+  auto k = dsgl_kernel<DIM>;
   hipError_t e = hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   if (e != hipSuccess) return dg_fail(ctx, DG_ERR_HIP, "DSGL kernel LDS attribute: %s", hipGetErrorString(e));
   k<<<grid, 64, lds, ctx->stream>>>(a);
@@ -964,41 +839,19 @@ int launch_unit(dg_ctx* ctx, const DsglArgs& a, size_t lds, unsigned grid) {
 }
 
 template <int DIM>
-int launch_dims(dg_ctx* ctx, const DsglArgs& a, bool sig, size_t lds, unsigned grid) {
-  if (a.yrows <= 8)
-    return sig ? launch_unit<DIM, 2, true>(ctx, a, lds, grid) : launch_unit<DIM, 2, false>(ctx, a, lds, grid);
-  return sig ? launch_unit<DIM, 4, true>(ctx, a, lds, grid) : launch_unit<DIM, 4, false>(ctx, a, lds, grid);
-}
-
-constexpr size_t kSigBytes = ((kDsglExpTable + 1) * sizeof(float) + 15) & ~(size_t)15;
-
-// Workgroups (wavefronts) of a kernel that fit a CU.
-template <int DIM, int NX, bool SIG>
-int resident_unit(dg_ctx* ctx, size_t lds, unsigned* per_cu) {
-  int n = 0;
-  hipError_t e = hipFuncSetAttribute((const void*)dsgl_kernel<DIM, NX, SIG>,
-                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-  if (e == hipSuccess) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, dsgl_kernel<DIM, NX, SIG>, 64, lds);
-  if (e != hipSuccess) return dg_fail(ctx, DG_ERR_HIP, "DSGL occupancy: %s", hipGetErrorString(e));
-  *per_cu = n < 1 ? 1u : (unsigned)n;
-  return DG_OK;
-}
-
-template <int DIM>
 int plan_dims(dg_ctx* ctx, uint32_t lcap, uint32_t vcap, uint32_t ncap, uint32_t yrows, uint32_t gl,
-              size_t* lds, unsigned* per_cu, unsigned* per_cu_sig) {
-  const size_t used = dsgl_lds_bytes<DIM>(lcap, vcap, ncap, yrows, gl);
-  *lds = used + kPlanBytes;
+              size_t* lds, unsigned* per_cu) {
+  *lds = dsgl_lds_bytes<DIM>(lcap, vcap, ncap, yrows, gl);
   if (*lds > 160 * 1024)
     return dg_fail(ctx, DG_ERR_UNSUPPORTED,
                    "DSGL form: sentences of %u tokens at dim %d need %zu bytes of LDS per wavefront "
                    "(160 KB available)", lcap, DIM, *lds);
-  const bool few = yrows <= 8;
-  DG_CHECK((few ? resident_unit<DIM, 2, false>(ctx, *lds, per_cu) : resident_unit<DIM, 4, false>(ctx, *lds, per_cu)));
-  *per_cu_sig = 0;
-  const size_t more = used + kSigBytes;
-  if (more <= 160 * 1024)
-    DG_CHECK((few ? resident_unit<DIM, 2, true>(ctx, more, per_cu_sig) : resident_unit<DIM, 4, true>(ctx, more, per_cu_sig)));
+  int n = 0;
+  hipError_t e = hipFuncSetAttribute((const void*)dsgl_kernel<DIM>,
+                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)*lds);
+  if (e == hipSuccess) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, dsgl_kernel<DIM>, 64, *lds);
+  if (e != hipSuccess) return dg_fail(ctx, DG_ERR_HIP, "DSGL occupancy: %s", hipGetErrorString(e));
+  *per_cu = n < 1 ? 1u : (unsigned)n;
   return DG_OK;
 }
 
@@ -1056,11 +909,11 @@ int dg_dsgl_train(dg_ctx* ctx, const dg_dsgl_call& c, uint64_t* kept, double* ms
   const uint32_t vcap = std::max<uint32_t>(1u, std::min<uint32_t>(lcap, most));
   const uint32_t yrows = c.K + 2, gl = dsgl_gl(c.window);
   size_t lds = 0;
-  unsigned per_cu = 1, per_cu_sig = 0;
+  unsigned per_cu = 1;
   switch (c.dim) {
-    case 64: DG_CHECK(plan_dims<64>(ctx, lcap, vcap, ncap, yrows, gl, &lds, &per_cu, &per_cu_sig)); break;
-    case 128: DG_CHECK(plan_dims<128>(ctx, lcap, vcap, ncap, yrows, gl, &lds, &per_cu, &per_cu_sig)); break;
-    default: DG_CHECK(plan_dims<256>(ctx, lcap, vcap, ncap, yrows, gl, &lds, &per_cu, &per_cu_sig)); break;
+    case 64: DG_CHECK(plan_dims<64>(ctx, lcap, vcap, ncap, yrows, gl, &lds, &per_cu)); break;
+    case 128: DG_CHECK(plan_dims<128>(ctx, lcap, vcap, ncap, yrows, gl, &lds, &per_cu)); break;
+    default: DG_CHECK(plan_dims<256>(ctx, lcap, vcap, ncap, yrows, gl, &lds, &per_cu)); break;
   }
   const uint64_t resident = (uint64_t)per_cu * (uint64_t)ctx->num_cus;
   // default: one worker per resident wavefront, at most five per CU.  Every
@@ -1071,10 +924,6 @@ int dg_dsgl_train(dg_ctx* ctx, const dg_dsgl_call& c, uint64_t* kept, double* ms
   uint32_t workers = c.workers ? c.workers : (uint32_t)dflt;
   if ((uint64_t)workers > c.n_walks + c.n_tok) workers = (uint32_t)std::max<uint64_t>(1, (c.n_walks + c.n_tok) / 64);
   const unsigned grid = c.deterministic ? 1u : (unsigned)std::min<uint64_t>(workers, resident);
-  // the sigmoid table goes to LDS where that leaves as many wavefronts resident:
-  // it saves 3 to 4% of a launch, a wavefront less per CU costs a fifth
-  const bool sig = (uint64_t)per_cu_sig * (uint64_t)ctx->num_cus >= grid;
-  lds += sig ? kSigBytes - kPlanBytes : 0;
   const uint64_t stride = ((uint64_t)2 * lcap + 2 * (uint64_t)ncap) * c.dim;
   DG_CHECK(dg_reserve(ctx, &st->scratch, &st->scratch_cap, (size_t)(grid * stride)));
   DG_CHECK(dg_reserve(ctx, &st->actual, &st->actual_cap, (size_t)workers));
@@ -1120,9 +969,9 @@ int dg_dsgl_train(dg_ctx* ctx, const dg_dsgl_call& c, uint64_t* kept, double* ms
     a.key = dg_epoch_key(c.seed, c.epoch0 + ep);
     DG_CHECK(dg_time_begin(ctx, "sgns_dsgl", &tk));
     switch (c.dim) {
-      case 64: DG_CHECK(launch_dims<64>(ctx, a, sig, lds, grid)); break;
-      case 128: DG_CHECK(launch_dims<128>(ctx, a, sig, lds, grid)); break;
-      default: DG_CHECK(launch_dims<256>(ctx, a, sig, lds, grid)); break;
+      case 64: DG_CHECK(launch_dims<64>(ctx, a, lds, grid)); break;
+      case 128: DG_CHECK(launch_dims<128>(ctx, a, lds, grid)); break;
+      default: DG_CHECK(launch_dims<256>(ctx, a, lds, grid)); break;
     }
     DG_CHECK(dg_time_end(ctx, tk));
   }
