@@ -304,8 +304,10 @@ int dg_dsgl_train(dg_ctx* ctx, const dg_dsgl_call& c, uint64_t* kept, double* ms
 void dg_dsgl_free(dg_ctx* ctx);
 
 // Copies device memory to the caller's pageable buffer, after the context's
-// queued work, and returns when the bytes are there (hostcopy.hip).
-int dg_copy_to_host(dg_ctx* ctx, void* dst, const void* src, size_t bytes);
+// queued work, and returns when the bytes are there (hostcopy.hip).  Where that
+// work has set the host-visible word `refused`, the buffer stays as it is (and
+// DG_OK is returned: the caller looks at the word).
+int dg_copy_to_host(dg_ctx* ctx, void* dst, const void* src, size_t bytes, const uint32_t* refused = nullptr);
 void dg_hostcopy_open();   // a context opened / closed: the last one gives the
 void dg_hostcopy_close();  // staging memory and threads back
 

@@ -51,15 +51,19 @@ CopyRing* ring_locked() {
   return g_ring;
 }
 
+bool is_set(const uint32_t* word) { return word && __atomic_load_n(word, __ATOMIC_ACQUIRE) != 0u; }
+
 // The stream's transfers into the ring, an event for each slot.
 struct StreamEngine {
   hipStream_t stream;
   const CopyRing& ring;
   const char* src;
+  const uint32_t* refused;
   hipError_t err = hipSuccess;
   hipEvent_t ev[CopyRing::kChunks] = {};
 
-  StreamEngine(hipStream_t s, const CopyRing& r, const char* from) : stream(s), ring(r), src(from) {
+  StreamEngine(hipStream_t s, const CopyRing& r, const char* from, const uint32_t* no)
+      : stream(s), ring(r), src(from), refused(no) {
     for (auto& x : ev)
       if (err == hipSuccess) err = hipEventCreateWithFlags(&x, hipEventDisableTiming);
   }
@@ -73,7 +77,7 @@ struct StreamEngine {
     return err == hipSuccess;
   }
   bool wait(size_t slot) { return (err = hipEventSynchronize(ev[slot])) == hipSuccess; }
-  bool go() const { return true; }
+  bool go() const { return !is_set(refused); }
   void drain() { (void)hipStreamSynchronize(stream); }
 };
 
@@ -90,20 +94,24 @@ void dg_hostcopy_close() {
   g_failed = false;
 }
 
-int dg_copy_to_host(dg_ctx* ctx, void* dst, const void* src, size_t bytes) {
+int dg_copy_to_host(dg_ctx* ctx, void* dst, const void* src, size_t bytes, const uint32_t* refused) {
   if (bytes >= kMinBytes) {
     std::unique_lock<std::mutex> lk(g_mu, std::try_to_lock);
     if (CopyRing* r = lk.owns_lock() ? ring_locked() : nullptr) {
       if (bytes > CopyRing::kChunk) {
-        StreamEngine e(ctx->stream, *r, static_cast<const char*>(src));
-        if (e.err == hipSuccess && r->copy(static_cast<char*>(dst), bytes, e) == CopyEnd::kDone) return DG_OK;
+        StreamEngine e(ctx->stream, *r, static_cast<const char*>(src), refused);
+        if (e.err == hipSuccess && r->copy(static_cast<char*>(dst), bytes, e) != CopyEnd::kFailed) return DG_OK;
         return dg_fail(ctx, DG_ERR_HIP, "copy to the host: %s", hipGetErrorString(e.err));
       }
       DG_HIP(ctx, hipMemcpyAsync(r->pinned(0), src, bytes, hipMemcpyDeviceToHost, ctx->stream));
       DG_HIP(ctx, hipStreamSynchronize(ctx->stream));
-      memcpy(dst, r->pinned(0), bytes);
+      if (!is_set(refused)) memcpy(dst, r->pinned(0), bytes);
       return DG_OK;
     }
+  }
+  if (refused) {
+    DG_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    if (is_set(refused)) return DG_OK;
   }
   DG_HIP(ctx, hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, ctx->stream));
   DG_HIP(ctx, hipStreamSynchronize(ctx->stream));

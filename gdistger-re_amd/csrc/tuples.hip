@@ -1138,9 +1138,10 @@ dg_tuple_state* tuple_state(dg_ctx* ctx) {
 }
 
 // Check a tuple batch's shape and copy it to the device, where the gathering
-// kernel checks every row id as it reads it (check_rows after the call): a
-// host pass over 65,536 tuples of 7 ids took longer than the whole step's
-// kernels.  Makes the words those checks report to.
+// kernel checks every row id as it reads it (check_call once the kernels have
+// run, before anything goes to the caller): a host pass over 65,536 tuples of
+// 7 ids took longer than the whole step's kernels.  Makes the words those
+// checks report to.
 int upload_tuples(dg_ctx* ctx, dg_tuple_state* st, const dg_table_view& tv, const uint32_t* tuples,
                   uint64_t n, uint32_t K) {
   if (K > (uint32_t)kMaxTupleNeg)
@@ -1289,7 +1290,7 @@ extern "C" int dg_sgns_tuples_forward(dg_ctx* ctx, const uint32_t* tuples, uint6
   DG_HIP(ctx, hipGetLastError());
   DG_CHECK(dg_time_end(ctx, tk));
   if (logits)
-    DG_CHECK(dg_copy_to_host(ctx, logits, st->d_logits, sizeof(float) * n * K1));
+    DG_CHECK(dg_copy_to_host(ctx, logits, st->d_logits, sizeof(float) * n * K1, st->h_err));
   else
     DG_HIP(ctx, hipStreamSynchronize(ctx->stream));
   DG_CHECK(dg_time_resolve(ctx));
@@ -1539,7 +1540,7 @@ int tuples_backward_run(dg_ctx* ctx, const uint32_t* tuples, uint64_t n, uint32_
     if (shadow) st->bf_version = v;  // the shadow rows were updated with the FP32 rows
   }
   if (fused && logits)
-    DG_CHECK(dg_copy_to_host(ctx, logits, st->d_logits, sizeof(float) * n * K1));
+    DG_CHECK(dg_copy_to_host(ctx, logits, st->d_logits, sizeof(float) * n * K1, st->h_err));
   else
     DG_HIP(ctx, hipStreamSynchronize(ctx->stream));
   DG_CHECK(dg_time_resolve(ctx));
