@@ -192,6 +192,7 @@ int dg_reserve(dg_ctx* ctx, T** ptr, size_t* cap, size_t need) {
   hipError_t e = hipMalloc((void**)ptr, n * sizeof(T));
   if (e != hipSuccess) {
     *ptr = nullptr;
+    (void)hipGetLastError();  // not the next launch's
     return dg_fail(ctx, DG_ERR_NOMEM, "hipMalloc(%zu bytes): %s", n * sizeof(T),
                    hipGetErrorString(e));
   }
@@ -206,9 +207,11 @@ int dg_grow_keep(dg_ctx* ctx, T** ptr, size_t* cap, size_t need, size_t keep) {
   size_t n = need > 2 * *cap ? need : 2 * *cap;
   T* np = nullptr;
   hipError_t e = hipMalloc((void**)&np, n * sizeof(T));
-  if (e != hipSuccess)
+  if (e != hipSuccess) {
+    (void)hipGetLastError();
     return dg_fail(ctx, DG_ERR_NOMEM, "hipMalloc(%zu bytes): %s", n * sizeof(T),
                    hipGetErrorString(e));
+  }
   if (*ptr && keep) {
     e = hipMemcpyAsync(np, *ptr, keep * sizeof(T), hipMemcpyDeviceToDevice, ctx->stream);
     if (e != hipSuccess) return dg_fail(ctx, DG_ERR_HIP, "hipMemcpyAsync: %s", hipGetErrorString(e));

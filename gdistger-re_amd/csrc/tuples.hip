@@ -1084,7 +1084,8 @@ struct dg_tuple_state {
   // look-back wait, a store bound), [2..3] the loss (a double)
   uint32_t* h_err = nullptr;
   uint32_t* d_err = nullptr;    // the device's address of h_err
-  uint32_t* d_fail = nullptr;   // the failed check's code on the device; zero between calls
+  uint32_t* d_fail = nullptr;   // the failed check's code on the device
+  bool fail_clean = false;      // d_fail is zero: false from a call's start to the end of its checks
   float* d_grad = nullptr;
   size_t grad_cap = 0;
   float* d_carry = nullptr;
@@ -1156,12 +1157,14 @@ int upload_tuples(dg_ctx* ctx, dg_tuple_state* st, const dg_table_view& tv, cons
     DG_HIP(ctx, hipHostMalloc((void**)&st->h_err, 4 * sizeof(uint32_t), hipHostMallocMapped | hipHostMallocCoherent));
     DG_HIP(ctx, hipHostGetDevicePointer((void**)&st->d_err, st->h_err, 0));
   }
-  if (!st->d_fail) {
-    DG_HIP(ctx, hipMalloc((void**)&st->d_fail, sizeof(uint32_t)));
+  if (!st->d_fail) DG_HIP(ctx, hipMalloc((void**)&st->d_fail, sizeof(uint32_t)));
+  if (!st->fail_clean) {  // the first call, or the one before ended early: its kernels may still run
     clear_word_kernel<<<1, 64, 0, ctx->stream>>>(st->d_fail);
     DG_HIP(ctx, hipGetLastError());
+    DG_HIP(ctx, hipStreamSynchronize(ctx->stream));
   }
-  *st->h_err = 0u;  // the previous call's kernels have finished
+  st->fail_clean = false;
+  *st->h_err = 0u;
   DG_CHECK(dg_reserve(ctx, &st->d_tuples, &st->tuples_cap, (size_t)(n * W)));
   DG_HIP(ctx, hipMemcpyAsync(st->d_tuples, tuples, sizeof(uint32_t) * n * W, hipMemcpyHostToDevice,
                              ctx->stream));
@@ -1172,9 +1175,8 @@ int upload_tuples(dg_ctx* ctx, dg_tuple_state* st, const dg_table_view& tv, cons
 int check_call(dg_ctx* ctx, dg_tuple_state* st, const dg_table_view& tv, const uint32_t* tuples, uint64_t n,
                uint32_t K) {
   const uint32_t code = *st->h_err;
+  st->fail_clean = code == 0u;
   if (code == 0u) return DG_OK;
-  clear_word_kernel<<<1, 64, 0, ctx->stream>>>(st->d_fail);
-  DG_HIP(ctx, hipGetLastError());
   const uint64_t W = K + 2;
   for (uint64_t i = 0; i < n * W; ++i)
     if (tuples[i] >= tv.rows)
@@ -1439,6 +1441,11 @@ int tuples_backward_run(dg_ctx* ctx, const uint32_t* tuples, uint64_t n, uint32_
   const uint64_t n_lb = o_sort + (uint64_t)passes * pass_words;
   const bool tickets = n_tiles > (uint64_t)ctx->num_cus;
   DG_CHECK(dg_reserve(ctx, &st->d_lb, &st->lb_cap, (size_t)n_lb));
+  // every buffer before the first launch: a call without room has run nothing
+  DG_CHECK(dg_reserve(ctx, &st->d_grad, &st->grad_cap, (size_t)(N * dim)));
+  DG_CHECK(dg_reserve(ctx, &st->d_carry, &st->carry_cap, (size_t)(n_blocks * dim)));
+  DG_CHECK(dg_reserve(ctx, &st->d_headp, &st->headp_cap, (size_t)(n_blocks * dim)));
+  DG_CHECK(dg_reserve(ctx, &st->d_fin, &st->fin_cap, (size_t)n_blocks));
   TupleArgs a{};
   a.tuples = st->d_tuples;
   a.n = n;
@@ -1492,10 +1499,6 @@ int tuples_backward_run(dg_ctx* ctx, const uint32_t* tuples, uint64_t n, uint32_
   DG_HIP(ctx, hipGetLastError());
   DG_CHECK(dg_time_end(ctx, tk));
   // segmented sums, then the rows that cross blocks (and, with apply, the updates)
-  DG_CHECK(dg_reserve(ctx, &st->d_grad, &st->grad_cap, (size_t)(N * dim)));
-  DG_CHECK(dg_reserve(ctx, &st->d_carry, &st->carry_cap, (size_t)(n_blocks * dim)));
-  DG_CHECK(dg_reserve(ctx, &st->d_headp, &st->headp_cap, (size_t)(n_blocks * dim)));
-  DG_CHECK(dg_reserve(ctx, &st->d_fin, &st->fin_cap, (size_t)n_blocks));
   SegArgs sa{};
   sa.rows = tv.rows;
   sa.keys = st->d_k[cur];
