@@ -580,6 +580,18 @@ static void host_rows(uint32_t n, F f) {
 
 namespace {
 
+// An allocation: without room the call ends with DG_ERR_NOMEM (and the
+// allocation's error is not the next launch's).
+#define DG_ROOM(ctx, expr)                                                              \
+  do {                                                                                  \
+    hipError_t _e = (expr);                                                             \
+    if (_e != hipSuccess) {                                                             \
+      (void)hipGetLastError();                                                          \
+      return dg_fail((ctx), _e == hipErrorOutOfMemory ? DG_ERR_NOMEM : DG_ERR_HIP,      \
+                     "%s failed: %s (%s:%d)", #expr, hipGetErrorString(_e), __FILE__, __LINE__); \
+    }                                                                                   \
+  } while (0)
+
 // Device memory of one call, freed with it.
 struct Scratch {
   std::vector<void*> bufs;
@@ -608,8 +620,8 @@ static int enqueue_cn(dg_ctx* ctx, Scratch& mem, uint32_t v_num, uint64_t m, con
   if (cap) {
     uint32_t* d_count = nullptr;
     HubRec* d_hubs = nullptr;
-    DG_HIP(ctx, mem.get(&d_count, 2));
-    DG_HIP(ctx, mem.get(&d_hubs, cap));
+    DG_ROOM(ctx, mem.get(&d_count, 2));
+    DG_ROOM(ctx, mem.get(&d_hubs, cap));
     fill_kernel<<<1, 64, 0, ctx->stream>>>(d_count, 1, 0u);
     hub_list_kernel<<<grid_for(ctx, v_num, 256), 256, 0, ctx->stream>>>(d_rp, v_num, d_count, (uint32_t)cap,
                                                                        d_hubs);
@@ -638,12 +650,12 @@ static int enqueue_cn(dg_ctx* ctx, Scratch& mem, uint32_t v_num, uint64_t m, con
   uint32_t *d_big = nullptr, *d_tsize = nullptr, *d_tab = nullptr, *d_it_hub = nullptr;
   uint64_t *d_toff = nullptr, *d_it_k0 = nullptr;
   if (!big.empty()) {
-    DG_HIP(ctx, mem.get(&d_big, big.size()));
-    DG_HIP(ctx, mem.get(&d_tsize, big.size()));
-    DG_HIP(ctx, mem.get(&d_toff, big.size()));
-    DG_HIP(ctx, mem.get(&d_tab, tslots));
-    DG_HIP(ctx, mem.get(&d_it_hub, it_hub.size()));
-    DG_HIP(ctx, mem.get(&d_it_k0, it_k0.size()));
+    DG_ROOM(ctx, mem.get(&d_big, big.size()));
+    DG_ROOM(ctx, mem.get(&d_tsize, big.size()));
+    DG_ROOM(ctx, mem.get(&d_toff, big.size()));
+    DG_ROOM(ctx, mem.get(&d_tab, tslots));
+    DG_ROOM(ctx, mem.get(&d_it_hub, it_hub.size()));
+    DG_ROOM(ctx, mem.get(&d_it_k0, it_k0.size()));
     DG_HIP(ctx, hipMemcpy(d_big, big.data(), sizeof(uint32_t) * big.size(), hipMemcpyHostToDevice));
     DG_HIP(ctx, hipMemcpy(d_tsize, tsize.data(), sizeof(uint32_t) * big.size(), hipMemcpyHostToDevice));
     DG_HIP(ctx, hipMemcpy(d_toff, toff.data(), sizeof(uint64_t) * big.size(), hipMemcpyHostToDevice));
@@ -707,9 +719,9 @@ static int cn_of_multigraph(dg_ctx* ctx, uint32_t v_num, uint64_t m) {
     Scratch mem;
     uint64_t* d_rp = nullptr;
     uint32_t *d_nbr = nullptr, *d_cn = nullptr;
-    DG_HIP(ctx, mem.get(&d_rp, v_num + 1ull));
-    DG_HIP(ctx, mem.get(&d_nbr, cm));
-    DG_HIP(ctx, mem.get(&d_cn, cm));
+    DG_ROOM(ctx, mem.get(&d_rp, v_num + 1ull));
+    DG_ROOM(ctx, mem.get(&d_nbr, cm));
+    DG_ROOM(ctx, mem.get(&d_cn, cm));
     DG_HIP(ctx, hipMemcpy(d_rp, srp.data(), sizeof(uint64_t) * (v_num + 1ull), hipMemcpyHostToDevice));
     if (cm) DG_HIP(ctx, hipMemcpy(d_nbr, snbr.data(), sizeof(uint32_t) * cm, hipMemcpyHostToDevice));
     DG_CHECK(enqueue_cn(ctx, mem, v_num, cm, d_rp, d_nbr, nullptr, d_cn, nullptr));
@@ -748,7 +760,7 @@ static int finish_graph(dg_ctx* ctx, const float* d_w, const uint64_t* d_rev, co
     // hot set for visit counting: walks visit vertices in proportion to degree
     const uint32_t n_hot = v_num < kHotMax ? v_num : kHotMax;
     uint32_t* d_hist = nullptr;
-    DG_HIP(ctx, mem.get(&d_hist, kDegBins + 4));
+    DG_ROOM(ctx, mem.get(&d_hist, kDegBins + 4));
     fill_kernel<<<grid_for(ctx, kDegBins + 4, 256), 256, 0, ctx->stream>>>(d_hist, kDegBins + 4, 0u);
     const unsigned gd = (unsigned)std::min<uint64_t>((uint64_t)ctx->num_cus, ((uint64_t)v_num + 255) / 256);
     degree_hist_kernel<<<gd, 256, 0, ctx->stream>>>(ctx->d_deg, v_num, d_hist);
@@ -760,7 +772,7 @@ static int finish_graph(dg_ctx* ctx, const float* d_w, const uint64_t* d_rev, co
   DG_HIP(ctx, hipGetLastError());
   if (cn_mode == DG_CN_COMPUTE || cn_mode == DG_CN_COMPUTE_WEIGHTED) {
     uint32_t* d_flag = nullptr;
-    DG_HIP(ctx, mem.get(&d_flag, 1));
+    DG_ROOM(ctx, mem.get(&d_flag, 1));
     DG_CHECK(enqueue_cn(ctx, mem, v_num, m, ctx->d_row_ptr, ctx->d_nbr, d_rev, ctx->d_cn, d_flag));
     uint32_t not_simple = 0;
     DG_HIP(ctx, hipMemcpyAsync(&not_simple, d_flag, sizeof(not_simple), hipMemcpyDeviceToHost, ctx->stream));
@@ -783,13 +795,13 @@ static int alloc_graph(dg_ctx* ctx, uint32_t v_num, uint64_t m) {
   dg_walk_free(ctx);  // walker state belongs to the previous graph
   dg_graph_free(ctx);
   const uint64_t n = m ? m : 1;
-  DG_HIP(ctx, hipMalloc((void**)&ctx->d_row_ptr, sizeof(uint64_t) * (v_num + 1ull)));
-  DG_HIP(ctx, hipMalloc((void**)&ctx->d_nbr, sizeof(uint32_t) * n));
-  DG_HIP(ctx, hipMalloc((void**)&ctx->d_cn, sizeof(uint32_t) * n));
-  DG_HIP(ctx, hipMalloc((void**)&ctx->d_adj, sizeof(uint4) * n));
-  DG_HIP(ctx, hipMalloc((void**)&ctx->d_deg, sizeof(uint32_t) * v_num));
-  DG_HIP(ctx, hipMalloc((void**)&ctx->d_hot_slot, sizeof(uint16_t) * v_num));
-  DG_HIP(ctx, hipMalloc((void**)&ctx->d_hot_id, sizeof(uint32_t) * kHotMax));
+  DG_ROOM(ctx, hipMalloc((void**)&ctx->d_row_ptr, sizeof(uint64_t) * (v_num + 1ull)));
+  DG_ROOM(ctx, hipMalloc((void**)&ctx->d_nbr, sizeof(uint32_t) * n));
+  DG_ROOM(ctx, hipMalloc((void**)&ctx->d_cn, sizeof(uint32_t) * n));
+  DG_ROOM(ctx, hipMalloc((void**)&ctx->d_adj, sizeof(uint4) * n));
+  DG_ROOM(ctx, hipMalloc((void**)&ctx->d_deg, sizeof(uint32_t) * v_num));
+  DG_ROOM(ctx, hipMalloc((void**)&ctx->d_hot_slot, sizeof(uint16_t) * v_num));
+  DG_ROOM(ctx, hipMalloc((void**)&ctx->d_hot_id, sizeof(uint32_t) * kHotMax));
   ctx->v_num = v_num;
   ctx->m = m;
   return DG_OK;
@@ -824,11 +836,8 @@ struct CsrScratch {
   }
 };
 
-// CSR built on the device: the edges go up once and only the first bad
-// index, the hubs and one flag come back.
-static int build_on_device(dg_ctx* ctx, Scratch& mem, CsrScratch& t, uint32_t v_num, const dg_edge* edges,
-                           uint64_t e_num, int undirected, int cn_mode) {
-  const uint64_t m = e_num * (undirected ? 2 : 1);
+// The edges on the device, and none of them out of range.
+static int send_edges(dg_ctx* ctx, CsrScratch& t, uint32_t v_num, const dg_edge* edges, uint64_t e_num) {
   unsigned long long bad = ~0ull;
   set_u64_kernel<<<1, 64, 0, ctx->stream>>>(t.bad, bad);
   DG_HIP(ctx, hipMemcpyAsync(t.edges, edges, sizeof(dg_edge) * e_num, hipMemcpyHostToDevice, ctx->stream));
@@ -836,7 +845,13 @@ static int build_on_device(dg_ctx* ctx, Scratch& mem, CsrScratch& t, uint32_t v_
   DG_HIP(ctx, hipGetLastError());
   DG_HIP(ctx, hipMemcpyAsync(&bad, t.bad, sizeof(bad), hipMemcpyDeviceToHost, ctx->stream));
   DG_HIP(ctx, hipStreamSynchronize(ctx->stream));
-  if (bad != ~0ull) return edge_range_error(ctx, edges, bad, v_num);
+  return bad == ~0ull ? DG_OK : edge_range_error(ctx, edges, bad, v_num);
+}
+
+// CSR built on the device from edges that are there: only the hubs and one
+// flag come back.
+static int build_on_device(dg_ctx* ctx, CsrScratch& t, uint32_t v_num, uint64_t e_num, int undirected, int cn_mode) {
+  const uint64_t m = e_num * (undirected ? 2 : 1);
   DG_CHECK(alloc_graph(ctx, v_num, m));
   entry_keys_kernel<<<grid_for(ctx, e_num, 256), 256, 0, ctx->stream>>>(t.edges, e_num, undirected, t.keys[0],
                                                                        t.ids[0]);
@@ -861,12 +876,10 @@ static int build_on_device(dg_ctx* ctx, Scratch& mem, CsrScratch& t, uint32_t v_
 }
 
 // CSR built on the host (entries past 32 bits, or no room for the device
-// build's working memory): include/graph.hpp:671-699 then :509-540, the
+// build and its working memory): include/graph.hpp:671-699 then :509-540, the
 // doubled list counted and placed in order.
 static int build_on_host(dg_ctx* ctx, uint32_t v_num, const dg_edge* edges, uint64_t e_num, int undirected,
                          int cn_mode) {
-  for (uint64_t i = 0; i < e_num; ++i)
-    if (edges[i].src >= v_num || edges[i].dst >= v_num) return edge_range_error(ctx, edges, i, v_num);
   const uint64_t m = e_num * (undirected ? 2 : 1);
   std::vector<uint64_t> rp(v_num + 1ull, 0);
   for (uint64_t i = 0; i < e_num; ++i) {
@@ -911,11 +924,11 @@ static int build_on_host(dg_ctx* ctx, uint32_t v_num, const dg_edge* edges, uint
     DG_HIP(ctx, hipMemcpy(ctx->d_nbr, nbr.data(), sizeof(uint32_t) * m, hipMemcpyHostToDevice));
     if (from_data) DG_HIP(ctx, hipMemcpy(ctx->d_cn, cn.data(), sizeof(uint32_t) * m, hipMemcpyHostToDevice));
     if (want_rev) {
-      DG_HIP(ctx, mem.get(&d_rev, m));
+      DG_ROOM(ctx, mem.get(&d_rev, m));
       DG_HIP(ctx, hipMemcpy(d_rev, rev.data(), sizeof(uint64_t) * m, hipMemcpyHostToDevice));
     }
     if (weighted) {  // only needed for the thresholds, so not kept
-      DG_HIP(ctx, mem.get(&d_w, m));
+      DG_ROOM(ctx, mem.get(&d_w, m));
       DG_HIP(ctx, hipMemcpy(d_w, weight.data(), sizeof(float) * m, hipMemcpyHostToDevice));
     }
   }
@@ -929,14 +942,24 @@ extern "C" int dg_graph_from_edges(dg_ctx* ctx, uint32_t v_num, const dg_edge* e
     return dg_fail(ctx, DG_ERR_ARG, "unknown cn_mode %d", cn_mode);
   DG_HIP(ctx, hipSetDevice(ctx->device));
   const uint64_t m = e_num * (undirected ? 2 : 1);
+  int rc = DG_ERR_NOMEM;
   if (m > 0 && m < (1ull << 32)) {
     Scratch mem;
     CsrScratch t;
-    if (t.get(mem, e_num, m, undirected && cn_mode != DG_CN_FROM_DATA, cn_mode == DG_CN_COMPUTE_WEIGHTED))
-      return build_on_device(ctx, mem, t, v_num, edges, e_num, undirected, cn_mode);
-    (void)hipGetLastError();
+    if (t.get(mem, e_num, m, undirected && cn_mode != DG_CN_FROM_DATA, cn_mode == DG_CN_COMPUTE_WEIGHTED)) {
+      DG_CHECK(send_edges(ctx, t, v_num, edges, e_num));  // the graph before stays
+      rc = build_on_device(ctx, t, v_num, e_num, undirected, cn_mode);
+    } else {
+      (void)hipGetLastError();
+    }
   }
-  return build_on_host(ctx, v_num, edges, e_num, undirected, cn_mode);
+  if (rc == DG_ERR_NOMEM) {
+    for (uint64_t i = 0; i < e_num; ++i)
+      if (edges[i].src >= v_num || edges[i].dst >= v_num) return edge_range_error(ctx, edges, i, v_num);
+    rc = build_on_host(ctx, v_num, edges, e_num, undirected, cn_mode);
+  }
+  if (rc != DG_OK) dg_graph_free(ctx);  // never a part of one
+  return rc;
 }
 
 extern "C" int dg_graph_load_bin(dg_ctx* ctx, const char* path, uint32_t v_num, int undirected,
@@ -987,7 +1010,7 @@ extern "C" int dg_graph_get_thresholds(dg_ctx* ctx, uint32_t* thr) {
   if (ctx->m == 0) return DG_OK;
   Scratch mem;
   uint32_t* d_thr = nullptr;
-  DG_HIP(ctx, mem.get(&d_thr, ctx->m));
+  DG_ROOM(ctx, mem.get(&d_thr, ctx->m));
   take_thresholds_kernel<<<grid_for(ctx, ctx->m, 256), 256, 0, ctx->stream>>>(ctx->d_adj, ctx->m, d_thr);
   DG_HIP(ctx, hipGetLastError());
   DG_CHECK(dg_copy_to_host(ctx, thr, d_thr, sizeof(uint32_t) * ctx->m));
