@@ -39,19 +39,28 @@ extern "C" int dg_open(int device, dg_ctx** out) {
     delete ctx;
     return DG_ERR_HIP;
   }
-  if (hipMalloc((void**)&ctx->d_queue, sizeof(dg_walk_queue)) != hipSuccess ||
-      hipMalloc((void**)&ctx->d_shards, sizeof(dg_walk_shard) * kWalkShards) != hipSuccess ||
-      hipHostMalloc((void**)&ctx->h_queue, sizeof(dg_walk_queue), hipHostMallocDefault) !=
-          hipSuccess) {
+  constexpr size_t kQueue = 256, kFlag = 64, kWords = 192;  // queue, flag and words before the stage
+  static_assert(sizeof(dg_walk_queue) <= kQueue, "");
+  char* dev = nullptr;
+  if (hipMalloc((void**)&dev, kQueue + sizeof(dg_walk_shard) * kWalkShards) != hipSuccess) {
     dg_close(ctx);
     return DG_ERR_NOMEM;
   }
-  memset(ctx->h_queue, 0, sizeof(dg_walk_queue));
-  if (hipHostMalloc((void**)&ctx->h_flag, 64, hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess ||
-      hipHostGetDevicePointer((void**)&ctx->d_flag, ctx->h_flag, 0) != hipSuccess) {
+  ctx->d_queue = reinterpret_cast<dg_walk_queue*>(dev);
+  ctx->d_shards = reinterpret_cast<dg_walk_shard*>(dev + kQueue);
+  if (hipHostMalloc((void**)&ctx->h_block, kQueue + kFlag + kWords + kStageBytes,
+                    hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess ||
+      hipHostGetDevicePointer((void**)&dev, ctx->h_block, 0) != hipSuccess) {
     dg_close(ctx);
     return DG_ERR_NOMEM;
   }
+  memset(ctx->h_block, 0, kQueue + kFlag + kWords);
+  ctx->h_queue = reinterpret_cast<dg_walk_queue*>(ctx->h_block);
+  ctx->h_flag = reinterpret_cast<uint32_t*>(ctx->h_block + kQueue);
+  ctx->d_flag = reinterpret_cast<uint32_t*>(dev + kQueue);
+  ctx->h_words = reinterpret_cast<uint32_t*>(ctx->h_block + kQueue + kFlag);
+  ctx->d_words = reinterpret_cast<uint32_t*>(dev + kQueue + kFlag);
+  ctx->h_stage = ctx->h_block + kQueue + kFlag + kWords;
   if (dg_tuples_scratch_setup(ctx) != DG_OK) {
     dg_close(ctx);
     return DG_ERR_HIP;
@@ -79,9 +88,7 @@ extern "C" void dg_close(dg_ctx* ctx) {
   for (auto e : ctx->event_pool) hipEventDestroy(e);
   if (ctx->d_stamps) hipFree(ctx->d_stamps);
   if (ctx->d_queue) hipFree(ctx->d_queue);
-  if (ctx->d_shards) hipFree(ctx->d_shards);
-  if (ctx->h_queue) hipHostFree(ctx->h_queue);
-  if (ctx->h_flag) hipHostFree(ctx->h_flag);
+  if (ctx->h_block) hipHostFree(ctx->h_block);
   if (ctx->stream) hipStreamDestroy(ctx->stream);
   if (ctx->opened) dg_hostcopy_close();
   delete ctx;

@@ -13,6 +13,23 @@
 #include <mutex>
 #include <thread>
 
+// Whether memory that makes copies faster is to be made for the next one: once
+// the copies that went without it come to `after` bytes.  What it costs to make
+// is about what those lost, so a program with few copies does not pay for it,
+// and none pays more than twice what it would have to.
+class MadeAfter {
+ public:
+  bool due(size_t bytes, size_t after) {
+    if (without_ >= after) return true;
+    without_ += bytes;
+    return false;
+  }
+  void reset() { without_ = 0; }
+
+ private:
+  size_t without_ = 0;
+};
+
 // What became of a copy.
 enum class CopyEnd {
   kDone,

@@ -100,7 +100,7 @@ struct dg_ctx {
   // walker buffers
   dg_walk_queue* d_queue = nullptr;
   dg_walk_queue* h_queue = nullptr;  // pinned mirror
-  dg_walk_shard* d_shards = nullptr; // kWalkShards
+  dg_walk_shard* d_shards = nullptr; // kWalkShards, behind the queue
   uint32_t* d_freq = nullptr;        // cumulative visit counts
   uint64_t freq_total = 0;           // sum of d_freq
   uint32_t* d_tok_raw = nullptr;     // walk slots, longer walks, the packing's words
@@ -140,10 +140,17 @@ struct dg_ctx {
   dg_tuple_state* tuples = nullptr;
   dg_pipe_state* pipe = nullptr;
   dg_dsgl_state* dsgl = nullptr;
+  // the context's pinned memory, in one allocation (they cost 20 us and more
+  // each): h_queue, then
+  char* h_block = nullptr;
   // a host-visible word a kernel sets when an id it was given is out of range,
   // and the device's address of it
   uint32_t* h_flag = nullptr;
   uint32_t* d_flag = nullptr;
+  // host-visible words of the tuple calls, and their device address
+  uint32_t* h_words = nullptr;
+  uint32_t* d_words = nullptr;
+  char* h_stage = nullptr;  // kStageBytes: small results on their way to the caller
   // this device's copy of the allocation-free entry point's scratch array
   // (its address from hipGetSymbolAddress, set when the context opens)
   float* noalloc_scratch = nullptr;
@@ -305,6 +312,8 @@ struct dg_dsgl_call {
 };
 int dg_dsgl_train(dg_ctx* ctx, const dg_dsgl_call& c, uint64_t* kept, double* ms, float* alpha_end);
 void dg_dsgl_free(dg_ctx* ctx);
+
+constexpr size_t kStageBytes = 64u << 10;
 
 // Copies device memory to the caller's pageable buffer, after the context's
 // queued work, and returns when the bytes are there (hostcopy.hip).  Where that

@@ -1080,8 +1080,8 @@ struct dg_tuple_state {
   size_t v_cap[2] = {0, 0};
   uint32_t* d_lb = nullptr;     // tickets, then the look-back words of the sort and segment launches
   size_t lb_cap = 0;
-  // host-visible words: [0] set by a kernel whose check failed (a row id, a
-  // look-back wait, a store bound), [2..3] the loss (a double)
+  // the context's host-visible words: [0] set by a kernel whose check failed (a
+  // row id, a look-back wait, a store bound), [2..3] the loss (a double)
   uint32_t* h_err = nullptr;
   uint32_t* d_err = nullptr;    // the device's address of h_err
   uint32_t* d_fail = nullptr;   // the failed check's code on the device
@@ -1122,7 +1122,6 @@ void dg_tuples_free(dg_ctx* ctx) {
                   t->d_rows,   t->d_rows_out};
   for (void* b : bufs)
     if (b) hipFree(b);
-  if (t->h_err) hipHostFree(t->h_err);
   delete t;
   ctx->tuples = nullptr;
 }
@@ -1141,7 +1140,7 @@ dg_tuple_state* tuple_state(dg_ctx* ctx) {
 // Check a tuple batch's shape and copy it to the device, where the gathering
 // kernel checks every row id as it reads it (check_call once the kernels have
 // run, before anything goes to the caller): a host pass over 65,536 tuples of
-// 7 ids took longer than the whole step's kernels.  Makes the words those
+// 7 ids took longer than the whole step's kernels.  Clears the words those
 // checks report to.
 int upload_tuples(dg_ctx* ctx, dg_tuple_state* st, const dg_table_view& tv, const uint32_t* tuples,
                   uint64_t n, uint32_t K) {
@@ -1153,10 +1152,8 @@ int upload_tuples(dg_ctx* ctx, dg_tuple_state* st, const dg_table_view& tv, cons
   if (n == 0 || n * W >= (1ull << 31))
     return dg_fail(ctx, DG_ERR_ARG, "tuple count %llu: must be in [1, 2^31 / (K + 2))",
                    (unsigned long long)n);
-  if (!st->h_err) {
-    DG_HIP(ctx, hipHostMalloc((void**)&st->h_err, 4 * sizeof(uint32_t), hipHostMallocMapped | hipHostMallocCoherent));
-    DG_HIP(ctx, hipHostGetDevicePointer((void**)&st->d_err, st->h_err, 0));
-  }
+  st->h_err = ctx->h_words;
+  st->d_err = ctx->d_words;
   if (!st->d_fail) DG_HIP(ctx, hipMalloc((void**)&st->d_fail, sizeof(uint32_t)));
   if (!st->fail_clean) {  // the first call, or the one before ended early: its kernels may still run
     clear_word_kernel<<<1, 64, 0, ctx->stream>>>(st->d_fail);

@@ -83,5 +83,14 @@ int main() {
   check("refused, one chunk", 100, kNever, kNever, false, CopyEnd::kRefused, 0, 0);
   check("whole again", 33 * C + 5, kNever, kNever, true, CopyEnd::kDone, 34, 34);
   ring.stop([](char* p) { free(p); });
-  return bad ? 1 : 0;
+  // memory for faster copies: not for a few small ones, and after so many bytes without it
+  MadeAfter made;
+  int without = 0;
+  while (!made.due(100, 1000)) ++without;
+  bool late = made.due(1, 1000);
+  made.reset();
+  const bool again = made.due(5000, 1000), then = made.due(1, 1000);
+  const bool ok = without == 10 && late && !again && then;
+  printf("%s made after 10 of 100 bytes, at once later, anew after the last user\n", ok ? "ok" : "WRONG");
+  return bad || !ok ? 1 : 0;
 }

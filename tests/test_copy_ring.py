@@ -1,7 +1,7 @@
 """The ring that carries large results to the caller's buffers, on the CPU, with
 a transfer engine that fails or refuses at a chosen chunk: a buffer gets bytes
 of its own copy and nothing else, in particular not what the ring's chunks held
-before, and every copy ends."""
+before, and every copy ends.  And the rule by which the ring is made at all."""
 
 import os
 import subprocess
@@ -17,4 +17,4 @@ def test_copy_ring(tmp_path):
     r = subprocess.run([exe], capture_output=True, text=True, timeout=120)
     print(r.stdout)
     assert r.returncode == 0, r.stdout
-    assert r.stdout.count("ok ") == 17
+    assert r.stdout.count("ok ") == 18
