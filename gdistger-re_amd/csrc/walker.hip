@@ -1041,10 +1041,13 @@ static int plan_round(dg_ctx* ctx, const dg_walk_params* p, uint32_t round,
   const uint64_t need_blocks = ((uint64_t)walker_num + kWalkBlock - 1) / kWalkBlock;
   if (blocks > need_blocks) blocks = need_blocks ? need_blocks : 1;
   // spill space for the longest walk, (limit - kPathLds) vertices per lane
-  // (1 GB for the default limit): only once a walk has needed it, or when
-  // every walk will (the reference's walks end at 22 vertices)
+  // (1 GB for the default limit): only once a walk has needed it, or where they
+  // will (the reference's walks end at 22 vertices): past min_length, or with a
+  // threshold well below the reference's 0.999, at which walks run on
+  // (walk.hpp:979-985; of 50,000 walks on a Chung-Lu graph 1 passes 24 vertices
+  // at 0.97, 138 at 0.95 and 4,698 at 0.9)
   const uint32_t longest = p->max_length != 0 ? p->max_length : length_limit;
-  if (p->min_length + 1 >= (uint32_t)kPathLds) ctx->walks_spill = true;
+  if (p->min_length + 1 >= (uint32_t)kPathLds || p->mu <= 0.95) ctx->walks_spill = true;
   const uint32_t spill_per_slot =
       ctx->walks_spill && longest > (uint32_t)kPathLds ? longest - (uint32_t)kPathLds : 0;
 
@@ -1251,12 +1254,22 @@ static int walk_round_impl(dg_ctx* ctx, const dg_walk_params* p, uint32_t round,
   // at most one repeat for spill space and two for token space
   for (int attempt = 0; attempt < 4; ++attempt) {
     DG_CHECK(plan_round(ctx, p, round, walker_begin, walker_num, &pl));
-    DG_CHECK(reserve_tokens(ctx));
+    // where the packed corpus has to be allocated, a round that needs more room
+    // is known before that (one host wait more, once per size)
+    const bool fits = ctx->d_tokens && ctx->tokens_cap >= ctx->tok_raw_cap;
     DG_CHECK(enqueue_walk(ctx, pl, true));
-    DG_CHECK(enqueue_tail(ctx, pl, true));
-    DG_CHECK(read_queue(ctx));
     bool retry = false;
-    const int rc = check_flags(ctx, pl, &retry);
+    int rc = DG_OK;
+    if (!fits) {
+      DG_CHECK(read_queue(ctx));
+      rc = check_flags(ctx, pl, &retry);
+    }
+    if (rc == DG_OK && !retry) {
+      DG_CHECK(reserve_tokens(ctx));
+      DG_CHECK(enqueue_tail(ctx, pl, true));
+      DG_CHECK(read_queue(ctx));
+      rc = check_flags(ctx, pl, &retry);
+    }
     if (rc != DG_OK || retry) {
       DG_CHECK(dg_time_resolve(ctx));
       if (rc != DG_OK) return rc;

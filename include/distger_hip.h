@@ -104,7 +104,8 @@ int dg_graph_get_thresholds(dg_ctx* ctx, uint32_t* thr);
 /* Safety limit on vertices per walk when dg_walk_params.length_limit is 0.
  * The reference has no limit (walk.hpp:979-985); a walk that reaches it ends
  * the round with DG_ERR_WALK_TOO_LONG.  The walker keeps (limit - 24)
- * vertices of spill space per resident lane once a walk has needed it. */
+ * vertices of spill space per resident lane once a walk has needed it, or where
+ * min_length or a mu of at most 0.95 says that walks will. */
 #define DG_WALK_LENGTH_LIMIT_DEFAULT 1024
 
 #define DG_ROUNDS_REFERENCE 0 /* stop after max_rounds rounds (walk.hpp:740-744) */
