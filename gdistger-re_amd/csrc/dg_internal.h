@@ -32,8 +32,8 @@ struct dg_walk_queue {
 // one after another (about 50 ns each, 0.2 ms for the 4,096 resident ones at
 // the start of every round).
 struct alignas(256) dg_walk_shard {
-  unsigned long long next;    // walks handed out
   unsigned long long draws, moves, tokens;
+  unsigned int next;          // pools of walks handed out
   unsigned int max_len;
 };
 constexpr uint32_t kWalkShards = 64;

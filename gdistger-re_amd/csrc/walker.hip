@@ -9,9 +9,9 @@
 // Design (MI355X-first, not a translation of the OpenMP/MPI loop):
 //   * One lane per walk, 64 walks per wavefront, in one persistent launch.
 //     Walks have uneven lengths; a lane whose walk ends takes the next walk id
-//     from its wave's pool, and a wave refills its pool with one 64-bit atomic
-//     on its shard of the device work queue, so every lane stays busy until
-//     the shard drains and every wave then leaves the loop.
+//     from its wave's pool, and a wave refills its pool with one atomic on its
+//     shard of the device work queue, so every lane stays busy until the shard
+//     drains and every wave then leaves the loop.
 //   * Each lane keeps its walk in LDS (kPathLds vertices, in 16-byte groups of
 //     four) and spills longer walks to a private global area.  The visit count
 //     f_i of walk.hpp:816 (an unordered_map per walk) is a scan of that
@@ -235,8 +235,8 @@ __device__ __forceinline__ uint64_t wave_sum_u64(uint64_t v) {
 // chain, per step one random adjacency read (about 1,100 cycles), the scan of
 // the walk, the entropy arithmetic and half a Philox block (300 to 700
 // each); at large ones the instructions of four wavefronts per SIMD.
-// 10,000 vertices (50,000 walks): 104 -> 44 us; 262,144 vertices: 1.31M walks
-// 649 -> 303 us, 262,144 walks 355 -> 88 us.  Most of it is the sharded queue;
+// 10,000 vertices (50,000 walks): 107 -> 46 us; 262,144 vertices: 1.31M walks
+// 655 -> 303 us, 262,144 walks 352 -> 75 us.  Most of it is the sharded queue;
 // the one-read step, the 16-byte scan, the reciprocals and the shared Philox
 // evaluations took 12% with the queue as it was.
 __global__ __launch_bounds__(kWalkBlock) void walk_kernel(WalkArgs a) {
@@ -250,14 +250,13 @@ __global__ __launch_bounds__(kWalkBlock) void walk_kernel(WalkArgs a) {
   const uint64_t slot = (uint64_t)blockIdx.x * kWalkBlock + threadIdx.x;
   uint32_t* spill = a.spill + slot * a.spill_per_slot;
 
-  // this workgroup's shard of the walks: the round's walks divided in
-  // proportion to the workgroups of each shard
+  // this workgroup's shard of the walks, dealt out in pools of 64: pool p is
+  // workgroup (p mod grid)'s, and a shard hands out its workgroups' pools in
+  // order.  A contiguous range each leaves most shards without work where the
+  // ids follow the degrees (walks start at id mod V): a round on R-MAT scale 25
+  // 10.5 ms, and 9.1 so (8.95 with one counter and no shards).
   const uint32_t n_sh = gridDim.x < kWalkShards ? gridDim.x : kWalkShards;
-  const uint32_t sh = blockIdx.x % n_sh, b_per = gridDim.x / n_sh, b_more = gridDim.x % n_sh;
-  const uint64_t b_before = (uint64_t)sh * b_per + (sh < b_more ? sh : b_more);
-  const uint64_t b_mine = b_per + (sh < b_more ? 1u : 0u);
-  const uint64_t id0 = a.walker_num * b_before / gridDim.x;
-  const uint64_t id1 = a.walker_num * (b_before + b_mine) / gridDim.x;
+  const uint32_t sh = blockIdx.x % n_sh, b_mine = gridDim.x / n_sh + (sh < gridDim.x % n_sh ? 1u : 0u);
   dg_walk_shard* const shard = a.shards + sh;
 
   bool active = false;
@@ -288,14 +287,15 @@ __global__ __launch_bounds__(kWalkBlock) void walk_kernel(WalkArgs a) {
           id = pool_next + rank;
           pool_next += nwant;
         } else {
-          unsigned long long base = 0;
-          if (lane == 0) base = atomicAdd(&shard->next, (unsigned long long)kPool);
-          base = id0 + __shfl(base, 0, 64);
+          uint32_t c = 0;
+          if (lane == 0) c = atomicAdd(&shard->next, 1u);
+          c = __builtin_amdgcn_readfirstlane(c);
+          const uint64_t base = ((uint64_t)(c / b_mine) * gridDim.x + sh + (c % b_mine) * n_sh) * kPool;
           id = rank < avail ? pool_next + rank : base + (rank - avail);
           pool_next = base + (nwant - avail);
           pool_end = base + kPool;
         }
-        if (!active && id < id1) {
+        if (!active && id < a.walker_num) {
           // walk.hpp:529-589 (start = id mod V), :661-669 (footprint, step 0),
           // :849-856 (first-visit state)
           wid = (uint32_t)id;
