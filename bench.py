@@ -231,7 +231,8 @@ def rmat25(args):
         log(f"{args.steps} rounds: walker {walk_ms / n_walk:.2f} ms/round, SGNS {bf_ms / args.steps:.1f} ms/round")
         walk_bytes = 2 * 64 * steps_last + 4 * len(tok)
         walk_gbs = walk_bytes / (walk_ms / n_walk * 1e-3) / 1e9
-        resident = 8 * (V + 1) + 16 * m + 2 * V * 128 * 4 + 4 * args.table_size
+        # row offsets; per entry neighbour, count and the 16-byte walker view; tables, unigram table
+        resident = 8 * (V + 1) + 24 * m + 2 * V * 128 * 4 + 4 * args.table_size
         out = {"walk": {"walk_steps_per_s": steps_last / (walk_ms / n_walk * 1e-3),
                         "kernel_ms": walk_ms / n_walk, "algorithmic_bytes_per_launch": walk_bytes,
                         "achieved_gbs": walk_gbs, "frac_hbm": walk_gbs / HBM_GBS},

@@ -90,8 +90,8 @@ __device__ __forceinline__ bool hash_find(const uint32_t* tbl, uint32_t mask, ui
 // binary search over the sums), so that the loads of a whole pass are in
 // flight together.  Bound by the latency of three dependent loads per pass.
 // One list at a time instead (those loads per entry, most lanes idle on the
-// short lists of a power-law graph): 6.2 ms against 1.3 ms (small rows 0.54,
-// hubs 0.74) at 131,072 vertices and 2.7M entries.
+// short lists of a power-law graph): 6.2 ms against 1.1 ms (small rows and hubs
+// 0.55 each) at 131,072 vertices and 2.7M entries.
 constexpr int kFlat = 4;
 
 struct CnLists {
